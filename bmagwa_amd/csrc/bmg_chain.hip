@@ -55,6 +55,19 @@ __device__ __forceinline__ void put(T (&a)[N], int i, T v) {
   for (int q = 0; q < N; ++q) a[q] = (i == q) ? v : a[q];
 }
 
+// A pointer that every lane of a wave holds alike, as a scalar register pair
+// into global memory.  The chain's pointers are read from LDS, and the
+// compiler would take one for an address anywhere (flat instructions, whose
+// waits also cover every LDS access in flight) that may differ by lane.
+template <typename T>
+__device__ __forceinline__ T* gp(T* p) {
+  uint64_t u = (uint64_t)p;
+  const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)u);
+  const uint32_t hi = __builtin_amdgcn_readfirstlane((uint32_t)(u >> 32));
+  u = (uint64_t)hi << 32 | lo;
+  return (T*)(__attribute__((address_space(1))) T*)u;
+}
+
 // ------------------------------------------------------------- state -----
 // The proposed model's factor (packed upper): an LDS array up to 160
 // columns; a larger capacity keeps it in a per-chain global array (L2/HBM),
@@ -62,11 +75,36 @@ __device__ __forceinline__ void put(T (&a)[N], int i, T v) {
 // member is a plain array in the LDS case (as a base-class member the
 // compiler's code for the triangular loops was a fifth slower).
 constexpr int KMAX_LDS = 160;
+struct GlobalFactor {
+  double* p;
+  __device__ __forceinline__ operator double*() const { return gp(p); }
+};
 template <int KMAX>
-using FactorT = std::conditional_t<(KMAX <= KMAX_LDS), double[KMAX * (KMAX + 1) / 2], double*>;
+using FactorT = std::conditional_t<(KMAX <= KMAX_LDS), double[KMAX * (KMAX + 1) / 2], GlobalFactor>;
 
+// counters of ChainScal that change in every iteration
+struct Counters {
+  uint64_t n_accepted, n_acpt[4], n_moves[4];
+  uint64_t tr_count, th_count, th_loci_len, th_beta_len;
+};
+
+// The dataset's, the chain's and its arrays' descriptions, the counters, the
+// move-size tables and the phase clocks are copies too: read through their
+// global addresses, each use between two stores was a vector load of several
+// hundred cycles in front of the work, and each counter a load-add-store
+// that wave 0 waited out.  (With the pointers made global ones and the chain's
+// scalars kept in registers as well, 500 iterations of 16 chains at n =
+// 10,000, p = 500,000 went from 339 to 309 ms, of 64 chains on four datasets
+// of up to 20,000 individuals from 137 to 116 ms.)
 template <int KMAX>
 struct Smem {
+  DevData D;
+  ChainConst K;
+  ChainArrays A;
+  Counters cnt;
+  uint64_t prof[24];
+  double cdf[3][BMG_MAXMS];              // move-size distributions: add/remove, swap, state change
+  double r_ms_sum[BMG_MAXMS], r_ms_n[BMG_MAXMS];
   FactorT<KMAX> L;                       // proposed model's factor (packed upper)
   double xy[KMAX], v[KMAX], d[KMAX];     // proposed model vectors
   double beta[KMAX], mu[KMAX];           // the chain's beta / mu_beta
@@ -139,7 +177,7 @@ struct Ctx {
   const DevData& D;
   const ChainConst& K;
   const ChainArrays& A;
-  uint64_t* prof;   // the chain's phase counters (thread 0 writes), or null
+  uint64_t* prof;   // the chain's phase counters (thread 0 writes)
 };
 
 __device__ __forceinline__ int lane_id() { return threadIdx.x & 63; }
@@ -210,9 +248,9 @@ __global__ __launch_bounds__(BMG_BLOCK) void k_xy_all(DevData D, int coding, dou
 
 template <int KMAX>
 __device__ __forceinline__ double snp_dot_y(Ctx<KMAX>& C, uint64_t snp, int coding) {
-  const double* pre = C.D.xy[coding];
+  const double* pre = gp(C.D.xy[coding]);
   if (pre) return pre[snp];   // precomputed at set-up in this same order
-  return dot_y_block(C.D.g + snp * C.D.W32, C.D.W32, C.D.y, coding, C.S.red);
+  return dot_y_block(gp(C.D.g) + snp * C.D.W32, C.D.W32, gp(C.D.y), coding, C.S.red);
 }
 
 // value planes of a word under a coding known at compile time (CODING >= 0)
@@ -253,8 +291,8 @@ template <int KMAX, int CODING, int T0, int NTH>
 __device__ __forceinline__ void column_dots(Ctx<KMAX>& C, uint64_t snp_new, int cols, uint32_t* __restrict__ xnew,
                                             int32_t* acc) {
   const uint32_t W = C.D.W32;                 // a multiple of 32 words
-  const uint32_t* __restrict__ wn = C.D.g + snp_new * W;
-  const uint32_t* __restrict__ xcol = C.A.xcol;
+  const uint32_t* __restrict__ wn = gp(C.D.g) + snp_new * W;
+  const uint32_t* __restrict__ xcol = gp(C.A.xcol);
   Smem<KMAX>& S = C.S;
   const int me = C.D.me;
   const uint32_t cpc = W / 16;                // chunks per column
@@ -335,9 +373,9 @@ __device__ __forceinline__ void column_dots(Ctx<KMAX>& C, uint64_t snp_new, int 
 template <int KMAX>
 __device__ __forceinline__ void cov_dots(Ctx<KMAX>& C, uint64_t snp_new, int coding_new) {
   const int me = C.D.me;
-  const uint32_t* __restrict__ wn = C.D.g + snp_new * C.D.W32;
+  const uint32_t* __restrict__ wn = gp(C.D.g) + snp_new * C.D.W32;
   for (int c = 1; c < me; ++c) {
-    const double* __restrict__ e = C.D.E + (size_t)(c - 1) * C.D.n_pad;
+    const double* __restrict__ e = gp(C.D.E) + (size_t)(c - 1) * C.D.n_pad;
     double acc = 0.0;
     for (uint32_t i = threadIdx.x; i < C.D.n; i += BMG_BLOCK) {
       const int iv = code_ival((wn[i >> 4] >> (2 * (i & 15))) & 3u, coding_new);
@@ -867,7 +905,7 @@ __device__ __forceinline__ int chol_full(Smem<KMAX>& S, int m) {
 template <int KMAX>
 __device__ __forceinline__ double tree_val(Ctx<KMAX>& C, int tr, int h, uint64_t i) {
   if (h < 2) {
-    const double* base = tr == 0 ? C.A.tree_add : C.A.tree_rem;
+    const double* base = tr == 0 ? gp(C.A.tree_add) : gp(C.A.tree_rem);
     return base[C.D.lev_off[h] + i];
   }
   return C.S.tlev[tr][C.D.lev_off[h] - C.D.lev_off[2] + i];
@@ -982,8 +1020,8 @@ __device__ __forceinline__ uint64_t tree_pick(Ctx<KMAX>& C, int tr, double u) {
 // set leaf i to its weight (unzero) or 0 (zero) and update the path
 template <int KMAX>
 __device__ __forceinline__ void tree_set(Ctx<KMAX>& C, int tr, uint64_t i, int zero) {
-  double* g0 = tr == 0 ? C.A.tree_add : C.A.tree_rem;
-  const double* w = tr == 0 ? C.A.q_add : C.A.q_rem;
+  double* g0 = tr == 0 ? gp(C.A.tree_add) : gp(C.A.tree_rem);
+  const double* w = tr == 0 ? gp(C.A.q_add) : gp(C.A.q_rem);
   double total;
   if (wave_id() == 0) {
     const int lane = lane_id();
@@ -1035,7 +1073,7 @@ __device__ __forceinline__ void tree_set(Ctx<KMAX>& C, int tr, uint64_t i, int z
 // after the two calls.  *w_out: the picked leaf's weight.
 template <int KMAX>
 __device__ __forceinline__ uint64_t tree_pick_zero(Ctx<KMAX>& C, int tr, double u, double* w_out) {
-  double* g0 = tr == 0 ? C.A.tree_add : C.A.tree_rem;
+  double* g0 = tr == 0 ? gp(C.A.tree_add) : gp(C.A.tree_rem);
   if (wave_id() == 0) {
     const int lane = lane_id();
     double total = tr == 0 ? C.R.tot_add : C.R.tot_rem;
@@ -1134,7 +1172,7 @@ __device__ __forceinline__ void journal_restore(Ctx<KMAX>& C) {
     for (int k = C.R.tj_n - 1; k >= 0; --k) {
       const uint64_t v = C.S.tj_ind[k];
       const uint64_t i = v & ~(1ull << 63);
-      double* g0 = (v >> 63) ? C.A.tree_rem : C.A.tree_add;
+      double* g0 = (v >> 63) ? gp(C.A.tree_rem) : gp(C.A.tree_add);
       g0[C.D.lev_off[0] + i] = C.S.tj_old[k][0];
       if (C.D.top >= 1) g0[C.D.lev_off[1] + (i >> 6)] = C.S.tj_old[k][1];
     }
@@ -1176,9 +1214,16 @@ __device__ __forceinline__ void set_slot_bit(Ctx<KMAX>& C, int s, int on) {
 // a sum of non-negative terms equal to it in exact arithmetic.
 #define BMG_S_TINY 1e-8
 template <int KMAX>
-__device__ __noinline__ double direct_syx(Ctx<KMAX>& C) {
-  Smem<KMAX>& S = C.S;
-  const int k = C.R.cols;
+__device__ __forceinline__ void xcoef(Ctx<KMAX>& C, const double* coef, int L, double* out8, int write_yhat);
+
+// out of line (it hardly ever runs), with the model's sizes by value: the
+// caller's state must not have its address taken, which would keep it in
+// scratch memory instead of registers
+template <int KMAX>
+__device__ __noinline__ double direct_syx(Smem<KMAX>& S, int k, int nloci) {
+  Reg R;
+  R.cols = k; R.nloci = nloci;
+  Ctx<KMAX> C{S, R, S.D, S.K, S.A, S.prof};
   __syncthreads();
   for (int i = threadIdx.x; i < k; i += BMG_BLOCK) S.work[i] = S.v[i];
   __syncthreads();
@@ -1189,12 +1234,12 @@ __device__ __noinline__ double direct_syx(Ctx<KMAX>& C) {
   double md = 0.0;
   for (int i = threadIdx.x; i < k; i += BMG_BLOCK) md += S.d[i] * S.work[i] * S.work[i];
   md = block_sum(md, S.red);
-  return C.K.nus2 + o[7] + md;
+  return S.K.nus2 + o[7] + md;
 }
 
 template <int KMAX>
 __device__ __forceinline__ void guard_syx(Ctx<KMAX>& C) {
-  if (!(C.R.syx >= BMG_S_TINY * C.K.nus2_plus_yy)) C.R.syx = direct_syx(C);
+  if (!(C.R.syx >= BMG_S_TINY * C.K.nus2_plus_yy)) C.R.syx = direct_syx(C.S, C.R.cols, C.R.nloci);
 }
 
 // src/model.hpp:432-506 for one column (type A, H, D or R)
@@ -1239,14 +1284,14 @@ __device__ __forceinline__ void update_on_add(Ctx<KMAX>& C, uint32_t ind, int mo
     for (int c = threadIdx.x; c <= col; c += BMG_BLOCK) S.work[c] = (double)S.iacc2[c];
     __syncthreads();
   } else {
-    new_column_dots(C, ind, coding, col, C.A.xcol + (size_t)slot * C.D.W32);
+    new_column_dots(C, ind, coding, col, gp(C.A.xcol) + (size_t)slot * C.D.W32);
   }
   const uint64_t tc = wall_clock64();
   // record the new X^T X row/column in the slot matrix
   for (int c = threadIdx.x; c <= col; c += BMG_BLOCK) {
     int sc = c == col ? slot : S.slot[c];
-    C.A.xxs[(size_t)slot * BMG_KMAXG + sc] = S.work[c];
-    C.A.xxs[(size_t)sc * BMG_KMAXG + slot] = S.work[c];
+    gp(C.A.xxs)[(size_t)slot * BMG_KMAXG + sc] = S.work[c];
+    gp(C.A.xxs)[(size_t)sc * BMG_KMAXG + slot] = S.work[c];
   }
   if (threadIdx.x == 0) S.xy[col] = xy;
   // the next addition of the move (next >= 0): its column's dots with every
@@ -1263,7 +1308,7 @@ __device__ __forceinline__ void update_on_add(Ctx<KMAX>& C, uint32_t ind, int mo
   if (wave_id() == 0) {
     trsv_ut_w0(S, S.L + P(col), col);
   } else if (nslot >= 0) {
-    uint32_t* xn = C.A.xcol + (size_t)nslot * C.D.W32;
+    uint32_t* xn = gp(C.A.xcol) + (size_t)nslot * C.D.W32;
     switch (C.D.type) {
       case 0: column_dots<KMAX, 0, 64, BMG_BLOCK - 64>(C, (uint64_t)next, col + 1, xn, S.iacc2); break;
       case 1: column_dots<KMAX, 1, 64, BMG_BLOCK - 64>(C, (uint64_t)next, col + 1, xn, S.iacc2); break;
@@ -1299,7 +1344,7 @@ __device__ __forceinline__ void update_on_add(Ctx<KMAX>& C, uint32_t ind, int mo
   R.ldq += 0.5 * log(dval);
   R.ldl += log(lcc);
   R.ll = finite_ll(R.ldq - R.ldl + C.K.minus_n_plus_nu_2 * log(R.syx));
-  if (threadIdx.x == 0 && C.prof) {
+  if (threadIdx.x == 0) {
     const uint64_t te = wall_clock64();
     C.prof[8] += tb - ta; C.prof[9] += tc - tb; C.prof[10] += td - tc; C.prof[11] += te - td;
     C.prof[12] += 1;
@@ -1354,7 +1399,7 @@ template <int KMAX>
 __device__ __forceinline__ void update_on_remove(Ctx<KMAX>& C, int x_ind, long long next = -1) {
   const uint64_t t0 = wall_clock64();
   update_on_remove_impl(C, x_ind, next);
-  if (threadIdx.x == 0 && C.prof) { C.prof[13] += 1; C.prof[14] += wall_clock64() - t0; }
+  if (threadIdx.x == 0) { C.prof[13] += 1; C.prof[14] += wall_clock64() - t0; }
 }
 
 template <int KMAX>
@@ -1393,7 +1438,7 @@ __device__ __forceinline__ void update_on_remove_impl(Ctx<KMAX>& C, int x_ind, l
     }
     auto ahead = [&]() {
       if (nslot < 0) return;
-      uint32_t* xn = C.A.xcol + (size_t)nslot * C.D.W32;
+      uint32_t* xn = gp(C.A.xcol) + (size_t)nslot * C.D.W32;
       switch (C.D.type) {
         case 0: column_dots<KMAX, 0, 64, BMG_BLOCK - 64>(C, (uint64_t)next, R.cols, xn, S.iacc2); break;
         case 1: column_dots<KMAX, 1, 64, BMG_BLOCK - 64>(C, (uint64_t)next, R.cols, xn, S.iacc2); break;
@@ -1406,7 +1451,7 @@ __device__ __forceinline__ void update_on_remove_impl(Ctx<KMAX>& C, int x_ind, l
     chol_downdate(S, k, x_ind, ahead);
     if (nslot >= 0) { R.pre_snp = next; R.pre_slot = nslot; }
     const uint64_t tb = wall_clock64();
-    if (threadIdx.x == 0 && C.prof) { C.prof[16] += tb - ta; C.prof[17] += wall_clock64() - tb; }
+    if (threadIdx.x == 0) { C.prof[16] += tb - ta; C.prof[17] += wall_clock64() - tb; }
     double ld = 0.0, vv = 0.0;
     for (int i = threadIdx.x; i < R.cols; i += BMG_BLOCK) {
       ld += log(S.L[P(i) + i]);
@@ -1477,7 +1522,7 @@ __device__ __forceinline__ void compute_log_likelihood(Ctx<KMAX>& C) {
   // matrix holds column j's entries), so the loads are in flight together
   if ((int)threadIdx.x < k) {
     const int j = (int)threadIdx.x;
-    const double* __restrict__ row = C.A.xxs + (size_t)S.slot[j] * BMG_KMAXG;
+    const double* __restrict__ row = gp(C.A.xxs) + (size_t)S.slot[j] * BMG_KMAXG;
     double* col = S.L + P(j);
     for (int i0 = 0; i0 <= j; i0 += 8) {
       double v[8];
@@ -1549,7 +1594,7 @@ __device__ __forceinline__ void commit(Ctx<KMAX>& C) {
   Smem<KMAX>& S = C.S;
   Reg& R = C.R;
   __syncthreads();
-  copy_factor(C.A.Lcur, S.L, P(R.lmin < R.cols ? R.lmin : R.cols), P(R.cols));
+  copy_factor(gp(C.A.Lcur), S.L, P(R.lmin < R.cols ? R.lmin : R.cols), P(R.cols));
   for (int i = threadIdx.x; i < R.cols; i += BMG_BLOCK) {
     S.c_xy[i] = S.xy[i]; S.c_v[i] = S.v[i]; S.c_d[i] = S.d[i];
     S.c_slot[i] = S.slot[i]; S.c_snp[i] = S.snp[i]; S.c_xtype[i] = S.xtype[i];
@@ -1558,9 +1603,9 @@ __device__ __forceinline__ void commit(Ctx<KMAX>& C) {
     S.c_loci[i] = S.loci[i]; S.c_xi1[i] = S.xi1[i]; S.c_xi2[i] = S.xi2[i]; S.c_tind[i] = S.tind[i];
   }
   // current model_inds: removed loci first, then the positions of all loci
-  for (int i = threadIdx.x; i < R.n_rm; i += BMG_BLOCK) C.A.model_inds[S.rm_list[i]] = -1;
+  for (int i = threadIdx.x; i < R.n_rm; i += BMG_BLOCK) gp(C.A.model_inds)[S.rm_list[i]] = -1;
   __syncthreads();
-  for (int i = threadIdx.x; i < R.nloci; i += BMG_BLOCK) C.A.model_inds[S.loci[i]] = i;
+  for (int i = threadIdx.x; i < R.nloci; i += BMG_BLOCK) gp(C.A.model_inds)[S.loci[i]] = i;
   if (threadIdx.x < (KMAX + 63) / 64) S.slots_cur[threadIdx.x] = S.slots_prop[threadIdx.x];
   __syncthreads();
   R.c_cols = R.cols; R.c_nloci = R.nloci;
@@ -1576,7 +1621,7 @@ __device__ __forceinline__ void restore(Ctx<KMAX>& C) {
   Reg& R = C.R;
   __syncthreads();
   int lm = R.lmin < R.c_cols ? R.lmin : R.c_cols;
-  copy_factor(S.L, C.A.Lcur, P(lm), P(R.c_cols));
+  copy_factor(S.L, gp(C.A.Lcur), P(lm), P(R.c_cols));
   for (int i = threadIdx.x; i < R.c_cols; i += BMG_BLOCK) {
     S.xy[i] = S.c_xy[i]; S.v[i] = S.c_v[i]; S.d[i] = S.c_d[i];
     S.slot[i] = S.c_slot[i]; S.snp[i] = S.c_snp[i]; S.xtype[i] = S.c_xtype[i];
@@ -1681,9 +1726,9 @@ __device__ __forceinline__ void xbeta_impl(Ctx<KMAX>& C, const double* coef, int
   const double b0 = coef[0];
   const int me = C.D.me;
   const uint32_t n = C.D.n, W = C.D.W32;
-  const uint32_t* __restrict__ xcol = C.A.xcol;
-  const double* __restrict__ y = C.D.y;
-  double* __restrict__ yhat = C.A.y_hat;
+  const uint32_t* __restrict__ xcol = gp(C.A.xcol);
+  const double* __restrict__ y = gp(C.D.y);
+  double* __restrict__ yhat = gp(C.A.y_hat);
   double sxb = 0, sxb2 = 0, sy = 0, sy2 = 0, syx = 0, se = 0, se2 = 0, srr = 0;
   for (uint32_t w = threadIdx.x; w * 16 < n; w += BMG_BLOCK) {
     double acc[16];
@@ -1718,7 +1763,7 @@ __device__ __forceinline__ void xbeta_impl(Ctx<KMAX>& C, const double* coef, int
         sxb += a; sxb2 += a * a;
         // E beta_E of this individual in column order (the constant first)
         double e = b0;
-        for (int c = 1; c < me; ++c) e = e + C.D.E[(size_t)(c - 1) * C.D.n_pad + i] * coef[c];
+        for (int c = 1; c < me; ++c) e = e + gp(C.D.E)[(size_t)(c - 1) * C.D.n_pad + i] * coef[c];
         se += e; se2 += e * e;
         // with covariates and no loci the reference adds E beta_E to the
         // y_hat it holds (src/model.hpp:369-373 leaves the genetic part
@@ -1891,10 +1936,12 @@ __device__ __forceinline__ void sample_alpha_and_tau2(Ctx<KMAX>& C) {
 }
 
 // ---------------------------------------------------------------- moves ---
+// first i with u * cumsum[m - 1] < cumsum[i], m <= 64 (a lane per entry)
 __device__ __forceinline__ int sample_naive(const double* cumsum, int m, double u) {
-  double r = u * cumsum[m - 1];
-  for (int i = 0; i < m; ++i) if (r < cumsum[i]) return i;
-  return m - 1;
+  const int lane = lane_id();
+  const double r = u * cumsum[m - 1];
+  const unsigned long long b = __ballot(lane < m && r < cumsum[lane < m ? lane : 0]);
+  return b ? __ffsll((long long)b) - 1 : m - 1;
 }
 
 template <int KMAX>
@@ -2079,7 +2126,8 @@ __device__ __forceinline__ double exh_moveleft(Smem<KMAX>& S, const ChainConst& 
 // inlined, its registers crowd the kernel's hot loops.
 template <int KMAX>
 __device__ __noinline__ double exh_walk(Smem<KMAX>& S, const ChainConst& K, Exh X, int n,
-                                        double ll0, double* lp) {
+                                        double ll0, double* lp_any) {
+  double* lp = gp(lp_any);
   const bool st = lane_id() == 0;
   uint32_t ci[BMG_DR_MAX + 2];   // walk order; indexed only through `sel`/`put`
   for (int i = 0; i < BMG_DR_MAX + 2; ++i) ci[i] = (uint32_t)i;
@@ -2321,7 +2369,7 @@ __device__ __forceinline__ uint64_t dr_second_stage(Ctx<KMAX>& C, int n, double 
 template <int KMAX>
 __device__ __forceinline__ bool readd_removed(Ctx<KMAX>& C, uint64_t ind) {
   Smem<KMAX>& S = C.S;
-  const int mi = C.A.model_inds[ind];
+  const int mi = gp(C.A.model_inds)[ind];
   const int t_ind = S.c_tind[mi];
   double d2[2];
   d2[0] = S.c_d[S.c_xi1[mi]];
@@ -2348,7 +2396,7 @@ __device__ __forceinline__ void dr_keep(Ctx<KMAX>& C, int cl, int n, uint64_t sm
 // proposal probability, and one is drawn.  Returns the number of moved SNPs
 // kept (0: the current model stays).
 template <int KMAX>
-__device__ __forceinline__ int dr_addrem(Ctx<KMAX>& C, int ms, double* adapt) {
+__device__ __forceinline__ int dr_addrem(Ctx<KMAX>& C, int ms) {
   Smem<KMAX>& S = C.S;
   Reg& R = C.R;
   int ms_rem = 0;
@@ -2360,7 +2408,7 @@ __device__ __forceinline__ int dr_addrem(Ctx<KMAX>& C, int ms, double* adapt) {
   bool ok = true;
   for (int i = 0; i < ms && ok; ++i) {
     const uint64_t ind = S.mi[i];
-    if (S.mi_isadd[i]) { z_add += C.A.q_add[ind]; z_rem -= C.A.q_rem[ind]; }
+    if (S.mi_isadd[i]) { z_add += gp(C.A.q_add)[ind]; z_rem -= gp(C.A.q_rem)[ind]; }
     else ok = readd_removed(C, ind);
   }
   if (!ok) { restore(C); undo_dd(C, ms); return 0; }
@@ -2369,18 +2417,18 @@ __device__ __forceinline__ int dr_addrem(Ctx<KMAX>& C, int ms, double* adapt) {
     const int pos = find_locus(C, ind);
     if (threadIdx.x == 0 && pos >= cl && pos - cl < ms) {
       S.ex_b2n[pos - cl] = (uint8_t)i;
-      S.dq_add[i] = C.A.q_add[ind];
-      S.dq_rem[i] = C.A.q_rem[ind];
+      S.dq_add[i] = gp(C.A.q_add)[ind];
+      S.dq_rem[i] = gp(C.A.q_rem)[ind];
     }
   }
   __syncthreads();
-  double* lp = C.A.dr_lp;
+  double* lp = gp(C.A.dr_lp);
   const uint64_t t0 = wall_clock64();
   const double max_log = exhaustive_modelset(C, cl, ms, lp);
   dr_proposal_probs(S, ms, z_add, z_rem, (uint64_t)cl, C.D.p, lp);
   __syncthreads();
   const uint64_t sm = dr_second_stage(C, ms, max_log, lp);
-  if (threadIdx.x == 0 && C.prof) C.prof[19] += wall_clock64() - t0;
+  if (threadIdx.x == 0) C.prof[19] += wall_clock64() - t0;
   if (sm == ((~nmb) & mask)) { restore(C); undo_dd(C, ms); return 0; }
   int moved = 0;
   for (int i = 0; i < ms; ++i) {
@@ -2391,7 +2439,7 @@ __device__ __forceinline__ int dr_addrem(Ctx<KMAX>& C, int ms, double* adapt) {
     else { tree_set(C, 0, ind, 0); tree_set(C, 1, ind, 1); }
   }
   dr_keep(C, cl, ms, sm);
-  if (threadIdx.x == 0) adapt[3 * 256 + ms - 1] += (double)moved / (double)ms;
+  if (threadIdx.x == 0) S.r_ms_sum[ms - 1] += (double)moved / (double)ms;
   commit(C);
   return moved;
 }
@@ -2406,13 +2454,13 @@ __device__ __forceinline__ int dr_statechange(Ctx<KMAX>& C, int ms, int ms_add, 
   const uint64_t nmb = (1ull << ms_add) - 1, mask = (1ull << ms) - 1;
   for (int i = 0; i < ms_rem; ++i)
     if (!readd_removed(C, S.mi_rem[i])) { restore(C); return 0; }
-  double* lp = C.A.dr_lp;
+  double* lp = gp(C.A.dr_lp);
   const uint64_t t0 = wall_clock64();
   const double max_log = exhaustive_modelset(C, cl, ms, lp);
   for (uint64_t i = threadIdx.x; i <= mask; i += BMG_BLOCK) lp[i] -= log((double)(cl + __popcll(i)));
   __syncthreads();
   const uint64_t sm = dr_second_stage(C, ms, max_log, lp);
-  if (threadIdx.x == 0 && C.prof) C.prof[19] += wall_clock64() - t0;
+  if (threadIdx.x == 0) C.prof[19] += wall_clock64() - t0;
   if (sm == ((~nmb) & mask)) { restore(C); return 0; }
   int moved = 0;
   for (int i = 0; i < ms; ++i) {
@@ -2429,13 +2477,13 @@ __device__ __forceinline__ int dr_statechange(Ctx<KMAX>& C, int ms, int ms_add, 
 
 // src/sampler.hpp:899-1123
 template <int KMAX>
-__device__ __forceinline__ int move_addrem(Ctx<KMAX>& C, double* adapt) {
+__device__ __forceinline__ int move_addrem(Ctx<KMAX>& C) {
   Smem<KMAX>& S = C.S;
   Reg& R = C.R;
   const ChainConst& K = C.K;
   const int type = C.D.type;
   int max_ms = (int)K.max_ms;
-  int ms = sample_naive(adapt, max_ms, rng_u01(R.rng)) + 1;
+  int ms = sample_naive(S.cdf[0], max_ms, rng_u01(R.rng)) + 1;
   R.movesize = ms;
   double lqf = 0, lqb = 0, lmpc = 0;
   // the move's tree writes are journalled, so a rejection puts the trees
@@ -2518,10 +2566,10 @@ __device__ __forceinline__ int move_addrem(Ctx<KMAX>& C, double* adapt) {
         int lr = ms - 1, seen = 0;
         for (;; --lr) if (S.mi_isadd[lr] && seen++ == k) break;
         ind = (uint64_t)S.mi_map[lr];
-        S.bq[i] = C.A.q_rem[ind];
+        S.bq[i] = gp(C.A.q_rem)[ind];
       } else {
         ind = (uint64_t)S.mi_map[i];
-        S.bq[i] = C.A.q_add[ind];
+        S.bq[i] = gp(C.A.q_add)[ind];
       }
     }
     __syncthreads();
@@ -2545,33 +2593,31 @@ __device__ __forceinline__ int move_addrem(Ctx<KMAX>& C, double* adapt) {
   double log_r = lqb - lqf;
   log_r += lmpc + R.ll - R.c_ll;
   const uint64_t tq4 = wall_clock64();
-  if (threadIdx.x == 0 && C.prof) {
+  if (threadIdx.x == 0) {
     C.prof[20] += tq2 - tq1; C.prof[21] += tq3 - tq2; C.prof[22] += tq4 - tq3; C.prof[23] += tq1 - tq0;
   }
-  double* r_ms_sum = adapt + 3 * 256;
-  double* r_ms_n = adapt + 4 * 256;
   if (threadIdx.x == 0) {
-    if (K.dr == 0) r_ms_sum[ms - 1] += (log_r >= 0 ? 1.0 : exp(log_r));
-    r_ms_n[ms - 1] += 1.0;
+    if (K.dr == 0) S.r_ms_sum[ms - 1] += (log_r >= 0 ? 1.0 : exp(log_r));
+    S.r_ms_n[ms - 1] += 1.0;
   }
   if (log_r >= 0 || log(rng_u01(R.rng)) <= log_r) {
     R.tj_on = 0;
     commit(C);
-    if (K.dr != 0 && threadIdx.x == 0) r_ms_sum[ms - 1] += 1.0;
-    if (threadIdx.x == 0 && C.prof) C.prof[23] += wall_clock64() - tq4;
+    if (K.dr != 0 && threadIdx.x == 0) S.r_ms_sum[ms - 1] += 1.0;
+    if (threadIdx.x == 0) C.prof[23] += wall_clock64() - tq4;
     return ms;
   }
   // a proposal past the compiled capacity has no second stage
   if (ms <= K.dr && ms > 1 && !(R.err & ERR_CAPACITY)) {
     R.tj_on = 0;
     const uint64_t t0 = wall_clock64();
-    const int moved = dr_addrem(C, ms, adapt);
-    if (threadIdx.x == 0 && C.prof) C.prof[18] += wall_clock64() - t0;
+    const int moved = dr_addrem(C, ms);
+    if (threadIdx.x == 0) C.prof[18] += wall_clock64() - t0;
     return moved;
   }
   restore(C);
   journal_restore(C);
-  if (threadIdx.x == 0 && C.prof) C.prof[23] += wall_clock64() - tq4;
+  if (threadIdx.x == 0) C.prof[23] += wall_clock64() - tq4;
   return 0;
 }
 
@@ -2581,7 +2627,7 @@ __device__ __forceinline__ int cur_in_model(Ctx<KMAX>& C, int64_t j, int64_t wba
   if (j < 0 || j >= (int64_t)C.D.p) return 0;   // outside the genome: stops a walk
   for (int q = 0; q < C.R.n_marks; ++q) if ((int64_t)C.S.marks[q] == j) return 1;
   if (j >= wbase && j < wbase + 512) return C.S.win[j - wbase] >= 0;
-  return C.A.model_inds[j] >= 0;
+  return gp(C.A.model_inds)[j] >= 0;
 }
 
 template <int KMAX>
@@ -2591,7 +2637,7 @@ __device__ __forceinline__ void load_window(Ctx<KMAX>& C, int64_t center, int64_
   __syncthreads();
   for (int t = threadIdx.x; t < 512; t += BMG_BLOCK) {
     int64_t j = b + t;
-    C.S.win[t] = (j < (int64_t)C.D.p) ? C.A.model_inds[j] : -1;
+    C.S.win[t] = (j < (int64_t)C.D.p) ? gp(C.A.model_inds)[j] : -1;
   }
   __syncthreads();
   *wbase = b;
@@ -2599,7 +2645,7 @@ __device__ __forceinline__ void load_window(Ctx<KMAX>& C, int64_t center, int64_
 
 // src/sampler.hpp:1271-1418
 template <int KMAX>
-__device__ __forceinline__ int move_switch(Ctx<KMAX>& C, double* adapt) {
+__device__ __forceinline__ int move_switch(Ctx<KMAX>& C) {
   Smem<KMAX>& S = C.S;
   Reg& R = C.R;
   const ChainConst& K = C.K;
@@ -2607,7 +2653,7 @@ __device__ __forceinline__ int move_switch(Ctx<KMAX>& C, double* adapt) {
   uint64_t mm2 = (K.max_ms + 1) / 2;
   uint64_t mx = mm2 < (full + 1) / 2 ? mm2 : (full + 1) / 2;
   mx = mx < (uint64_t)R.c_nloci ? mx : (uint64_t)R.c_nloci;
-  int ms = sample_naive(adapt + 256, (int)mx, rng_u01(R.rng)) + 1;
+  int ms = sample_naive(S.cdf[1], (int)mx, rng_u01(R.rng)) + 1;
   R.movesize = ms;
   uint64_t nbh = (full - ms) / 2;
   if (nbh < 1) nbh = 1;
@@ -2719,7 +2765,7 @@ __device__ __forceinline__ int move_learned_swap(Ctx<KMAX>& C) {
   if (threadIdx.x < 2 * H) {
     int64_t k = j + lw_off(H, threadIdx.x);
     double w = 0.0;
-    if (k >= 0 && k < m_g && C.A.model_inds[k] < 0) w = (double)C.D.lw[(size_t)j * 2 * H + threadIdx.x];
+    if (k >= 0 && k < m_g && gp(C.A.model_inds)[k] < 0) w = (double)gp(C.D.lw)[(size_t)j * 2 * H + threadIdx.x];
     wf[threadIdx.x] = w;
   }
   __syncthreads();
@@ -2742,8 +2788,8 @@ __device__ __forceinline__ int move_learned_swap(Ctx<KMAX>& C) {
   if (threadIdx.x < 2 * H) {
     int64_t q = k + lw_off(H, threadIdx.x);
     double w = 0.0;
-    if (q >= 0 && q < m_g && (q == j || C.A.model_inds[q] < 0))
-      w = (double)C.D.lw[(size_t)k * 2 * H + threadIdx.x];
+    if (q >= 0 && q < m_g && (q == j || gp(C.A.model_inds)[q] < 0))
+      w = (double)gp(C.D.lw)[(size_t)k * 2 * H + threadIdx.x];
     wr[threadIdx.x] = w;
   }
   __syncthreads();
@@ -2772,7 +2818,7 @@ __device__ __forceinline__ int move_learned_swap(Ctx<KMAX>& C) {
 
 // src/sampler.hpp:1421-1669
 template <int KMAX>
-__device__ __forceinline__ int move_statechange(Ctx<KMAX>& C, double* adapt) {
+__device__ __forceinline__ int move_statechange(Ctx<KMAX>& C) {
   Smem<KMAX>& S = C.S;
   Reg& R = C.R;
   const ChainConst& K = C.K;
@@ -2780,7 +2826,7 @@ __device__ __forceinline__ int move_statechange(Ctx<KMAX>& C, double* adapt) {
   uint64_t m_g = C.D.p;
   uint64_t a = (uint64_t)K.max_nbh * 2, b = m_g - 1 < K.max_ms ? m_g - 1 : K.max_ms;
   uint64_t mx = a < b ? a : b;
-  int ms = sample_naive(adapt + 2 * 256, (int)mx, rng_u01(R.rng)) + 1;
+  int ms = sample_naive(S.cdf[2], (int)mx, rng_u01(R.rng)) + 1;
   R.movesize = ms;
   uint64_t nbh = K.max_nbh < m_g / 2 ? K.max_nbh : m_g / 2;
   int mic = (int)floor(rng_u01(R.rng) * R.nloci);
@@ -2857,7 +2903,7 @@ __device__ __forceinline__ int move_statechange(Ctx<KMAX>& C, double* adapt) {
   if (ms <= K.dr && ms > 1 && !(R.err & ERR_CAPACITY)) {
     const uint64_t t0 = wall_clock64();
     const int moved = dr_statechange(C, ms, ms_add, ms_rem);
-    if (threadIdx.x == 0 && C.prof) C.prof[18] += wall_clock64() - t0;
+    if (threadIdx.x == 0) C.prof[18] += wall_clock64() - t0;
     return moved;
   }
   restore(C);
@@ -2865,10 +2911,8 @@ __device__ __forceinline__ int move_statechange(Ctx<KMAX>& C, double* adapt) {
 }
 
 // src/sampler.hpp:1728-1769
-__device__ __forceinline__ void adapt_jd_mb(double* p_ms, double* adapt, int max_ms) {
-  double* q_p0 = adapt + 5 * 256;
-  const double* r_ms = adapt + 3 * 256;
-  const double* r_n = adapt + 4 * 256;
+__device__ __forceinline__ void adapt_jd_mb(double* p_ms, double* q_p0, const double* r_ms, const double* r_n,
+                                            int max_ms) {
   double q = 1 - *p_ms;
   double zp = 1 - pow(q, max_ms);
   double q_p = *p_ms / zp;
@@ -2897,6 +2941,27 @@ __device__ __forceinline__ void geometric_cdf(int maxsize, double p, double* val
 
 // --------------------------------------------------------------- kernel ---
 
+// the descriptions of the chain's dataset, options and arrays into LDS
+template <typename T>
+__device__ __forceinline__ void copy_words(T& dst, const T* src) {
+  static_assert(sizeof(T) % 4 == 0, "whole words");
+  uint32_t* d = (uint32_t*)&dst;
+  const uint32_t* w = (const uint32_t*)src;
+  for (int i = threadIdx.x; i < (int)(sizeof(T) / 4); i += BMG_BLOCK) d[i] = w[i];
+}
+template <int KMAX>
+__device__ __forceinline__ void load_descriptions(Smem<KMAX>& S, const DevData* data, const ChainConst* K,
+                                                  const ChainArrays* A) {
+  copy_words(S.K, K);
+  copy_words(S.A, A);
+  copy_words(S.D, data + K->ds);
+  __syncthreads();
+  if constexpr (KMAX > KMAX_LDS) {
+    if (threadIdx.x == 0) S.L.p = S.A.Lwork;
+    __syncthreads();
+  }
+}
+
 template <int KMAX>
 __device__ __forceinline__ void load_chain(Ctx<KMAX>& C, const ChainScal& CS) {
   Smem<KMAX>& S = C.S;
@@ -2914,12 +2979,28 @@ __device__ __forceinline__ void load_chain(Ctx<KMAX>& C, const ChainScal& CS) {
   R.lmin = KMAX; R.n_rm = 0; R.n_marks = 0; R.movesize = CS.movesize;
   R.tot_add = CS.tot_add; R.tot_rem = CS.tot_rem;
   R.err = CS.err;
+  if (threadIdx.x < 24) S.prof[threadIdx.x] = CS.prof[threadIdx.x];
+  if (threadIdx.x < 4) {
+    S.cnt.n_acpt[threadIdx.x] = CS.n_acpt[threadIdx.x];
+    S.cnt.n_moves[threadIdx.x] = CS.n_moves[threadIdx.x];
+  }
+  if (threadIdx.x == 0) {
+    S.cnt.n_accepted = CS.n_accepted;
+    S.cnt.tr_count = CS.tr_count; S.cnt.th_count = CS.th_count;
+    S.cnt.th_loci_len = CS.th_loci_len; S.cnt.th_beta_len = CS.th_beta_len;
+  }
+  if (threadIdx.x < BMG_MAXMS) {
+    const double* ad = gp(C.A.adapt) + threadIdx.x;
+    for (int q = 0; q < 3; ++q) S.cdf[q][threadIdx.x] = ad[q * 256];
+    S.r_ms_sum[threadIdx.x] = ad[3 * 256];
+    S.r_ms_n[threadIdx.x] = ad[4 * 256];
+  }
   R.learn_on = CS.learn_on && C.D.lw != nullptr && C.D.lH >= 1 && C.D.lH <= BMG_LH_MAX;
   R.tj_on = 0; R.tj_n = 0; R.tj_tot[0] = R.tj_tot[1] = 0.0;
   R.pre_snp = -1; R.pre_slot = -1;
-  const double* vec = C.A.vec;
-  const int32_t* idx = C.A.idx;
-  for (int e = threadIdx.x; e < P(R.cols); e += BMG_BLOCK) S.L[e] = C.A.Lcur[e];
+  const double* vec = gp(C.A.vec);
+  const int32_t* idx = gp(C.A.idx);
+  for (int e = threadIdx.x; e < P(R.cols); e += BMG_BLOCK) S.L[e] = gp(C.A.Lcur)[e];
   for (int i = threadIdx.x; i < KMAX; i += BMG_BLOCK) {
     S.xy[i] = S.c_xy[i] = vec[i];
     S.v[i] = S.c_v[i] = vec[BMG_KMAXG + i];
@@ -2944,8 +3025,8 @@ __device__ __forceinline__ void load_chain(Ctx<KMAX>& C, const ChainScal& CS) {
   if (C.D.top >= 2) {
     uint64_t o2 = C.D.lev_off[2];
     for (uint64_t e = threadIdx.x; e < C.D.lds_lev_size; e += BMG_BLOCK) {
-      S.tlev[0][e] = C.A.tree_add[o2 + e];
-      S.tlev[1][e] = C.A.tree_rem[o2 + e];
+      S.tlev[0][e] = gp(C.A.tree_add)[o2 + e];
+      S.tlev[1][e] = gp(C.A.tree_rem)[o2 + e];
     }
   }
   __syncthreads();
@@ -2956,8 +3037,8 @@ __device__ __forceinline__ void store_chain(Ctx<KMAX>& C, ChainScal& CS) {
   Smem<KMAX>& S = C.S;
   Reg& R = C.R;
   __syncthreads();
-  double* vec = C.A.vec;
-  int32_t* idx = C.A.idx;
+  double* vec = gp(C.A.vec);
+  int32_t* idx = gp(C.A.idx);
   for (int i = threadIdx.x; i < KMAX; i += BMG_BLOCK) {
     vec[i] = S.c_xy[i]; vec[BMG_KMAXG + i] = S.c_v[i]; vec[2 * BMG_KMAXG + i] = S.c_d[i];
     vec[3 * BMG_KMAXG + i] = S.beta[i]; vec[4 * BMG_KMAXG + i] = S.mu[i];
@@ -2968,8 +3049,8 @@ __device__ __forceinline__ void store_chain(Ctx<KMAX>& C, ChainScal& CS) {
   if (C.D.top >= 2) {
     uint64_t o2 = C.D.lev_off[2];
     for (uint64_t e = threadIdx.x; e < C.D.lds_lev_size; e += BMG_BLOCK) {
-      C.A.tree_add[o2 + e] = S.tlev[0][e];
-      C.A.tree_rem[o2 + e] = S.tlev[1][e];
+      gp(C.A.tree_add)[o2 + e] = S.tlev[0][e];
+      gp(C.A.tree_rem)[o2 + e] = S.tlev[1][e];
     }
   }
   if (threadIdx.x == 0) {
@@ -2983,6 +3064,19 @@ __device__ __forceinline__ void store_chain(Ctx<KMAX>& C, ChainScal& CS) {
     CS.movesize = R.movesize;
     CS.tot_add = R.tot_add; CS.tot_rem = R.tot_rem;
     CS.err = R.err;
+    CS.n_accepted = S.cnt.n_accepted;
+    CS.tr_count = S.cnt.tr_count; CS.th_count = S.cnt.th_count;
+    CS.th_loci_len = S.cnt.th_loci_len; CS.th_beta_len = S.cnt.th_beta_len;
+  }
+  if (threadIdx.x < 24) CS.prof[threadIdx.x] = S.prof[threadIdx.x];
+  if (threadIdx.x < 4) {
+    CS.n_acpt[threadIdx.x] = S.cnt.n_acpt[threadIdx.x];
+    CS.n_moves[threadIdx.x] = S.cnt.n_moves[threadIdx.x];
+  }
+  if (threadIdx.x < BMG_MAXMS) {
+    double* ad = gp(C.A.adapt) + threadIdx.x;
+    ad[3 * 256] = S.r_ms_sum[threadIdx.x];
+    ad[4 * 256] = S.r_ms_n[threadIdx.x];
   }
   __syncthreads();
 }
@@ -3001,7 +3095,7 @@ __device__ __forceinline__ void refresh_tau2(Ctx<KMAX>& C) {
   for (int q = 0; q < 4; ++q) ita[q] = R.ita2[q];
   const uint64_t t0 = wall_clock64();
   sample_alpha_and_tau2(C);
-  if (threadIdx.x == 0 && C.prof) C.prof[15] += wall_clock64() - t0;
+  if (threadIdx.x == 0) C.prof[15] += wall_clock64() - t0;
   compute_log_likelihood(C);
   R.lmin = 0;
   if (isfinite(R.ll)) {
@@ -3019,7 +3113,7 @@ __device__ __forceinline__ void run_iterations(Ctx<KMAX>& C, ChainScal& CS, uint
   Smem<KMAX>& S = C.S;
   Reg& R = C.R;
   const ChainConst& K = C.K;
-  double* adapt = C.A.adapt;
+  double* adapt = gp(C.A.adapt);
   uint64_t it0 = CS.n_iter;
   uint64_t pr[8] = {0, 0, 0, 0, 0, 0, 0, 0};
   for (uint64_t iter = it0; iter < it0 + n_iter; ++iter) {
@@ -3033,7 +3127,7 @@ __device__ __forceinline__ void run_iterations(Ctx<KMAX>& C, ChainScal& CS, uint
       if (threadIdx.x == 0) {
         CS.big = 1;
 #pragma unroll
-        for (int q = 0; q < 8; ++q) CS.prof[q] += pr[q];
+        for (int q = 0; q < 8; ++q) S.prof[q] += pr[q];
       }
       break;
     }
@@ -3059,11 +3153,11 @@ __device__ __forceinline__ void run_iterations(Ctx<KMAX>& C, ChainScal& CS, uint
     int jd = 0;
     if (move == 3) {
       if (R.c_nloci > 0) jd = move_learned_swap(C);
-    } else if (move == 0) jd = move_addrem(C, adapt);
+    } else if (move == 0) jd = move_addrem(C);
     else if (move == 1) {
-      if (R.c_nloci > 0 && (uint64_t)R.c_nloci < C.D.p - 1) jd = move_switch(C, adapt);
+      if (R.c_nloci > 0 && (uint64_t)R.c_nloci < C.D.p - 1) jd = move_switch(C);
     } else {
-      if (R.c_nloci > 0 && C.D.p > 2) jd = move_statechange(C, adapt);
+      if (R.c_nloci > 0 && C.D.p > 2) jd = move_statechange(C);
     }
     {
       const uint64_t t1 = wall_clock64(), dt = t1 - t0;
@@ -3074,43 +3168,43 @@ __device__ __forceinline__ void run_iterations(Ctx<KMAX>& C, ChainScal& CS, uint
       t0 = t1;
     }
     if (threadIdx.x == 0) {
-      CS.n_moves[move]++;
-      CS.n_acpt[move] += jd > 0;
-      CS.n_accepted += jd > 0;
+      S.cnt.n_moves[move]++;
+      S.cnt.n_acpt[move] += jd > 0;
+      S.cnt.n_accepted += jd > 0;
     }
     if ((iter + 1) % K.thin == 0 || (iter + 2) % K.n_st == 0) {
       sample_beta_sigma2(C);
       uint64_t t1 = wall_clock64(); pr[5] += t1 - t0; t0 = t1;
     }
     if (K.trace_iter && threadIdx.x == 0) {
-      uint64_t t = CS.tr_count;
+      uint64_t t = S.cnt.tr_count;
       if (t < K.tr_cap) {
-        C.A.tr_move[t] = (uint8_t)move; C.A.tr_jd[t] = (uint8_t)jd;
-        C.A.tr_ms[t] = (uint8_t)R.movesize; C.A.tr_size[t] = (uint32_t)R.c_nloci;
-        C.A.tr_ll[t] = R.c_ll;
+        gp(C.A.tr_move)[t] = (uint8_t)move; gp(C.A.tr_jd)[t] = (uint8_t)jd;
+        gp(C.A.tr_ms)[t] = (uint8_t)R.movesize; gp(C.A.tr_size)[t] = (uint32_t)R.c_nloci;
+        gp(C.A.tr_ll)[t] = R.c_ll;
       } else {
         R.err |= ERR_TRACE;
       }
-      CS.tr_count = t + 1;
+      S.cnt.tr_count = t + 1;
     }
     if ((iter + 1) % K.thin == 0) {
       double pves[3];
       compute_pve(C, pves);
       if (threadIdx.x == 0) {
-        uint64_t t = CS.th_count;
-        uint64_t ll0 = CS.th_loci_len;
+        uint64_t t = S.cnt.th_count;
+        uint64_t ll0 = S.cnt.th_loci_len;
         if (t < K.th_cap && ll0 + R.c_nloci <= K.th_loci_cap) {
-          C.A.th_size[t] = (uint32_t)R.c_nloci;
-          for (int q = 0; q < R.c_nloci; ++q) C.A.th_loci[ll0 + q] = S.c_loci[q];
-          C.A.th_ll[t] = R.c_ll; C.A.th_s2[t] = R.sigma2; C.A.th_alpha[t] = R.alpha;
-          C.A.th_pve[3 * t] = pves[0]; C.A.th_pve[3 * t + 1] = pves[1]; C.A.th_pve[3 * t + 2] = pves[2];
-          CS.th_count = t + 1; CS.th_loci_len = ll0 + R.c_nloci;
+          gp(C.A.th_size)[t] = (uint32_t)R.c_nloci;
+          for (int q = 0; q < R.c_nloci; ++q) gp(C.A.th_loci)[ll0 + q] = S.c_loci[q];
+          gp(C.A.th_ll)[t] = R.c_ll; gp(C.A.th_s2)[t] = R.sigma2; gp(C.A.th_alpha)[t] = R.alpha;
+          gp(C.A.th_pve)[3 * t] = pves[0]; gp(C.A.th_pve)[3 * t + 1] = pves[1]; gp(C.A.th_pve)[3 * t + 2] = pves[2];
+          S.cnt.th_count = t + 1; S.cnt.th_loci_len = ll0 + R.c_nloci;
           // save_beta (src/sampler.cpp:710-713): the beta drawn for this sample
           if (K.th_beta_cap) {
-            const uint64_t b0 = CS.th_beta_len;
+            const uint64_t b0 = S.cnt.th_beta_len;
             if (b0 + R.beta_len <= K.th_beta_cap) {
-              for (int q = 0; q < R.beta_len; ++q) C.A.th_beta[b0 + q] = S.beta[q];
-              CS.th_beta_len = b0 + R.beta_len;
+              for (int q = 0; q < R.beta_len; ++q) gp(C.A.th_beta)[b0 + q] = S.beta[q];
+              S.cnt.th_beta_len = b0 + R.beta_len;
             } else {
               R.err |= ERR_TRACE;
             }
@@ -3126,7 +3220,7 @@ __device__ __forceinline__ void run_iterations(Ctx<KMAX>& C, ChainScal& CS, uint
     if ((iter + 1) % K.n_rao == 0 || iter + 1 == it0 + n_iter) {
       if (threadIdx.x == 0) {
 #pragma unroll
-        for (int q = 0; q < 8; ++q) CS.prof[q] += pr[q];
+        for (int q = 0; q < 8; ++q) S.prof[q] += pr[q];
       }
 #pragma unroll
       for (int q = 0; q < 8; ++q) pr[q] = 0;
@@ -3157,13 +3251,13 @@ __device__ __forceinline__ void run_iterations(Ctx<KMAX>& C, ChainScal& CS, uint
           if (K.adapt_p_ms) {
             if (K.acpt_goal > 0) {
               double t = fmax(1.0, K.k_move_size * (double)CS.p_proposal_n);
-              double ar = (double)CS.n_acpt[0] / (double)CS.n_moves[0];
+              double ar = (double)S.cnt.n_acpt[0] / (double)S.cnt.n_moves[0];
               double pm2 = CS.p_ms + (K.acpt_goal - ar) / (2.0 + t);
               CS.p_ms = fmax(fmin(pm2, 0.99), 0.01);
-              CS.n_acpt[0] = 1; CS.n_moves[0] = 2;
+              S.cnt.n_acpt[0] = 1; S.cnt.n_moves[0] = 2;
             } else {
               double pms = CS.p_ms;
-              adapt_jd_mb(&pms, adapt, (int)K.max_ms);
+              adapt_jd_mb(&pms, adapt + 5 * 256, S.r_ms_sum, S.r_ms_n, (int)K.max_ms);
               CS.p_ms = pms;
             }
             geometric_cdf((int)K.max_ms, CS.p_ms, adapt);
@@ -3186,15 +3280,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
   int c = blockIdx.x;
   if (c >= args.n_chains) return;
   ChainScal& CS = args.scal[c];
-  const ChainConst& K = args.consts[c];
-  const DevData& D = args.data[K.ds];
-  const ChainArrays& A = args.arrays[c];
-  if constexpr (KMAX > KMAX_LDS) {
-    if (threadIdx.x == 0) S.L = A.Lwork;
-    __syncthreads();
-  }
+  load_descriptions(S, args.data, args.consts + c, args.arrays + c);
   Reg R;
-  Ctx<KMAX> C{S, R, D, K, A, CS.prof};
+  Ctx<KMAX> C{S, R, S.D, S.K, S.A, S.prof};
   if (args.mode == 1) {
     // setup (src/sampler.cpp:591-620): state was initialised on the host
     // with an empty model; compute its factor, then sample
@@ -3224,7 +3312,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
     // every column's slot exists there
     int top = 0;
     for (int i = 0; i < R.c_cols; ++i) top = max(top, (int)S.c_slot[i]);
-    if (!(R.err & ERR_STOP) && R.c_cols + K.col_reserve + 8 <= args.small_kmax && top < args.small_kmax)
+    if (!(R.err & ERR_STOP) && R.c_cols + S.K.col_reserve + 8 <= args.small_kmax && top < args.small_kmax)
       CS.big = 0;
   }
 }
@@ -3279,15 +3367,9 @@ template <int KMAX>
 __global__ __launch_bounds__(256) void k_model_op(ModelOpArgs a) {
   __shared__ Smem<KMAX> S;
   ChainScal& CS = a.scal[0];
-  const ChainConst& K = a.consts[0];
-  const DevData& D = a.data[K.ds];
-  const ChainArrays& A = a.arrays[0];
-  if constexpr (KMAX > KMAX_LDS) {
-    if (threadIdx.x == 0) S.L = A.Lwork;
-    __syncthreads();
-  }
+  load_descriptions(S, a.data, a.consts, a.arrays);
   Reg R;
-  Ctx<KMAX> C{S, R, D, K, A, nullptr};
+  Ctx<KMAX> C{S, R, S.D, S.K, S.A, S.prof};
   load_chain(C, CS);
   R.err &= ~ERR_CAPACITY;   // a capacity error belongs to the call that hit it
   if (a.op == 0) {
