@@ -253,119 +253,155 @@ __device__ __forceinline__ double snp_dot_y(Ctx<KMAX>& C, uint64_t snp, int codi
   return dot_y_block(gp(C.D.g) + snp * C.D.W32, C.D.W32, gp(C.D.y), coding, C.S.red);
 }
 
-// value planes of a word under a coding known at compile time (CODING >= 0)
-// or given at run time (CODING < 0)
-template <int CODING>
-__device__ __forceinline__ void planes_c(uint32_t w, int coding, uint32_t& p1, uint32_t& p2) {
-  if (CODING < 0) {
-    planes(w, coding, p1, p2);
-  } else {
-    const uint32_t lo = w & BMG_EVEN, hi = (w >> 1) & BMG_EVEN;
-    if (CODING == 0) { p1 = hi; p2 = hi & lo; }
-    else if (CODING == 1) { p1 = hi & ~lo; p2 = 0u; }
-    else if (CODING == 2) { p1 = hi; p2 = 0u; }
-    else { p1 = hi & lo; p2 = 0u; }
-  }
+// value word of a packed word: the coded genotype (0..2) in each 2-bit field
+__device__ __forceinline__ uint32_t value_word(uint32_t w, int coding) {
+  const uint32_t lo = w & BMG_EVEN, hi = (w >> 1) & BMG_EVEN;
+  const uint32_t het = hi & ~lo, hom = hi & lo;
+  // A: het + 2 hom, H: het, D: het + hom, R: hom
+  const uint32_t one = (coding == 3 ? 0u : het) | (coding >= 2 ? hom : 0u);
+  return one | (coding == 0 ? hom << 1 : 0u);
 }
 
-// S.work[c] = x_c^T x_new for c in [0, cols], column `cols` being the new
-// one itself; column 0 is the constant.  Exact integer dots: the slot
-// copies of the model's columns hold value words (the coded genotype, 0..2,
-// in each 2-bit field), whose even fields (masked in place) and odd fields
-// (the rest, four times their value) meet the new column's in two 8-way
-// unsigned 4-bit dot products (v_dot8_u32_u4); the odd sum is divided by
-// four at the end.  The constant column and the new column's own dot come
-// from the new column's nibbles alone.
+// acc[c] = x_c^T x_new for the constant column c = 0, the model's columns c
+// in [me, cols) and the new column itself, c = cols (covariate columns:
+// cov_dots).  Exact integer dots: the slot copies of the model's columns hold
+// value words, whose even fields (masked in place) and odd fields (the rest,
+// four times their value) meet the new column's in two 8-way unsigned 4-bit
+// dot products (v_dot8_u32_u4); the odd sum is divided by four at the end.
 //
-// A lane owns one 16-word chunk of the individuals and a group of columns:
-// it decodes the new column's chunk once, then streams its columns' chunks,
-// four columns' words in flight at a time, each column's loads issued as
-// soon as the previous column in its register set is summed; the chunk
-// sums meet in LDS integer accumulators (exact, so the order is free).
-// W / 16 lanes cover a column, so NTH / (W / 16) column groups run side by
-// side; the first group also writes the new column's value words to its
-// slot copy (xnew).  CODING: the new column's coding; threads [T0, T0 + NTH)
-// take part (the whole workgroup, or waves 1-3 while wave 0 runs a
-// triangular sweep); acc: the integer accumulators, zeroed by the caller.
-template <int KMAX, int CODING, int T0, int NTH>
-__device__ __forceinline__ void column_dots(Ctx<KMAX>& C, uint64_t snp_new, int cols, uint32_t* __restrict__ xnew,
-                                            int32_t* acc) {
-  const uint32_t W = C.D.W32;                 // a multiple of 32 words
-  const uint32_t* __restrict__ wn = gp(C.D.g) + snp_new * W;
-  const uint32_t* __restrict__ xcol = gp(C.A.xcol);
+// A group of SPAN lanes (16, 32 or 64, as the columns are short or long)
+// holds NP pieces of 16 bytes a lane of the new column, decoded once, and
+// streams whole columns past them: consecutive lanes read consecutive 16
+// bytes, up to four columns' pieces are in flight while those before are
+// summed, and a column's sum meets in its group by DPP adds.  Bound by the
+// L2 reads of the columns (2,560 bytes each at n = 10,000).  (With a lane
+// reading 64 consecutive bytes, each load instruction touched 32 cache lines
+// for a quarter of their bytes, and 40 lanes added their sums to one LDS
+// word: 8.7 us per addition at 105 columns on four waves, 12 us on three.)
+// Columns longer than SPAN x NP pieces go in several passes.  Threads
+// [T0, T0 + NTH) take part (the whole workgroup, or waves 1-3 while wave 0
+// runs a triangular sweep); the first group also writes the new column's
+// value words to its slot copy xnew.
+template <int KMAX, int T0, int NTH, int SPAN, int NP>
+__device__ __forceinline__ void column_dots_np(Ctx<KMAX>& C, uint64_t snp_new, int coding, int cols,
+                                               uint32_t* __restrict__ xnew, int32_t* acc) {
+  constexpr int UC = NP > 3 ? 2 : 4;          // columns in flight
+  constexpr int GRP = NTH / SPAN;             // groups side by side
   Smem<KMAX>& S = C.S;
+  const uint32_t W = C.D.W32, W4 = W / 4;     // words and 16-byte pieces per column
+  const uint4* __restrict__ wn = (const uint4*)(gp(C.D.g) + snp_new * W);
+  const char* __restrict__ xcol = (const char*)gp(C.A.xcol);
   const int me = C.D.me;
-  const uint32_t cpc = W / 16;                // chunks per column
   const int tid = (int)threadIdx.x - T0;
-  if (tid < 0 || tid >= NTH) return;
-  for (uint32_t ch0 = 0; ch0 < cpc; ch0 += NTH) {
-    const uint32_t span = min(cpc - ch0, (uint32_t)NTH);
-    const int groups = (int)(NTH / span);
-    const int grp = (int)(tid / span);
-    const uint32_t w0 = (ch0 + tid % span) * 16;
-    if (grp < groups) {
-      uint32_t ne[16], no[16];   // the new column's even / odd fields as nibbles
-      uint32_t s_one = 0, s_self = 0;
+  const int grp = tid / SPAN, t = tid % SPAN;
+  auto group_sum = [](int v) -> int {         // valid in a group's last lane
+    v += dpp_i32<0x111, 0xf>(v);
+    v += dpp_i32<0x112, 0xf>(v);
+    v += dpp_i32<0x114, 0xf>(v);
+    v += dpp_i32<0x118, 0xf>(v);
+    if (SPAN > 16) v += dpp_i32<0x142, 0xa>(v);
+    if (SPAN > 32) v += dpp_i32<0x143, 0xc>(v);
+    return v;
+  };
+  for (uint32_t p0 = 0; p0 < W4; p0 += SPAN * NP) {
+    uint32_t ne[NP][4], no[NP][4];            // even / odd fields of the new column
+    uint32_t off[NP];                         // byte offset of this lane's pieces in a column
+    uint32_t s_one = 0, s_self = 0;
 #pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        const uint4 v = *(const uint4*)(wn + w0 + 4 * q);
-        const uint32_t xs[4] = {v.x, v.y, v.z, v.w};
-#pragma unroll
-        for (int u = 0; u < 4; ++u) {
-          uint32_t p1, p2;
-          planes_c<CODING>(xs[u], CODING, p1, p2);
-          const uint32_t vw = p1 + p2;
-          const int k = 4 * q + u;
-          if (grp == 0) xnew[w0 + k] = vw;
-          ne[k] = vw & 0x33333333u;
-          no[k] = (vw >> 2) & 0x33333333u;
-          s_one = __builtin_amdgcn_udot8(0x11111111u, ne[k], s_one, false);
-          s_one = __builtin_amdgcn_udot8(0x11111111u, no[k], s_one, false);
-          s_self = __builtin_amdgcn_udot8(ne[k], ne[k], s_self, false);
-          s_self = __builtin_amdgcn_udot8(no[k], no[k], s_self, false);
-        }
-      }
-      // column of round r, register set u: grp + (4 r + u) groups; every
-      // group runs the rounds of group 0, the one with the most columns
-      const int rounds = (cols / groups + 1 + 3) / 4;
-      auto src = [&](int cu) -> const uint32_t* {
-        const int cc = (cu >= me && cu < cols) ? cu : 0;
-        return (cu >= me && cu < cols) ? xcol + (size_t)S.slot[cc] * W : wn;
-      };
-      uint4 cur[4][4];
+    for (int q = 0; q < NP; ++q) {
+      const uint32_t pc = p0 + t + q * SPAN;
+      off[q] = (pc < W4 ? pc : W4 - 1) * 16;
+      const uint4 v = wn[off[q] / 16];
+      const uint32_t xs[4] = {v.x, v.y, v.z, v.w};
+      uint32_t vw[4];
 #pragma unroll
       for (int u = 0; u < 4; ++u) {
-        const uint32_t* pc = src(grp + u * groups);
-#pragma unroll
-        for (int q = 0; q < 4; ++q) cur[u][q] = *(const uint4*)(pc + w0 + 4 * q);
+        vw[u] = pc < W4 ? value_word(xs[u], coding) : 0u;
+        ne[q][u] = vw[u] & 0x33333333u;
+        no[q][u] = (vw[u] >> 2) & 0x33333333u;
       }
-      for (int r = 0; r < rounds; ++r) {
+      if (grp == 0) {
+        if (pc < W4) *(uint4*)((char*)xnew + off[q]) = make_uint4(vw[0], vw[1], vw[2], vw[3]);
 #pragma unroll
         for (int u = 0; u < 4; ++u) {
-          const int cu = grp + (4 * r + u) * groups;
-          uint32_t se = 0, so = 0;
-#pragma unroll
-          for (int q = 0; q < 4; ++q) {
-            const uint32_t xs[4] = {cur[u][q].x, cur[u][q].y, cur[u][q].z, cur[u][q].w};
-#pragma unroll
-            for (int k4 = 0; k4 < 4; ++k4) {
-              const int k = 4 * q + k4;
-              const uint32_t e = xs[k4] & 0x33333333u;
-              se = __builtin_amdgcn_udot8(e, ne[k], se, false);
-              so = __builtin_amdgcn_udot8(xs[k4] ^ e, no[k], so, false);
-            }
-          }
-          // next round's column of this register set
-          const uint32_t* pn = src(cu + 4 * groups);
-#pragma unroll
-          for (int q = 0; q < 4; ++q) cur[u][q] = *(const uint4*)(pn + w0 + 4 * q);
-          const uint32_t sum = cu == 0 ? s_one : (cu == cols ? s_self : se + (so >> 2));
-          // covariate columns (0 < c < me): cov_dots
-          if (cu <= cols && (cu == 0 || cu >= me)) atomicAdd(&acc[cu], (int)sum);
+          s_one = __builtin_amdgcn_udot8(0x11111111u, ne[q][u], s_one, false);
+          s_one = __builtin_amdgcn_udot8(0x11111111u, no[q][u], s_one, false);
+          s_self = __builtin_amdgcn_udot8(ne[q][u], ne[q][u], s_self, false);
+          s_self = __builtin_amdgcn_udot8(no[q][u], no[q][u], s_self, false);
         }
       }
     }
+    auto put_sum = [&](int c, int v) {
+      if (t == SPAN - 1) acc[c] = p0 == 0 ? v : acc[c] + v;
+    };
+    if (tid < 64) {                           // the wave that holds group 0
+      const int a = group_sum((int)s_one), b = group_sum((int)s_self);
+      if (grp == 0) { put_sum(0, a); put_sum(cols, b); }
+    }
+    // group g sums columns me + g + GRP k; every group runs group 0's rounds
+    const int n_col = cols - me;
+    const int rounds = n_col > 0 ? ((n_col + GRP - 1) / GRP + UC - 1) / UC : 0;
+    auto column = [&](int r, int u) { return me + grp + (UC * r + u) * GRP; };
+    auto load = [&](int r, uint4 (&w)[UC][NP]) {
+#pragma unroll
+      for (int u = 0; u < UC; ++u) {
+        const int c = column(r, u);
+        const uint32_t base = (uint32_t)S.slot[c < cols ? c : cols - 1] * W * 4;
+#pragma unroll
+        for (int q = 0; q < NP; ++q) w[u][q] = *(const uint4*)(xcol + (base + off[q]));
+      }
+    };
+    auto sum = [&](int r, const uint4 (&w)[UC][NP]) {
+      int v[UC];
+#pragma unroll
+      for (int u = 0; u < UC; ++u) {
+        uint32_t se = 0, so = 0;
+#pragma unroll
+        for (int q = 0; q < NP; ++q) {
+          const uint32_t xs[4] = {w[u][q].x, w[u][q].y, w[u][q].z, w[u][q].w};
+#pragma unroll
+          for (int k = 0; k < 4; ++k) {
+            const uint32_t e = xs[k] & 0x33333333u;
+            se = __builtin_amdgcn_udot8(e, ne[q][k], se, false);
+            so = __builtin_amdgcn_udot8(xs[k] ^ e, no[q][k], so, false);
+          }
+        }
+        v[u] = (int)(se + (so >> 2));
+      }
+#pragma unroll
+      for (int u = 0; u < UC; ++u) v[u] = group_sum(v[u]);
+#pragma unroll
+      for (int u = 0; u < UC; ++u) {
+        const int c = column(r, u);
+        if (c < cols) put_sum(c, v[u]);
+      }
+    };
+    uint4 wa[UC][NP], wb[UC][NP];
+    if (rounds > 0) load(0, wa);
+    for (int r = 0; r < rounds; r += 2) {
+      if (r + 1 < rounds) load(r + 1, wb);
+      sum(r, wa);
+      if (r + 1 < rounds) {
+        if (r + 2 < rounds) load(r + 2, wa);
+        sum(r + 1, wb);
+      }
+    }
   }
+}
+
+// the group width and pieces per lane for the column length: the narrowest
+// group that holds a column in one piece a lane, and from 64 pieces on the
+// fewest pieces a lane that hold it (at most five, then several passes)
+template <int KMAX, int T0, int NTH>
+__device__ __forceinline__ void column_dots(Ctx<KMAX>& C, uint64_t snp_new, int coding, int cols, uint32_t* xnew,
+                                            int32_t* acc) {
+  if ((int)threadIdx.x < T0) return;
+  const uint32_t W4 = C.D.W32 / 4;
+  if (W4 <= 16) column_dots_np<KMAX, T0, NTH, 16, 1>(C, snp_new, coding, cols, xnew, acc);
+  else if (W4 <= 32) column_dots_np<KMAX, T0, NTH, 32, 1>(C, snp_new, coding, cols, xnew, acc);
+  else if (W4 <= 64) column_dots_np<KMAX, T0, NTH, 64, 1>(C, snp_new, coding, cols, xnew, acc);
+  else if (W4 <= 192) column_dots_np<KMAX, T0, NTH, 64, 3>(C, snp_new, coding, cols, xnew, acc);
+  else column_dots_np<KMAX, T0, NTH, 64, 5>(C, snp_new, coding, cols, xnew, acc);
 }
 
 // S.work[c] = e_c^T x_new for the covariate columns c in [1, me): each
@@ -393,14 +429,7 @@ template <int KMAX>
 __device__ __forceinline__ void new_column_dots(Ctx<KMAX>& C, uint64_t snp_new, int coding_new, int cols,
                                                 uint32_t* xnew) {
   Smem<KMAX>& S = C.S;
-  for (int c = threadIdx.x; c <= cols; c += BMG_BLOCK) S.iacc[c] = 0;
-  __syncthreads();
-  switch (coding_new) {
-    case 0: column_dots<KMAX, 0, 0, BMG_BLOCK>(C, snp_new, cols, xnew, S.iacc); break;
-    case 1: column_dots<KMAX, 1, 0, BMG_BLOCK>(C, snp_new, cols, xnew, S.iacc); break;
-    case 2: column_dots<KMAX, 2, 0, BMG_BLOCK>(C, snp_new, cols, xnew, S.iacc); break;
-    default: column_dots<KMAX, 3, 0, BMG_BLOCK>(C, snp_new, cols, xnew, S.iacc); break;
-  }
+  column_dots<KMAX, 0, BMG_BLOCK>(C, snp_new, coding_new, cols, xnew, S.iacc);
   __syncthreads();
   for (int c = threadIdx.x; c <= cols; c += BMG_BLOCK) S.work[c] = (double)S.iacc[c];
   __syncthreads();
@@ -1300,21 +1329,14 @@ __device__ __forceinline__ void update_on_add(Ctx<KMAX>& C, uint32_t ind, int mo
   // will be given, the lowest free once this column's is taken
   int nslot = -1;
   if (next >= 0 && !C.D.mixed && C.D.type != BMG_AH && C.D.me <= 1 && col + 1 < KMAX) nslot = alloc_slot(C);
-  if (nslot >= 0)
-    for (int c = threadIdx.x; c <= col + 1; c += BMG_BLOCK) S.iacc2[c] = 0;
   // bordered update (src/symmmatrix.cpp:144-164)
   for (int i = threadIdx.x; i < col; i += BMG_BLOCK) S.L[P(col) + i] = S.work[i];
   __syncthreads();
   if (wave_id() == 0) {
     trsv_ut_w0(S, S.L + P(col), col);
   } else if (nslot >= 0) {
-    uint32_t* xn = gp(C.A.xcol) + (size_t)nslot * C.D.W32;
-    switch (C.D.type) {
-      case 0: column_dots<KMAX, 0, 64, BMG_BLOCK - 64>(C, (uint64_t)next, col + 1, xn, S.iacc2); break;
-      case 1: column_dots<KMAX, 1, 64, BMG_BLOCK - 64>(C, (uint64_t)next, col + 1, xn, S.iacc2); break;
-      case 2: column_dots<KMAX, 2, 64, BMG_BLOCK - 64>(C, (uint64_t)next, col + 1, xn, S.iacc2); break;
-      default: column_dots<KMAX, 3, 64, BMG_BLOCK - 64>(C, (uint64_t)next, col + 1, xn, S.iacc2); break;
-    }
+    column_dots<KMAX, 64, BMG_BLOCK - 64>(C, (uint64_t)next, C.D.type, col + 1,
+                                          gp(C.A.xcol) + (size_t)nslot * C.D.W32, S.iacc2);
   }
   __syncthreads();
   if (nslot >= 0) { R.pre_snp = next; R.pre_slot = nslot; }
@@ -1371,23 +1393,24 @@ __device__ __forceinline__ void add_term(Ctx<KMAX>& C, uint32_t ind, int t_ind, 
   R.nloci++;
   put(R.Ns, type, sel(R.Ns, type) + 1);
   R.mu_computed = 0;
-  if (is_ah) {
-    update_on_add(C, ind, model_ind, 0, 0, d2[0]);
-    if (isfinite(R.syx)) update_on_add(C, ind, model_ind, 1, 1, d2[1]);
-    else if (R.cols < KMAX && alloc_slot(C) >= 0) {
+  // A then H columns of an AH term (one copy of the update's code)
+#pragma unroll 1
+  for (int q = 0; q <= is_ah; ++q) {
+    const double dq = q ? d2[1] : d2[0];
+    if (q == 0 || isfinite(R.syx)) {
+      update_on_add(C, ind, model_ind, is_ah ? q : type, q, dq, is_ah ? -1 : next);
+    } else if (R.cols < KMAX && alloc_slot(C) >= 0) {
       // keep the bookkeeping of the second column (not factorised)
       int col = R.cols, slot = alloc_slot(C);
       __syncthreads();
       if (threadIdx.x == 0) {
         S.xi2[model_ind] = col; S.snp[col] = (int32_t)ind; S.xtype[col] = 1;
-        S.slot[col] = slot; S.d[col] = d2[1];
+        S.slot[col] = slot; S.d[col] = dq;
       }
       __syncthreads();
       set_slot_bit(C, slot, 1);
       R.cols = col + 1;
     }
-  } else {
-    update_on_add(C, ind, model_ind, type, 0, d2[0], next);
   }
 }
 
@@ -1432,19 +1455,10 @@ __device__ __forceinline__ void update_on_remove_impl(Ctx<KMAX>& C, int x_ind, l
     int nslot = -1;
     if (next >= 0 && !C.D.mixed && C.D.type != BMG_AH && C.D.me <= 1 && R.cols < KMAX)
       nslot = alloc_slot(C);
-    if (nslot >= 0) {
-      for (int c = threadIdx.x; c <= R.cols; c += BMG_BLOCK) S.iacc2[c] = 0;
-      __syncthreads();
-    }
     auto ahead = [&]() {
-      if (nslot < 0) return;
-      uint32_t* xn = gp(C.A.xcol) + (size_t)nslot * C.D.W32;
-      switch (C.D.type) {
-        case 0: column_dots<KMAX, 0, 64, BMG_BLOCK - 64>(C, (uint64_t)next, R.cols, xn, S.iacc2); break;
-        case 1: column_dots<KMAX, 1, 64, BMG_BLOCK - 64>(C, (uint64_t)next, R.cols, xn, S.iacc2); break;
-        case 2: column_dots<KMAX, 2, 64, BMG_BLOCK - 64>(C, (uint64_t)next, R.cols, xn, S.iacc2); break;
-        default: column_dots<KMAX, 3, 64, BMG_BLOCK - 64>(C, (uint64_t)next, R.cols, xn, S.iacc2); break;
-      }
+      if (nslot >= 0)
+        column_dots<KMAX, 64, BMG_BLOCK - 64>(C, (uint64_t)next, C.D.type, R.cols,
+                                              gp(C.A.xcol) + (size_t)nslot * C.D.W32, S.iacc2);
     };
     const uint64_t ta = wall_clock64();
     // v follows the downdate's rotations (no re-solve)
@@ -1487,12 +1501,10 @@ __device__ __forceinline__ void remove_term(Ctx<KMAX>& C, int model_ind, long lo
   __syncthreads();
   R.n_rm++;
   R.nloci = nl - 1;
-  if (type == 4) {
-    if (xi1 > xi2) { update_on_remove(C, xi1); update_on_remove(C, xi2); }
-    else { update_on_remove(C, xi2); update_on_remove(C, xi1); }
-  } else {
-    update_on_remove(C, xi1, next);
-  }
+  // the later column of an AH term first
+#pragma unroll 1
+  for (int q = 0; q < xmove; ++q)
+    update_on_remove(C, type != 4 ? xi1 : ((q == 0) == (xi1 > xi2) ? xi1 : xi2), type == 4 ? -1 : next);
   R.mu_computed = 0;
 }
 
