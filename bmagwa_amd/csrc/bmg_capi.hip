@@ -856,7 +856,7 @@ static int batch_create(bmg_ctx** ctxs, int n_ctx, int n_chains, const int32_t* 
   // a chain that leaves K continues in the 256-column kernel on the same state
   const size_t G = BMG_KMAXG;
   size_t o_L = add(8 * G * (G + 1) / 2), o_xx = add(8 * G * G);
-  size_t o_Lw = add(8 * G * (G + 1) / 2);
+  size_t o_Lw = add(8 * (G * (G + 1) / 2 + BMG_LPAD));
   size_t o_xc = add(4 * G * wmax);
   size_t o_yh = add(8 * npmax), o_vec = add(8 * 5 * G), o_idx = add(4 * 8 * G), o_ad = add(8 * 6 * 256);
   size_t o_trm = add(tr_cap), o_trj = add(tr_cap), o_trs = add(tr_cap), o_trz = add(4 * tr_cap),

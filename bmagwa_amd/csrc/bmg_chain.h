@@ -5,6 +5,7 @@
 
 #define BMG_MAXMS 64     // max_move_size supported on the device
 #define BMG_KMAXG 256    // largest compiled model capacity (columns)
+#define BMG_LPAD 8       // doubles after a packed factor that block reads may touch
 #define BMG_TREE_LEV 8
 #define BMG_LH_MAX 32    // largest learned-swap window
 #define BMG_DR_MAX 20    // largest delayed-rejection move size (2^20 sub-models)

@@ -80,7 +80,9 @@ struct GlobalFactor {
   __device__ __forceinline__ operator double*() const { return gp(p); }
 };
 template <int KMAX>
-using FactorT = std::conditional_t<(KMAX <= KMAX_LDS), double[KMAX * (KMAX + 1) / 2], GlobalFactor>;
+using FactorT = std::conditional_t<(KMAX <= KMAX_LDS),
+                                   double[KMAX * (KMAX + 1) / 2 + (KMAX + 63) / 64 * 64 - KMAX + BMG_LPAD],
+                                   GlobalFactor>;
 
 // counters of ChainScal that change in every iteration
 struct Counters {
@@ -445,118 +447,170 @@ __device__ __forceinline__ double readlane_d(double v, int src) {
   return *reinterpret_cast<double*>(&h);
 }
 
-// x := U^-T x for x[0..m) in LDS (dtrsv Upper/Trans order).  Wave 0 only.
-// Lane l holds x[l + 64 t] in b[t] and the reciprocal of that row's
-// diagonal entry in dg[t] (all computed at once before the sweep); the
-// outer loop over t is unrolled so the register arrays are only ever
-// indexed by constants.  Row i: the owner's scaled entry is read across
-// lanes and every lane subtracts its coefficient times it, so the serial
-// chain per row is one multiply, one cross-lane read and one fused
-// multiply-subtract, with no division.  The sweep has no branches and no
-// masks: every lane applies every row with the entry at its own column's
-// row i (a lane at or past its row reads another column's entry into a
-// value it no longer needs; its result was kept in xo when its row came),
-// and the coefficients are read two rows ahead from clamped addresses, so
-// no row waits on LDS.  Per element the subtractions come in row order, as
-// in the sequential loop; the reciprocal and the fused update round
-// differently from its divisions (by an ulp), which the log-likelihoods'
-// 1e-10 agreement with the oracle absorbs.
-template <int KMAX>
-__device__ __forceinline__ void trsv_ut_w0(Smem<KMAX>& S, double* x, int m) {
-  constexpr int NT = (KMAX + 63) / 64;
-  constexpr int LIM = KMAX * (KMAX + 1) / 2 - 1;
+// The triangular sweeps.  Wave 0 only.  Lane l holds the vector's entries
+// l + 64 t (t < NT, the fewest that hold the vector) and the reciprocals of
+// their rows' diagonal entries in registers; the outer loops over t are
+// unrolled so the register arrays are only ever indexed by constants.  Per
+// row the owner's scaled entry is read across lanes and every lane subtracts
+// its coefficient times it: the serial chain is one multiply, one cross-lane
+// read and one fused multiply-subtract, with no division, no branches and no
+// masks.  A lane at or past its row reads another column's entry into a value
+// it no longer needs (its result was kept when its row came), and rows past
+// the vector's end change nothing that is kept, so whole blocks of SWEEP
+// rows run.  Bound by that chain: the coefficients of a block are read into
+// registers while the block before it is applied, so no row waits for them.
+// (Read two rows ahead, each row took half an LDS round trip, 78 ns, and with
+// the factor in global memory half an L2 round trip, 125-180 ns.)  Per element
+// the subtractions come in row order, as in the sequential loop; the
+// reciprocal and the fused update round differently from its divisions (by an
+// ulp), which the log-likelihoods' 1e-10 agreement with the oracle absorbs.
+constexpr int SWEEP = 8;
+
+// x := T^-T x, T the n x n triangle of the factor L that begins at row and
+// column o (dtrsv Upper/Trans order).  ALPHA: a2 of entry i becomes 1 + the
+// sum of the squares of the results 0..i.
+template <int NT, bool ALPHA>
+__device__ __forceinline__ void sweep_ut(const double* L, int o, int n, const double (&dg)[NT], double (&b)[NT],
+                                         double (&xo)[NT], double (&a2)[NT]) {
   const int lane = lane_id();
-  double b[NT], dg[NT], xo[NT];
   int base[NT];
 #pragma unroll
   for (int t = 0; t < NT; ++t) {
     const int j = lane + 64 * t;
-    b[t] = j < m ? x[j] : 0.0;
-    dg[t] = j < m ? 1.0 / S.L[P(j) + j] : 1.0;
-    base[t] = j < m ? P(j) : 0;
+    base[t] = j < n ? P(o + j) + o : 0;
     xo[t] = 0.0;
+    if (ALPHA) a2[t] = 1.0;
   }
-  auto ld = [&](int t, int i) -> double {
-    const int a = base[t] + i;
-    return S.L[a < LIM ? a : LIM];
-  };
+  double al = 1.0;
 #pragma unroll
   for (int ti = 0; ti < NT; ++ti) {
     const int i0 = 64 * ti;
-    const int iend = m < 64 * (ti + 1) ? m : 64 * (ti + 1);
+    const int iend = n < 64 * (ti + 1) ? n : 64 * (ti + 1);
     if (i0 >= iend) break;
-    double ca[NT], cb[NT];
-#pragma unroll
-    for (int t = ti; t < NT; ++t) { ca[t] = ld(t, i0); cb[t] = ld(t, i0 + 1); }
-    auto row = [&](int i, double (&c)[NT]) {
-      const int owner = i & 63;
-      const double xi = readlane_d(b[ti] * dg[ti], owner);
-      xo[ti] = lane == owner ? xi : xo[ti];
+    double ca[SWEEP][NT], cb[SWEEP][NT];
+    auto load = [&](int i, double (&c)[SWEEP][NT]) {
 #pragma unroll
       for (int t = ti; t < NT; ++t)
-        if (64 * t < m) b[t] = fma(-c[t], xi, b[t]);
 #pragma unroll
-      for (int t = ti; t < NT; ++t) c[t] = ld(t, i + 2);
+        for (int q = 0; q < SWEEP; ++q) c[q][t] = L[base[t] + i + q];
     };
-    int i = i0;
-    for (; i + 1 < iend; i += 2) { row(i, ca); row(i + 1, cb); }
-    if (i < iend) row(i, ca);
+    auto rows = [&](int i, const double (&c)[SWEEP][NT]) {
+#pragma unroll
+      for (int q = 0; q < SWEEP; ++q) {
+        const int owner = (i + q) & 63;
+        const double xi = readlane_d(b[ti] * dg[ti], owner);
+        xo[ti] = lane == owner ? xi : xo[ti];
+        if (ALPHA) {
+          al = fma(xi, xi, al);
+          a2[ti] = lane == owner ? al : a2[ti];
+        }
+#pragma unroll
+        for (int t = ti; t < NT; ++t) b[t] = fma(-c[q][t], xi, b[t]);
+      }
+    };
+    load(i0, ca);
+#pragma unroll 1
+    for (int i = i0; i < iend; i += 2 * SWEEP) {
+      if (i + SWEEP < iend) load(i + SWEEP, cb);
+      rows(i, ca);
+      if (i + SWEEP < iend) {
+        if (i + 2 * SWEEP < iend) load(i + 2 * SWEEP, ca);
+        rows(i + SWEEP, cb);
+      }
+    }
   }
+}
+
+template <int NT>
+__device__ __forceinline__ void trsv_ut_nt(const double* L, double* x, int m) {
+  const int lane = lane_id();
+  double b[NT], dg[NT], xo[NT], a2[NT];
+#pragma unroll
+  for (int t = 0; t < NT; ++t) {
+    const int j = lane + 64 * t;
+    b[t] = j < m ? x[j] : 0.0;
+    dg[t] = j < m ? 1.0 / L[P(j) + j] : 1.0;
+  }
+  sweep_ut<NT, false>(L, 0, m, dg, b, xo, a2);
 #pragma unroll
   for (int t = 0; t < NT; ++t) { const int j = lane + 64 * t; if (j < m) x[j] = xo[t]; }
 }
 
-// x := U^-1 x (dtrsv Upper/NoTrans, back substitution).  Wave 0 only.  Lane
-// l holds x[l + 64 t] and the reciprocal of that row's diagonal; step j
-// reads the owner's scaled entry across lanes and every lane subtracts its
-// entry of column j (one column: consecutive addresses) times it, so the
-// serial chain per step is a multiply, a cross-lane read and a fused update
-// (rounding within an ulp of the divide-and-subtract loop).  As in the
-// forward sweep there are no branches or masks (a lane at or past its row
-// updates a value it no longer needs; its result is in xo) and the columns
-// are read two steps ahead.  A zero x_j leaves every entry as it was, as
-// the reference's skip of zero entries does.
+// x := U^-T x for x[0..m).  Wave 0 only.
 template <int KMAX>
-__device__ __forceinline__ void trsv_un_w0(Smem<KMAX>& S, double* x, int m) {
-  constexpr int NT = (KMAX + 63) / 64;
-  constexpr int LIM = KMAX * (KMAX + 1) / 2 - 1;
+__device__ __forceinline__ void trsv_ut_w0(Smem<KMAX>& S, double* x, int m) {
+  const double* L = S.L;
+  if (m <= 64) trsv_ut_nt<1>(L, x, m);
+  else if (KMAX <= 128 || m <= 128) trsv_ut_nt<2>(L, x, m);
+  else if (KMAX <= 192 || m <= 192) trsv_ut_nt<3>(L, x, m);
+  else trsv_ut_nt<4>(L, x, m);
+}
+
+// x := U^-1 x (dtrsv Upper/NoTrans, back substitution): step j subtracts
+// column j (consecutive addresses) times the owner's scaled entry, columns
+// in descending order.  A zero x_j leaves every entry as it was, as the
+// reference's skip of zero entries does.
+template <int NT>
+__device__ __forceinline__ void trsv_un_nt(const double* L, double* x, int m) {
   const int lane = lane_id();
-  if (m <= 0) return;
   double b[NT], rd[NT], xo[NT];
 #pragma unroll
   for (int t = 0; t < NT; ++t) {
     const int j = lane + 64 * t;
     b[t] = j < m ? x[j] : 0.0;
-    rd[t] = j < m ? 1.0 / S.L[P(j) + j] : 1.0;
+    rd[t] = j < m ? 1.0 / L[P(j) + j] : 1.0;
     xo[t] = 0.0;
   }
-  // entry (lane + 64 q) of column j, clamped into the factor
-  auto ld = [&](int q, int j) -> double {
-    const int a = (j > 0 ? P(j) : 0) + lane + 64 * q;
-    return S.L[a < LIM ? a : LIM];
-  };
 #pragma unroll
   for (int tj = NT - 1; tj >= 0; --tj) {
+    const int j0 = 64 * tj;
     const int jend = m < 64 * (tj + 1) ? m : 64 * (tj + 1);
-    if (64 * tj >= jend) continue;
-    double ca[NT], cb[NT];
+    if (j0 >= jend) continue;
+    double ca[SWEEP][NT], cb[SWEEP][NT];
+    // columns j, j - 1, ... (below the first: column 0)
+    auto load = [&](int j, double (&c)[SWEEP][NT]) {
 #pragma unroll
-    for (int q = 0; q <= tj; ++q) { ca[q] = ld(q, jend - 1); cb[q] = ld(q, jend - 2); }
-    auto step = [&](int j, double (&c)[NT]) {
-      const int owner = j & 63;
-      const double xj = readlane_d(b[tj] * rd[tj], owner);
-      xo[tj] = lane == owner ? xj : xo[tj];
+      for (int s = 0; s < SWEEP; ++s) {
+        const int pj = j - s > 0 ? P(j - s) : 0;
 #pragma unroll
-      for (int q = 0; q <= tj; ++q) b[q] = fma(-xj, c[q], b[q]);
-#pragma unroll
-      for (int q = 0; q <= tj; ++q) c[q] = ld(q, j - 2);
+        for (int q = 0; q <= tj; ++q) c[s][q] = L[pj + lane + 64 * q];
+      }
     };
-    int j = jend - 1;
-    for (; j - 1 >= 64 * tj; j -= 2) { step(j, ca); step(j - 1, cb); }
-    if (j >= 64 * tj) step(j, ca);
+    auto steps = [&](int j, const double (&c)[SWEEP][NT]) {
+#pragma unroll
+      for (int s = 0; s < SWEEP; ++s) {
+        if (j - s >= j0) {
+          const int owner = (j - s) & 63;
+          const double xj = readlane_d(b[tj] * rd[tj], owner);
+          xo[tj] = lane == owner ? xj : xo[tj];
+#pragma unroll
+          for (int q = 0; q <= tj; ++q) b[q] = fma(-xj, c[s][q], b[q]);
+        }
+      }
+    };
+    load(jend - 1, ca);
+#pragma unroll 1
+    for (int j = jend - 1; j >= j0; j -= 2 * SWEEP) {
+      if (j - SWEEP >= j0) load(j - SWEEP, cb);
+      steps(j, ca);
+      if (j - SWEEP >= j0) {
+        if (j - 2 * SWEEP >= j0) load(j - 2 * SWEEP, ca);
+        steps(j - SWEEP, cb);
+      }
+    }
   }
 #pragma unroll
   for (int t = 0; t < NT; ++t) { const int j = lane + 64 * t; if (j < m) x[j] = xo[t]; }
+}
+
+template <int KMAX>
+__device__ __forceinline__ void trsv_un_w0(Smem<KMAX>& S, double* x, int m) {
+  const double* L = S.L;
+  if (m <= 0) return;
+  if (m <= 64) trsv_un_nt<1>(L, x, m);
+  else if (KMAX <= 128 || m <= 128) trsv_un_nt<2>(L, x, m);
+  else if (KMAX <= 192 || m <= 192) trsv_un_nt<3>(L, x, m);
+  else trsv_un_nt<4>(L, x, m);
 }
 
 // netlib drotg (as the oracle restates it)
@@ -578,255 +632,147 @@ __device__ __forceinline__ void drotg(double& a, double& b, double& c, double& s
   a = r; b = z;
 }
 
-// The rotation drotg generates (same sign convention: r takes the sign of
-// the larger input), without its overflow scaling, which a Cholesky factor's
-// entries never need.  1 / r comes from the hardware reciprocal square root
-// of a^2 + b^2 refined by two Newton steps (each roughly doubles the correct
-// bits, ending within an ulp or two of the correctly rounded value), so the
-// downdate's serial chain per step is a handful of multiplies instead of a
-// square root and a division.  c, s and r agree with drotg's to rounding.
-__device__ __forceinline__ void rot_gen(double& a, double b, double& c, double& s) {
-  const double roe = fabs(a) > fabs(b) ? a : b;
-  const double q = fma(a, a, b * b);
-  double y = __builtin_amdgcn_rsq(q);
-  const double h = 0.5 * q;
-  y = y * fma(-h * y, y, 1.5);
-  y = y * fma(-h * y, y, 1.5);
-  const double ri = q > 0.0 ? (roe >= 0.0 ? y : -y) : 0.0;
-  c = q > 0.0 ? a * ri : 1.0;
-  s = b * ri;
-  a = q * ri;
-}
-
-// Cholesky downdate removing column cr of the m x m factor (LINPACK dchex
-// job 2 + drop + sign fix, src/symmmatrix.cpp:166-195).  Logical column jl >=
-// cr lives in physical column jl + 1 until it is written back; rotation j is
-// generated from logical column j's rows (j, j + 1) and applied to every
-// later column at once (per element the same sequence as the sequential
-// loop).  The two rows a rotation touches stay in registers: lane jl % 64
-// keeps rows (j, j + 1) of its columns, reads rows two steps ahead from LDS
-// (rows below j + 1 are not rotated yet) and stores only the finished row,
-// and the owner of column j hands the rotation's inputs to all lanes with a
-// cross-lane read, so no step waits on an LDS round trip.
+// Removing column cr of the m x m factor U (the result of LINPACK dchex job
+// 2 + drop + sign fix, src/symmmatrix.cpp:166-195): the rows above cr lose the
+// column; below, the triangle T of the later columns takes up the row r =
+// U[cr, cr+1..] by rotations that zero r entry by entry, T'T'^T = T^T T + r r^T.
+// dchex generates rotation k from the entries that rotation k - 1 left, a
+// square root and a division in a serial chain per row.  Here the rotations
+// are found first: with w = T^-T r, rotation k has cos = alpha_k-1 / alpha_k
+// and sin = w_k / alpha_k, alpha_k^2 = 1 + w_0^2 + ... + w_k^2 (Gill, Golub,
+// Murray and Saunders 1974, method C1), so the serial chain is one forward
+// sweep, the square roots and divisions are a lane per row, and the rotations
+// are then applied with every lane going down its own columns: a multiply and
+// a fused multiply-add per row in the chain.  cos, sin >= 0 in cos's case
+// give positive diagonals, dchex's after its sign fix.  (dchex's order took
+// 14 us at 105 columns, 250 ns a row, and 30-40 us with the factor in global
+// memory.  Over removals in a row from factors of LD columns up to r =
+// 0.999999 both orders' factors, log-determinants and v are equally far from
+// 80-bit ones.)
 //
-// Finished rows go straight to their place in the compacted factor
-// (physical column jl, whose entries at and past row cr were read two or
-// more steps earlier), with the sign fix folded in: a row whose diagonal
-// comes out negative is stored negated, which is what the separate pass
-// over the finished rows does.  Meanwhile wave 1 moves the rows above cr of
-// the later columns down by one column, in ascending order of destination
-// (every source lies above every earlier destination, so one wave's
-// batches never overwrite what a later batch reads); the two touch disjoint
-// entries.
-//
-// v (U^T v = X^T y) goes through the same rotations and sign fix as the
-// factor's rows, so after the removal it solves the new factor's system
-// without a second triangular solve (the reference re-solves,
-// src/model.hpp:530-545; the two agree to rounding).
-template <int KMAX, typename Extra>
-__device__ __forceinline__ void chol_downdate_lds(Smem<KMAX>& S, int m, int cr, Extra extra) {
-  constexpr int NT = (KMAX + 63) / 64;
-  constexpr int LIM = KMAX * (KMAX + 1) / 2 - 1;
+// The triangle's new rows go straight to their place in the compacted factor
+// (logical column cr + j from physical column cr + 1 + j): a step stores row
+// cr + k of a column, which the lane of the column before read as its row at
+// an earlier step.  v (U^T v = X^T y) goes through the same rotations, so
+// after the removal it solves the new factor's system without a second
+// triangular solve (the reference re-solves, src/model.hpp:530-545; the two
+// agree to rounding).  Wave 0 only.
+template <int KMAX, int NT>
+__device__ __forceinline__ void downdate_w0(Smem<KMAX>& S, double* L, int m, int cr) {
   const int lane = lane_id();
-  if (wave_id() == 0) {
-    double vt = S.v[cr], vb = S.v[cr + 1];   // rows (j, j + 1) of v, all lanes
-    double top[NT], nA[NT], nB[NT];
-    int pb[NT], lb[NT];   // physical and logical column offsets
+  const int o = cr + 1, n = m - 1 - cr;
+  double r[NT], b[NT], dg[NT], w[NT], a2[NT], cc[NT], ss[NT], vo[NT], vn[NT];
+  int src[NT], dst[NT];
 #pragma unroll
-    for (int t = 0; t < NT; ++t) {
-      const int jl = lane + 64 * t;
-      pb[t] = P(jl + 1);
-      lb[t] = P(jl);
-      top[t] = S.L[min(pb[t] + cr, LIM)];
-      nA[t] = S.L[min(pb[t] + cr + 1, LIM)];
-      nB[t] = S.L[min(pb[t] + cr + 2, LIM)];
-    }
+  for (int t = 0; t < NT; ++t) {
+    const int j = lane + 64 * t;
+    const bool on = j < n;
+    src[t] = on ? P(o + j) + o : 0;
+    dst[t] = on ? P(cr + j) + cr : 0;
+    r[t] = b[t] = on ? L[src[t] - 1] : 0.0;
+    dg[t] = on ? 1.0 / L[src[t] + j] : 1.0;
+    vo[t] = on ? S.v[o + j] : 0.0;
+    vn[t] = 0.0;
+  }
+  double vr = S.v[cr];
+  sweep_ut<NT, true>(L, o, n, dg, b, w, a2);
 #pragma unroll
-    for (int ti = 0; ti < NT; ++ti) {
-      const int jbeg = cr > 64 * ti ? cr : 64 * ti;
-      const int jend = (m - 1) < 64 * (ti + 1) ? (m - 1) : 64 * (ti + 1);
-      // step j: n1 holds row j + 1 of each column and takes row j + 3
-      auto step = [&](int j, double (&n1)[NT]) {
-        const int owner = j & 63;
-        // every lane generates the rotation from the same two values
-        double a = readlane_d(top[ti], owner), b = readlane_d(n1[ti], owner);
-        const double vbn = S.v[j + 2 < m ? j + 2 : m - 1];   // next row of v, read ahead
-        double cc, ss;
-        rot_gen(a, b, cc, ss);
-        const double sg = a < 0.0 ? -1.0 : 1.0;   // sign fix of row j
-        if (lane == owner) S.L[lb[ti] + j] = a * sg;
-        {
-          const double tv = cc * vt + ss * vb;
-          vt = cc * vb - ss * vt;
-          if (lane == 0) S.v[j] = tv * sg;
-          vb = vbn;
-        }
+  for (int t = 0; t < NT; ++t) {
+    a2[t] = sqrt(a2[t]);
+    double before = dpp_f64<0x138, 0xf>(a2[t]);          // wave_shr:1
+    const double first = t == 0 ? 1.0 : readlane_d(a2[t > 0 ? t - 1 : 0], 63);
+    before = lane == 0 ? first : before;
+    const double inv = 1.0 / a2[t];
+    cc[t] = before * inv;
+    ss[t] = w[t] * inv;
+  }
+#pragma unroll
+  for (int ti = 0; ti < NT; ++ti) {
+    const int k0 = 64 * ti;
+    const int kend = n < 64 * (ti + 1) ? n : 64 * (ti + 1);
+    if (k0 >= kend) break;
+    double ua[SWEEP][NT], ub[SWEEP][NT];
+    auto load = [&](int k, double (&u)[SWEEP][NT]) {
+#pragma unroll
+      for (int t = ti; t < NT; ++t)
+#pragma unroll
+        for (int q = 0; q < SWEEP; ++q) u[q][t] = L[src[t] + k + q];
+    };
+    auto rows = [&](int kb, const double (&u)[SWEEP][NT]) {
+#pragma unroll
+      for (int q = 0; q < SWEEP; ++q) {
+        const int k = kb + q, owner = k & 63;
+        const double c = readlane_d(cc[ti], owner), s = readlane_d(ss[ti], owner);
+        const double vk = readlane_d(vo[ti], owner);
+        const double vnew = fma(c, vk, s * vr);
+        vr = fma(c, vr, -(s * vk));
+        vn[ti] = lane == owner ? vnew : vn[ti];
 #pragma unroll
         for (int t = ti; t < NT; ++t) {
-          if (64 * t <= m - 2) {
-            const int jl = lane + 64 * t;
-            const double x1 = top[t], x2 = n1[t];
-            const double tt = cc * x1 + ss * x2;
-            const bool on = jl > j && jl <= m - 2;
-            top[t] = on ? cc * x2 - ss * x1 : top[t];
-            if (on) S.L[lb[t] + j] = tt * sg;
-            n1[t] = S.L[min(pb[t] + j + 3, LIM)];
-          }
+          const int j = lane + 64 * t;
+          const double x = fma(c, u[q][t], s * r[t]);
+          r[t] = fma(c, r[t], -(s * u[q][t]));
+          if (j >= k && j < n) L[dst[t] + k] = x;
         }
-      };
-      int j = jbeg;
-      for (; j + 1 < jend; j += 2) { step(j, nA); step(j + 1, nB); }
-      if (j < jend) {
-        step(j, nA);
-#pragma unroll
-        for (int t = 0; t < NT; ++t) { const double tmp = nA[t]; nA[t] = nB[t]; nB[t] = tmp; }
+      }
+    };
+    load(k0, ua);
+#pragma unroll 1
+    for (int k = k0; k < kend; k += 2 * SWEEP) {
+      if (k + SWEEP < kend) load(k + SWEEP, ub);
+      rows(k, ua);
+      if (k + SWEEP < kend) {
+        if (k + 2 * SWEEP < kend) load(k + 2 * SWEEP, ua);
+        rows(k + SWEEP, ub);
       }
     }
+  }
+#pragma unroll
+  for (int t = 0; t < NT; ++t) { const int j = lane + 64 * t; if (j < n) S.v[cr + j] = vn[t]; }
+}
+
+// The downdate on wave 0, while wave 1 moves the rows above cr of the later
+// columns down by one column, in ascending order of destination (every source
+// lies above every earlier destination, so a batch never overwrites what a
+// later one reads; the two waves touch disjoint entries), and waves 1-3 do
+// the extra work, which touches neither the factor nor v.
+template <int KMAX, typename Extra>
+__device__ __forceinline__ void chol_downdate(Smem<KMAX>& S, int m, int cr, Extra extra) {
+  double* L = S.L;
+  if (wave_id() == 0) {
+    const int n = m - 1 - cr;
+    if (n <= 64) downdate_w0<KMAX, 1>(S, L, m, cr);
+    else if (KMAX <= 128 || n <= 128) downdate_w0<KMAX, 2>(S, L, m, cr);
+    else if (KMAX <= 192 || n <= 192) downdate_w0<KMAX, 3>(S, L, m, cr);
+    else downdate_w0<KMAX, 4>(S, L, m, cr);
   } else {
     if (wave_id() == 1) {
       // rows [0, cr) of logical columns [cr, m - 2]: physical column jl + 1
       // -> jl, element k = (jl - cr) * cr + i in ascending order
+      constexpr int DEEP = KMAX <= KMAX_LDS ? 4 : 16;
       const int total = (m - 1 - cr) * cr;
       const float rcr = cr > 0 ? 1.0f / (float)cr : 0.0f;
-      for (int k0 = 0; k0 < total; k0 += 64) {
-        const int k = k0 + lane;
-        if (k < total) {
+      for (int k0 = 0; k0 < total; k0 += 64 * DEEP) {
+        double x[DEEP];
+        int to[DEEP];
+#pragma unroll
+        for (int u = 0; u < DEEP; ++u) {
+          const int k = k0 + 64 * u + lane_id();
           int q = (int)((float)k * rcr);
           if (q * cr > k) --q;
           if ((q + 1) * cr <= k) ++q;
           const int jl = cr + q, i = k - q * cr;
-          S.L[P(jl) + i] = S.L[P(jl + 1) + i];
-        }
-      }
-    }
-    extra();   // waves 1-3: work that touches neither the factor nor v
-  }
-  __syncthreads();
-}
-
-// The same downdate for a factor in global memory (capacity above the LDS
-// factor's): rows rotated in place, then the sign fix and the compaction as
-// separate passes (LINPACK dchex job 2 + drop + sign fix,
-// src/symmmatrix.cpp:166-195).  Logical column jl >=
-// cr lives in physical column jl + 1 until the final compaction; rotation j
-// is generated from logical column j's rows (j, j + 1) and applied to every
-// later column at once (per element the same sequence as the sequential
-// loop).  The two rows a rotation touches stay in registers: lane jl % 64
-// keeps rows (j, j + 1) of its columns, reads the next row ahead from LDS
-// (rows below j + 1 are not rotated yet) and stores only the finished row,
-// and the owner of column j hands the rotation's inputs to all lanes with a
-// cross-lane read, so no step waits on an LDS round trip.
-//
-// v (U^T v = X^T y) goes through the same rotations and sign fix as the
-// factor's rows, so after the removal it solves the new factor's system
-// without a second triangular solve (the reference re-solves,
-// src/model.hpp:530-545; the two agree to rounding).
-template <int KMAX, typename Extra>
-__device__ __forceinline__ void chol_downdate_glb(Smem<KMAX>& S, int m, int cr, Extra extra) {
-  constexpr int NT = (KMAX + 63) / 64;
-  if (wave_id() == 0) {
-    const int lane = lane_id();
-    double vt = S.v[cr], vb = S.v[cr + 1];   // rows (j, j + 1) of v, all lanes
-    double top[NT], nxt[NT];
-#pragma unroll
-    for (int t = 0; t < NT; ++t) {
-      const int jl = lane + 64 * t;
-      const bool on = jl >= cr && jl <= m - 2;
-      top[t] = on ? S.L[P(jl + 1) + cr] : 0.0;
-      nxt[t] = on ? S.L[P(jl + 1) + cr + 1] : 0.0;
-    }
-#pragma unroll
-    for (int ti = 0; ti < NT; ++ti) {
-      const int jbeg = cr > 64 * ti ? cr : 64 * ti;
-      const int jend = (m - 1) < 64 * (ti + 1) ? (m - 1) : 64 * (ti + 1);
-      for (int j = jbeg; j < jend; ++j) {
-        const int owner = j & 63;
-        // every lane generates the rotation from the same two values
-        double a = readlane_d(top[ti], owner), b = readlane_d(nxt[ti], owner);
-        const double vbn = j + 2 < m ? S.v[j + 2] : 0.0;   // next row of v, read ahead
-        double cc, ss;
-        rot_gen(a, b, cc, ss);
-        if (lane == owner) S.L[P(j + 1) + j] = a;
-        {
-          const double tv = cc * vt + ss * vb;
-          vt = cc * vb - ss * vt;
-          if (lane == 0) S.v[j] = tv;
-          vb = vbn;
+          to[u] = P(jl) + i;
+          x[u] = k < total ? L[P(jl + 1) + i] : 0.0;
         }
 #pragma unroll
-        for (int t = ti; t < NT; ++t) {
-          const int jl = lane + 64 * t;
-          if (jl > j && jl <= m - 2) {
-            const double x1 = top[t], x2 = nxt[t];
-            const double tt = cc * x1 + ss * x2;
-            top[t] = cc * x2 - ss * x1;
-            S.L[P(jl + 1) + j] = tt;
-            nxt[t] = S.L[P(jl + 1) + j + 2];   // j + 2 <= jl + 1: inside the column
-          }
-        }
+        for (int u = 0; u < DEEP; ++u)
+          if (k0 + 64 * u + lane_id() < total) L[to[u]] = x[u];
       }
     }
-  } else {
-    extra();   // waves 1-3: work that touches neither the factor nor v
+    extra();
   }
   __syncthreads();
-  // sign fix over the kept rows i in [cr, m-2]: flags first, then negation
-  for (int i = cr + threadIdx.x; i <= m - 2; i += BMG_BLOCK) S.work[i] = S.L[P(i + 1) + i] < 0 ? -1.0 : 1.0;
-  __syncthreads();
-  // eight rows at a time with unconditional stores: a row past jl is
-  // clamped to jl, so its store rewrites col[jl] with the value the last
-  // real row gives it (a conditional store per row waits out an LDS round
-  // trip each)
-  for (int jl = cr + threadIdx.x; jl <= m - 2; jl += BMG_BLOCK) {
-    double* col = S.L + P(jl + 1);
-    for (int i0 = cr; i0 <= jl; i0 += 8) {
-      double c[8], f[8];
-#pragma unroll
-      for (int q = 0; q < 8; ++q) {
-        const int i = i0 + q <= jl ? i0 + q : jl;
-        c[q] = col[i];
-        f[q] = S.work[i];
-      }
-#pragma unroll
-      for (int q = 0; q < 8; ++q) {
-        const int i = i0 + q <= jl ? i0 + q : jl;
-        col[i] = f[q] < 0 ? -c[q] : c[q];
-      }
-    }
-    if (S.work[jl] < 0) S.v[jl] = -S.v[jl];
-  }
-  __syncthreads();
-  // compaction: logical column jl rows 0..jl <- physical column jl+1
-  const int e0 = P(cr), e1 = P(m - 1);
-  for (int base = e0; base < e1; base += BMG_BLOCK * 8) {
-    double tmp[8];
-#pragma unroll
-    for (int q = 0; q < 8; ++q) {
-      int e = base + q * BMG_BLOCK + threadIdx.x;
-      if (e < e1) {
-        int jl = (int)((sqrt(8.0 * e + 1.0) - 1.0) * 0.5);
-        while (P(jl + 1) <= e) ++jl;
-        while (P(jl) > e) --jl;
-        tmp[q] = S.L[P(jl + 1) + (e - P(jl))];
-      }
-    }
-    __syncthreads();
-#pragma unroll
-    for (int q = 0; q < 8; ++q) {
-      int e = base + q * BMG_BLOCK + threadIdx.x;
-      if (e < e1) S.L[e] = tmp[q];
-    }
-    __syncthreads();
-  }
-}
-
-template <int KMAX, typename Extra>
-__device__ __forceinline__ void chol_downdate(Smem<KMAX>& S, int m, int cr, Extra extra) {
-  if constexpr (KMAX <= KMAX_LDS) {
-    chol_downdate_lds(S, m, cr, extra);
-  } else {
-    chol_downdate_glb(S, m, cr, extra);
-  }
 }
 
 // Full factorisation of S.L (m x m, in place) in panels of CF_PB rows;
