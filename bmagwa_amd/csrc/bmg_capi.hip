@@ -19,8 +19,8 @@
 using namespace bmg;
 
 // kernels of bmg_chain.hip and bmg_data.hip
-template <int KMAX> __global__ void k_chains(KernelArgs);
-template <int KMAX> __global__ void k_model_op(ModelOpArgs);
+__global__ void k_chains(KernelArgs);
+__global__ void k_model_op(ModelOpArgs);
 __global__ void k_restride(const uint8_t*, uint64_t, uint32_t, uint32_t, uint8_t*);
 
 static thread_local std::string g_err;
@@ -428,7 +428,7 @@ extern "C" int bmg_scan_xtr(bmg_ctx* c, const double* r, int nvec, int coding, i
 struct bmg_batch {
   std::vector<bmg_ctx*> ctxs;
   int n_chains = 0;
-  int kmax = 128;
+  int kmax = 160;
   bmg_batch_cfg cfg{};
   std::vector<DevData> h_data;
   std::vector<ChainConst> h_consts;
@@ -548,28 +548,11 @@ extern "C" __global__ void k_init_chain_arrays(const DevData* data, const ChainC
   }
 }
 
-// Below 256 columns an iterating segment is two launches on the stream: the
-// batch capacity's kernel, which hands a chain whose model comes within one
-// iteration's growth of its capacity to the 256-column kernel at that
-// iteration, then the 256-column kernel, which runs those chains to the end
-// of the segment (its other workgroups return at once).
+// one launch per segment, a workgroup per chain
 static int launch_chain_kernel(bmg_batch* b, uint64_t n_iter, int mode) {
-  const int two = mode == 0 && b->kmax < BMG_KMAXG;
-  KernelArgs a{b->d_data, b->d_consts, b->d_scal, b->d_arrays, b->n_chains, n_iter, mode, two ? 1 : 0, 0};
-  switch (b->kmax) {
-    case 64: hipLaunchKernelGGL(k_chains<64>, dim3(b->n_chains), dim3(256), 0, b->stream, a); break;
-    case 128: hipLaunchKernelGGL(k_chains<128>, dim3(b->n_chains), dim3(256), 0, b->stream, a); break;
-    case 160: hipLaunchKernelGGL(k_chains<160>, dim3(b->n_chains), dim3(256), 0, b->stream, a); break;
-    default: hipLaunchKernelGGL(k_chains<256>, dim3(b->n_chains), dim3(256), 0, b->stream, a); break;
-  }
+  KernelArgs a{b->d_data, b->d_consts, b->d_scal, b->d_arrays, b->n_chains, n_iter, mode, b->kmax};
+  hipLaunchKernelGGL(k_chains, dim3(b->n_chains), dim3(256), 0, b->stream, a);
   BMG_HIP(hipGetLastError());
-  if (two) {
-    KernelArgs a2 = a;
-    a2.role = 2;
-    a2.small_kmax = b->kmax;
-    hipLaunchKernelGGL(k_chains<BMG_KMAXG>, dim3(b->n_chains), dim3(256), 0, b->stream, a2);
-    BMG_HIP(hipGetLastError());
-  }
   return BMG_OK;
 }
 
@@ -766,25 +749,12 @@ static int batch_create(bmg_ctx** ctxs, int n_ctx, int n_chains, const int32_t* 
   b->ctxs.assign(ctxs, ctxs + n_ctx);
   b->n_chains = n_chains;
   if (cfg) b->cfg = *cfg;
-  int kmax = 128;
+  int kmax = 160;
   b->device = ctxs[0]->device;
   hipSetDevice(b->device);
-  // capacity of the launch: the smallest compiled one that holds a typical
-  // model (the prior mean plus one move, AH: two columns a locus); a chain
-  // whose model comes within one move of it continues in the 256-column
-  // kernel from that iteration, so the capacity changes speed, not results
-  double typical = 0;
+  // capacity: the columns the factor in LDS holds (a chain whose model comes
+  // within one move of it goes on with the factor in HBM)
   if (b->cfg.max_model_size < 0) { delete b; set_error("max_model_size must be >= 0"); return BMG_E_ARG; }
-  for (int c = 0; c < n_chains; ++c) {
-    double typ = opts[c].e_qg + (double)opts[c].max_move_size + 8.0;
-    if (b->cfg.max_model_size > 0)
-      typ = std::min(typ, (double)b->cfg.max_model_size + (double)opts[c].max_move_size + 1.0);
-    for (int t = 0; t < opts[c].n_types; ++t)
-      if (opts[c].types[t] == BMG_AH) typ *= 2;
-    typical = std::max(typical, typ + 1);
-  }
-  kmax = typical <= 64 ? 64 : (typical <= 128 ? 128 : (typical <= 160 ? 160 : 256));
-  if (model_api) kmax = 160;
   if (b->cfg.capacity) {
     if (b->cfg.capacity != 64 && b->cfg.capacity != 128 && b->cfg.capacity != 160 && b->cfg.capacity != 256) {
       delete b; set_error("capacity must be 0, 64, 128, 160 or 256");
@@ -1621,12 +1591,7 @@ extern "C" int bmg_model_kmax(void) { return 160; }
 
 static int launch_model_op(bmg_batch* b, ModelOpArgs a) {
   a.data = b->d_data; a.consts = b->d_consts; a.scal = b->d_scal; a.arrays = b->d_arrays;
-  switch (b->kmax) {
-    case 64: hipLaunchKernelGGL(k_model_op<64>, dim3(1), dim3(256), 0, b->stream, a); break;
-    case 128: hipLaunchKernelGGL(k_model_op<128>, dim3(1), dim3(256), 0, b->stream, a); break;
-    case 160: hipLaunchKernelGGL(k_model_op<160>, dim3(1), dim3(256), 0, b->stream, a); break;
-    default: hipLaunchKernelGGL(k_model_op<256>, dim3(1), dim3(256), 0, b->stream, a); break;
-  }
+  hipLaunchKernelGGL(k_model_op, dim3(1), dim3(256), 0, b->stream, a);
   BMG_HIP(hipGetLastError());
   BMG_HIP(hipStreamSynchronize(b->stream));
   return BMG_OK;

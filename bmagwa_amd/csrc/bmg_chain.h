@@ -94,11 +94,6 @@ struct ChainScal {
   int32_t err;
   uint64_t tr_count, th_count, th_loci_len, th_beta_len;
   double tot_add, tot_rem;   // sum-tree totals
-  // capacity: a chain whose model comes within col_reserve columns of the
-  // launch's capacity continues in the 256-column kernel (big = 1) from the
-  // same iteration; seg_end is the iteration the current segment ends at
-  int32_t big;
-  uint64_t seg_end;
 };
 
 // Per-chain device arrays.  Every per-column array is laid out for
@@ -146,11 +141,9 @@ struct KernelArgs {
   int n_chains;
   uint64_t n_iter;     // iterations to run in this launch
   int mode;            // 0 iterate, 1 set-up
-  // 0: the only chain kernel of the segment; 1: the launch capacity's kernel,
-  // followed by 2: the 256-column kernel, which runs the chains with big = 1
-  // up to their seg_end
-  int role;
-  int small_kmax;      // role 2: the capacity of the role-1 kernel
+  // columns: a chain whose model comes within one iteration's growth of it
+  // continues in the 256-column code (64, 128, 160 or 256)
+  int capacity;
 };
 
 // one Model method on a one-chain state (the drop-in Model API)

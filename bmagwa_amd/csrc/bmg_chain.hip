@@ -75,6 +75,10 @@ __device__ __forceinline__ T* gp(T* p) {
 // member is a plain array in the LDS case (as a base-class member the
 // compiler's code for the triangular loops was a fifth slower).
 constexpr int KMAX_LDS = 160;
+// a chain returns from the 256-column code once its model is this many
+// columns inside the smaller capacity (a change costs a store and a load of
+// the chain's state, about one iteration)
+constexpr int CAP_BACK = 8;
 struct GlobalFactor {
   double* p;
   __device__ __forceinline__ operator double*() const { return gp(p); }
@@ -126,7 +130,9 @@ struct Smem {
   uint64_t sc_perm[BMG_MAXMS], sc_from[BMG_MAXMS], sc_to[BMG_MAXMS];
   double tlev[2][TLEV_LDS];              // sum-tree levels >= 2 (add, rem)
   int32_t win[512];                      // window of the current model_inds
-  uint64_t slots_cur[(KMAX + 63) / 64], slots_prop[(KMAX + 63) / 64];
+  // column slots in use (the slot space is that of the per-chain arrays, the
+  // same in every capacity, so a chain keeps its slots when it changes it)
+  uint64_t slots_cur[BMG_KMAXG / 64], slots_prop[BMG_KMAXG / 64];
   int32_t iacc[KMAX + 1];                // integer column dots of new_column_dots
   int32_t iacc2[KMAX + 1];               // the next addition's dots, formed ahead
   // delayed rejection: factor block, v, d and log d of the toggled loci's
@@ -230,15 +236,14 @@ __device__ __forceinline__ double dot_y_block(const uint32_t* __restrict__ w, ui
   return block_sum(s, red);
 }
 
-// The Makefile compiles this file once per model capacity (BMG_KMAX_ONLY =
-// 64, 128, 160, 256) so the four instantiations build in parallel; the
-// non-template code lives in the 64-column unit.
-#ifndef BMG_KMAX_ONLY
-#define BMG_KMAX_ONLY 0
+// The Makefile compiles this file twice so that the two kernels build in
+// parallel: BMG_CHAIN_UNIT 1 holds the sampler's, 2 the Model methods'.
+#ifndef BMG_CHAIN_UNIT
+#define BMG_CHAIN_UNIT 0
 #endif
-#define BMG_INST(K) (BMG_KMAX_ONLY == 0 || BMG_KMAX_ONLY == (K))
+#define BMG_UNIT(u) (BMG_CHAIN_UNIT == 0 || BMG_CHAIN_UNIT == (u))
 
-#if BMG_INST(64)
+#if BMG_UNIT(1)
 __global__ __launch_bounds__(BMG_BLOCK) void k_xy_all(DevData D, int coding, double* __restrict__ out) {
   __shared__ double red[8];
   for (uint64_t j = blockIdx.x; j < D.p; j += gridDim.x) {
@@ -1163,11 +1168,11 @@ template <int KMAX>
 __device__ __forceinline__ int alloc_slot(Ctx<KMAX>& C) {
   // lowest slot free in both the current and proposed models
   int s = -1;
-  for (int q = 0; q < (KMAX + 63) / 64 && s < 0; ++q) {
+  for (int q = 0; q < BMG_KMAXG / 64 && s < 0; ++q) {
     uint64_t used = C.S.slots_cur[q] | C.S.slots_prop[q];
     if (~used) s = 64 * q + __ffsll((long long)~used) - 1;
   }
-  return s < KMAX ? s : -1;
+  return s;
 }
 
 template <int KMAX>
@@ -1564,7 +1569,7 @@ __device__ __forceinline__ void commit(Ctx<KMAX>& C) {
   for (int i = threadIdx.x; i < R.n_rm; i += BMG_BLOCK) gp(C.A.model_inds)[S.rm_list[i]] = -1;
   __syncthreads();
   for (int i = threadIdx.x; i < R.nloci; i += BMG_BLOCK) gp(C.A.model_inds)[S.loci[i]] = i;
-  if (threadIdx.x < (KMAX + 63) / 64) S.slots_cur[threadIdx.x] = S.slots_prop[threadIdx.x];
+  if (threadIdx.x < BMG_KMAXG / 64) S.slots_cur[threadIdx.x] = S.slots_prop[threadIdx.x];
   __syncthreads();
   R.c_cols = R.cols; R.c_nloci = R.nloci;
   for (int q = 0; q < 5; ++q) R.c_Ns[q] = R.Ns[q];
@@ -1587,7 +1592,7 @@ __device__ __forceinline__ void restore(Ctx<KMAX>& C) {
   for (int i = threadIdx.x; i < R.c_nloci; i += BMG_BLOCK) {
     S.loci[i] = S.c_loci[i]; S.xi1[i] = S.c_xi1[i]; S.xi2[i] = S.c_xi2[i]; S.tind[i] = S.c_tind[i];
   }
-  if (threadIdx.x < (KMAX + 63) / 64) S.slots_prop[threadIdx.x] = S.slots_cur[threadIdx.x];
+  if (threadIdx.x < BMG_KMAXG / 64) S.slots_prop[threadIdx.x] = S.slots_cur[threadIdx.x];
   __syncthreads();
   R.cols = R.c_cols; R.nloci = R.c_nloci;
   for (int q = 0; q < 5; ++q) R.Ns[q] = R.c_Ns[q];
@@ -2958,7 +2963,7 @@ __device__ __forceinline__ void load_chain(Ctx<KMAX>& C, const ChainScal& CS) {
   R.pre_snp = -1; R.pre_slot = -1;
   const double* vec = gp(C.A.vec);
   const int32_t* idx = gp(C.A.idx);
-  for (int e = threadIdx.x; e < P(R.cols); e += BMG_BLOCK) S.L[e] = gp(C.A.Lcur)[e];
+  copy_factor(S.L, gp(C.A.Lcur), 0, P(R.cols));
   for (int i = threadIdx.x; i < KMAX; i += BMG_BLOCK) {
     S.xy[i] = S.c_xy[i] = vec[i];
     S.v[i] = S.c_v[i] = vec[BMG_KMAXG + i];
@@ -2973,12 +2978,12 @@ __device__ __forceinline__ void load_chain(Ctx<KMAX>& C, const ChainScal& CS) {
     S.xtype[i] = S.c_xtype[i] = (int8_t)idx[5 * BMG_KMAXG + i];
     S.tind[i] = S.c_tind[i] = (int8_t)idx[6 * BMG_KMAXG + i];
   }
-  if (threadIdx.x < (KMAX + 63) / 64) {
-    uint64_t m = 0;
-    for (int i = 0; i < R.cols; ++i)
-      if ((idx[3 * BMG_KMAXG + i] >> 6) == (int)threadIdx.x) m |= 1ull << (idx[3 * BMG_KMAXG + i] & 63);
-    S.slots_cur[threadIdx.x] = S.slots_prop[threadIdx.x] = m;
-  }
+  if (threadIdx.x < BMG_KMAXG / 64) S.slots_cur[threadIdx.x] = 0;
+  __syncthreads();
+  for (int i = threadIdx.x; i < R.cols; i += BMG_BLOCK)
+    atomicOr((unsigned long long*)&S.slots_cur[S.slot[i] >> 6], 1ull << (S.slot[i] & 63));
+  __syncthreads();
+  if (threadIdx.x < BMG_KMAXG / 64) S.slots_prop[threadIdx.x] = S.slots_cur[threadIdx.x];
   // sum-tree levels >= 2
   if (C.D.top >= 2) {
     uint64_t o2 = C.D.lev_off[2];
@@ -3066,27 +3071,31 @@ __device__ __forceinline__ void refresh_tau2(Ctx<KMAX>& C) {
   }
 }
 
+// Iterations of one chain from iteration it0 up to `end`, to the next RB
+// point, or until the model's size asks for the other capacity's code (in
+// *change; `cap`: the launch's capacity, in the 256-column code the one to go
+// back to, or 256).  Returns the iteration reached.
 template <int KMAX>
-__device__ __forceinline__ void run_iterations(Ctx<KMAX>& C, ChainScal& CS, uint64_t n_iter) {
+__device__ __forceinline__ uint64_t run_iterations(Ctx<KMAX>& C, ChainScal& CS, uint64_t it0, uint64_t end, int cap,
+                                                   int* change) {
   Smem<KMAX>& S = C.S;
   Reg& R = C.R;
   const ChainConst& K = C.K;
   double* adapt = gp(C.A.adapt);
-  uint64_t it0 = CS.n_iter;
   uint64_t pr[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-  for (uint64_t iter = it0; iter < it0 + n_iter; ++iter) {
+  uint64_t iter = it0;
+  *change = 0;
+  for (; iter < end; ++iter) {
     // a chain whose current model turned non-finite stops here; the host
     // reports it (the oracle stops with an error at the same point)
     if (R.err & ERR_STOP) break;
-    // a model within one iteration's growth of this kernel's capacity
-    // continues in the 256-column kernel from this iteration, before any
-    // draw of it, so the trajectory is the one a 256-column launch gives
-    if (KMAX < BMG_KMAXG && R.c_cols + K.col_reserve > KMAX) {
-      if (threadIdx.x == 0) {
-        CS.big = 1;
-#pragma unroll
-        for (int q = 0; q < 8; ++q) S.prof[q] += pr[q];
-      }
+    // a model within one iteration's growth of the capacity continues in
+    // the 256-column code from this iteration, before any draw of it, so
+    // the trajectory is the one a 256-column launch gives; it comes back
+    // once it is CAP_BACK columns inside again
+    if (KMAX < BMG_KMAXG ? R.c_cols + K.col_reserve > cap
+                         : cap < BMG_KMAXG && R.c_cols + K.col_reserve + CAP_BACK <= cap) {
+      *change = 1;
       break;
     }
     const uint64_t t_it = wall_clock64();
@@ -3175,14 +3184,6 @@ __device__ __forceinline__ void run_iterations(Ctx<KMAX>& C, ChainScal& CS, uint
       uint64_t t1 = wall_clock64(); pr[6] += t1 - t0; t0 = t1;
     }
     pr[7] += wall_clock64() - t_it;
-    if ((iter + 1) % K.n_rao == 0 || iter + 1 == it0 + n_iter) {
-      if (threadIdx.x == 0) {
-#pragma unroll
-        for (int q = 0; q < 8; ++q) S.prof[q] += pr[q];
-      }
-#pragma unroll
-      for (int q = 0; q < 8; ++q) pr[q] = 0;
-    }
     if ((iter + 1) % K.n_rao == 0) {
       // decide the RB block now; the scan and proposal update run as
       // separate kernels before the next iteration (src/sampler.cpp:731-811)
@@ -3224,69 +3225,70 @@ __device__ __forceinline__ void run_iterations(Ctx<KMAX>& C, ChainScal& CS, uint
           if (!K.flat) CS.rb_rebuild = 1;
         }
       }
-      if (threadIdx.x == 0) CS.n_iter = iter + 1;
-      __syncthreads();
-      return;   // the RB block runs before the next iteration
+      ++iter;
+      break;   // the RB block runs before the next iteration
     }
-    if (threadIdx.x == 0) CS.n_iter = iter + 1;
   }
+  if (threadIdx.x == 0) {
+    CS.n_iter = iter;
+#pragma unroll
+    for (int q = 0; q < 8; ++q) S.prof[q] += pr[q];
+  }
+  __syncthreads();
+  return iter;
 }
 
+// The chain in the code of one capacity: load, set up (mode 1) or iterate,
+// store.  Out of line: with both codes in one body the compiler runs out of
+// registers.
+struct Progress { uint64_t iter; int change; };
 template <int KMAX>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) void k_chains(KernelArgs args) {
-  __shared__ Smem<KMAX> S;
-  int c = blockIdx.x;
-  if (c >= args.n_chains) return;
+__device__ __noinline__ Progress run_capacity(Smem<KMAX>& S, KernelArgs args, uint64_t it0, uint64_t end) {
+  const int c = blockIdx.x;
   ChainScal& CS = args.scal[c];
   load_descriptions(S, args.data, args.consts + c, args.arrays + c);
   Reg R;
   Ctx<KMAX> C{S, R, S.D, S.K, S.A, S.prof};
-  if (args.mode == 1) {
+  load_chain(C, CS);
+  Progress g{it0, 0};
+  if (KMAX < BMG_KMAXG && args.mode == 1) {
     // setup (src/sampler.cpp:591-620): state was initialised on the host
     // with an empty model; compute its factor, then sample
-    load_chain(C, CS);
     compute_log_likelihood(C);
     commit(C);
     sample_beta_sigma2(C);
     refresh_tau2(C);
-    store_chain(C, CS);
-    return;
+  } else {
+    g.iter = run_iterations(C, CS, it0, end, args.capacity, &g.change);
   }
-  // role 1 fixes the segment's end for every chain; role 2 runs the chains
-  // that left the role-1 kernel's capacity, up to that end
-  if (args.role == 1 && threadIdx.x == 0) CS.seg_end = CS.n_iter + args.n_iter;
-  if (CS.rb_pending) return;   // the RB block must run first
-  uint64_t n_iter = args.n_iter;
-  if (args.role == 1 && CS.big) return;
-  if (args.role == 2) {
-    if (!CS.big || CS.seg_end <= CS.n_iter) return;
-    n_iter = CS.seg_end - CS.n_iter;
-  }
-  load_chain(C, CS);
-  run_iterations(C, CS, n_iter);
   store_chain(C, CS);
-  if (args.role == 2 && threadIdx.x == 0) {
-    // back to the launch capacity once the model is well inside it and
-    // every column's slot exists there
-    int top = 0;
-    for (int i = 0; i < R.c_cols; ++i) top = max(top, (int)S.c_slot[i]);
-    if (!(R.err & ERR_STOP) && R.c_cols + S.K.col_reserve + 8 <= args.small_kmax && top < args.small_kmax)
-      CS.big = 0;
-  }
+  return g;
 }
 
-// explicit instantiations used by the host
-#if BMG_INST(64)
-template __global__ void k_chains<64>(KernelArgs);
-#endif
-#if BMG_INST(128)
-template __global__ void k_chains<128>(KernelArgs);
-#endif
-#if BMG_INST(160)
-template __global__ void k_chains<160>(KernelArgs);
-#endif
-#if BMG_INST(256)
-template __global__ void k_chains<256>(KernelArgs);
+// A workgroup runs its chain to the end of the segment.  The kernel holds two
+// codes, one with the factor in LDS for up to KMAX_LDS columns and the
+// 256-column one with the factor in HBM, and a chain changes between them
+// where its model's size asks for it without leaving its workgroup, so a
+// launch lasts as long as its slowest chain.
+#if BMG_UNIT(1)
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) void k_chains(KernelArgs args) {
+  __shared__ union {
+    Smem<KMAX_LDS> small;
+    Smem<BMG_KMAXG> large;
+  } U;
+  const int c = blockIdx.x;
+  if (c >= args.n_chains) return;
+  const ChainScal& CS = args.scal[c];
+  if (args.mode == 0 && CS.rb_pending) return;   // the RB block must run first
+  Progress g{CS.n_iter, 0};
+  const uint64_t end = g.iter + args.n_iter;
+  int large = args.mode == 0 && (args.capacity == BMG_KMAXG || CS.cols + args.consts[c].col_reserve > args.capacity);
+  for (;;) {
+    g = large ? run_capacity(U.large, args, g.iter, end) : run_capacity(U.small, args, g.iter, end);
+    if (!g.change) break;
+    large ^= 1;
+  }
+}
 #endif
 
 // ------------------------------------------------------- model op kernel --
@@ -3321,8 +3323,9 @@ __device__ __forceinline__ void swapadj_w0(Smem<KMAX>& S, int m, int col) {
   __syncthreads();
 }
 
-template <int KMAX>
+#if BMG_UNIT(2)
 __global__ __launch_bounds__(256) void k_model_op(ModelOpArgs a) {
+  constexpr int KMAX = KMAX_LDS;
   __shared__ Smem<KMAX> S;
   ChainScal& CS = a.scal[0];
   load_descriptions(S, a.data, a.consts, a.arrays);
@@ -3352,20 +3355,9 @@ __global__ __launch_bounds__(256) void k_model_op(ModelOpArgs a) {
   store_chain(C, CS);
 }
 
-#if BMG_INST(64)
-template __global__ void k_model_op<64>(ModelOpArgs);
-#endif
-#if BMG_INST(128)
-template __global__ void k_model_op<128>(ModelOpArgs);
-#endif
-#if BMG_INST(160)
-template __global__ void k_model_op<160>(ModelOpArgs);
-#endif
-#if BMG_INST(256)
-template __global__ void k_model_op<256>(ModelOpArgs);
 #endif
 
-#if BMG_INST(64)
+#if BMG_UNIT(1)
 namespace bmg {
 
 int launch_xy_all(const DevData& D, int coding, double* out, hipStream_t s) {

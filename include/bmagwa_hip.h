@@ -269,12 +269,11 @@ typedef struct {
   int32_t learn_window;        /* learned: partners within this many SNPs */
   int32_t learn_steps;         /* learned: Adam steps per training round */
   int32_t learn_batch;         /* learned: rows per Adam step */
-  int32_t capacity;            /* model columns of the launch: 64, 128, 160
-                                  (factor in LDS) or 256 (factor in HBM); 0:
-                                  the smallest that holds the prior mean plus
-                                  one move (AH: twice).  A chain whose model
-                                  comes within one move of it continues in the
-                                  256-column kernel from that iteration (same
+  int32_t capacity;            /* model columns kept with the factor in LDS: 64,
+                                  128 or 160 (0: 160), or 256: always in HBM.
+                                  A chain whose model comes within one move of
+                                  it continues with the factor in HBM, up to 256
+                                  columns, from that iteration (same
                                   results); a proposal past 256 columns stops
                                   the chain and bmg_batch_run fails with
                                   BMG_E_CAPACITY (the reference's MAXMODELSIZE
