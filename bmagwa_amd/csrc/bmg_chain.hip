@@ -1767,12 +1767,119 @@ __device__ __forceinline__ void xbeta(Ctx<KMAX>& C, double* out8, int write_yhat
   xcoef(C, C.S.beta, C.R.beta_len, out8, write_yhat);
 }
 
+// A sum kept as an unevaluated pair (Dekker 1971, Knuth's two-sum), about 106
+// bits: the quadratic forms below cancel where columns are correlated.
+struct Pair { double hi, lo; };
+__device__ __forceinline__ void pair_add(Pair& s, double x, double e) {
+  const double t = s.hi + x, z = t - s.hi;
+  s.lo += ((s.hi - (t - z)) + (x - z)) + e;
+  s.hi = t;
+}
+__device__ __forceinline__ void pair_fma(Pair& s, double x, double y) {
+  const double p = x * y;
+  pair_add(s, p, fma(x, y, -p));
+}
+__device__ __forceinline__ void pair_fma(Pair& s, const Pair& x, double y) {
+  const double p = x.hi * y;
+  pair_add(s, p, fma(x.hi, y, -p) + x.lo * y);
+}
+
+// xcoef's sums (all but the residual's, out8[7]) from the model's X^T X and
+// X^T y, O(k^2) instead of O(n k): with a = X_g b_g and e = E b_E, sum a^2 =
+// b_g' (X_g^T X_g) b_g and so on, every sum a pair.  Lane j of each wave
+// takes column j, the waves every fourth row, so a load reads one row of the
+// slot matrix.  Bound by those reads (k^2 doubles through L2).  (Formed per
+// individual, with a conversion and a fused multiply-add per genotype, the
+// sums of a 139-column model at n = 10,000 took 140 us, once per thinned
+// sample and once per refresh.)  The entries are whole numbers but the
+// covariates'.
+template <int KMAX>
+__device__ __forceinline__ void xmoments(Ctx<KMAX>& C, const double* coef, int L, double* out8) {
+  constexpr int NQ = (KMAX + 63) / 64;
+  constexpr int BAT = 8;
+  Smem<KMAX>& S = C.S;
+  const int me = C.D.me;
+  const int lane = lane_id(), w = wave_id();
+  const double* __restrict__ xxs = gp(C.A.xxs);
+  // sum a, a^2, a e, e, e^2, a y
+  Pair m[6];
+#pragma unroll
+  for (int q = 0; q < 6; ++q) m[q] = Pair{0.0, 0.0};
+#pragma unroll 1
+  for (int q = 0; q < NQ; ++q) {
+    if (64 * q >= L) break;
+    const int j = 64 * q + lane;
+    const bool on = j < L;
+    const int sj = on ? S.slot[j] : S.slot[0];
+    const double bj = on ? coef[j] : 0.0;
+    Pair ug{0.0, 0.0}, ue{0.0, 0.0};
+    double g0 = 0.0;
+#pragma unroll 1
+    for (int i0 = w; i0 < L; i0 += 4 * BAT) {
+      double g[BAT];
+#pragma unroll
+      for (int u = 0; u < BAT; ++u) {
+        const int i = i0 + 4 * u;
+        g[u] = xxs[(size_t)S.slot[i < L ? i : 0] * BMG_KMAXG + sj];
+      }
+#pragma unroll
+      for (int u = 0; u < BAT; ++u) {
+        const int i = i0 + 4 * u;
+        if (i < me) {
+          pair_fma(ue, g[u], coef[i]);
+          if (i == 0) g0 = g[u];
+        } else if (i < L) {
+          pair_fma(ug, g[u], coef[i]);
+        }
+      }
+    }
+    if (j >= me) {
+      pair_fma(m[0], g0, bj);
+      pair_fma(m[1], ug, bj);
+      pair_fma(m[2], ue, bj);
+      if (w == 0 && on) pair_fma(m[5], S.xy[j], bj);
+    } else {
+      pair_fma(m[3], g0, bj);
+      pair_fma(m[4], ue, bj);
+    }
+  }
+  // the lanes' pairs, then the waves', in a fixed order
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1)
+#pragma unroll
+    for (int q = 0; q < 6; ++q) {
+      const double h = __shfl_xor(m[q].hi, o, 64), l = __shfl_xor(m[q].lo, o, 64);
+      pair_add(m[q], h, l);
+    }
+  __syncthreads();
+  if (lane == 0)
+#pragma unroll
+    for (int q = 0; q < 6; ++q) { S.work[12 * w + 2 * q] = m[q].hi; S.work[12 * w + 2 * q + 1] = m[q].lo; }
+  __syncthreads();
+  double v[6];
+#pragma unroll
+  for (int q = 0; q < 6; ++q) {
+    Pair t{S.work[2 * q], S.work[2 * q + 1]};
+    for (int ww = 1; ww < BMG_BLOCK / 64; ++ww) pair_add(t, S.work[12 * ww + 2 * q], S.work[12 * ww + 2 * q + 1]);
+    v[q] = t.hi + t.lo;
+  }
+  __syncthreads();
+  out8[0] = v[0]; out8[1] = v[1];
+  out8[2] = v[0] + v[3]; out8[3] = v[1] + 2.0 * v[2] + v[4];
+  out8[4] = v[2] - v[5];
+  out8[5] = v[3]; out8[6] = v[4]; out8[7] = 0.0;
+}
+
 // src/model.hpp:345-392: shares of var(E beta_E) (covariates beyond the
 // constant), var(X_g beta_g) and var(y_hat) in var(y_hat) + sigma2
+// (need_y: leave y_hat too.  Nothing reads the one of a sample that no RB scan
+// follows, and without covariates each is formed anew; with them a model
+// without loci adds to the one it holds, so every sample's is formed.)
 template <int KMAX>
-__device__ __forceinline__ void compute_pve(Ctx<KMAX>& C, double* pves) {
+__device__ __forceinline__ void compute_pve(Ctx<KMAX>& C, double* pves, int need_y) {
   double s[8];
-  xbeta(C, s, 1);
+  if (need_y || C.D.me > 1) xbeta(C, s, 1);
+  if (C.D.me == 1) xmoments(C, C.S.beta, C.R.beta_len, s);
   const double n = (double)C.D.n;
   const bool ce = C.D.me > 1, cg = C.R.nloci > 0;
   pves[2] = ce ? (s[6] - s[5] * s[5] / n) / (n - 1) : 0.0;
@@ -1867,7 +1974,7 @@ __device__ __forceinline__ void sample_alpha_and_tau2(Ctx<KMAX>& C) {
   if (nterms > 0) {
     // x_b = X_g beta_g, e_b = E beta_E - y
     double s[8];
-    xbeta(C, s, 0);
+    xmoments(C, S.beta, R.beta_len, s);
     ebxb = s[4];
     xbxb = s[1];
   }
@@ -3156,29 +3263,25 @@ __device__ __forceinline__ uint64_t run_iterations(Ctx<KMAX>& C, ChainScal& CS, 
     }
     if ((iter + 1) % K.thin == 0) {
       double pves[3];
-      compute_pve(C, pves);
+      compute_pve(C, pves, (iter + 1) % K.n_rao == 0);
+      const uint64_t t = S.cnt.th_count, ll0 = S.cnt.th_loci_len, b0 = S.cnt.th_beta_len;
+      const bool fits = t < K.th_cap && ll0 + R.c_nloci <= K.th_loci_cap;
+      // save_beta (src/sampler.cpp:710-713): the beta drawn for this sample
+      const bool keep_beta = fits && K.th_beta_cap != 0 && b0 + R.beta_len <= K.th_beta_cap;
+      if (fits)
+        for (int q = threadIdx.x; q < R.c_nloci; q += BMG_BLOCK) gp(C.A.th_loci)[ll0 + q] = S.c_loci[q];
+      if (keep_beta)
+        for (int q = threadIdx.x; q < R.beta_len; q += BMG_BLOCK) gp(C.A.th_beta)[b0 + q] = S.beta[q];
+      __syncthreads();
       if (threadIdx.x == 0) {
-        uint64_t t = S.cnt.th_count;
-        uint64_t ll0 = S.cnt.th_loci_len;
-        if (t < K.th_cap && ll0 + R.c_nloci <= K.th_loci_cap) {
+        if (fits) {
           gp(C.A.th_size)[t] = (uint32_t)R.c_nloci;
-          for (int q = 0; q < R.c_nloci; ++q) gp(C.A.th_loci)[ll0 + q] = S.c_loci[q];
           gp(C.A.th_ll)[t] = R.c_ll; gp(C.A.th_s2)[t] = R.sigma2; gp(C.A.th_alpha)[t] = R.alpha;
           gp(C.A.th_pve)[3 * t] = pves[0]; gp(C.A.th_pve)[3 * t + 1] = pves[1]; gp(C.A.th_pve)[3 * t + 2] = pves[2];
           S.cnt.th_count = t + 1; S.cnt.th_loci_len = ll0 + R.c_nloci;
-          // save_beta (src/sampler.cpp:710-713): the beta drawn for this sample
-          if (K.th_beta_cap) {
-            const uint64_t b0 = S.cnt.th_beta_len;
-            if (b0 + R.beta_len <= K.th_beta_cap) {
-              for (int q = 0; q < R.beta_len; ++q) gp(C.A.th_beta)[b0 + q] = S.beta[q];
-              S.cnt.th_beta_len = b0 + R.beta_len;
-            } else {
-              R.err |= ERR_TRACE;
-            }
-          }
-        } else {
-          R.err |= ERR_TRACE;
+          if (keep_beta) S.cnt.th_beta_len = b0 + R.beta_len;
         }
+        if (!fits || (K.th_beta_cap != 0 && !keep_beta)) R.err |= ERR_TRACE;
         CS.pves[0] = pves[0]; CS.pves[1] = pves[1]; CS.pves[2] = pves[2];
       }
       uint64_t t1 = wall_clock64(); pr[6] += t1 - t0; t0 = t1;
@@ -3347,7 +3450,7 @@ __global__ __launch_bounds__(256) void k_model_op(ModelOpArgs a) {
     sample_beta_sigma2(C);   // from the model's own stream
   } else if (a.op == 5) {
     double pv[3];
-    compute_pve(C, pv);      // leaves y_hat = X beta
+    compute_pve(C, pv, 1);   // leaves y_hat = X beta
     if (threadIdx.x == 0) { CS.pves[0] = pv[0]; CS.pves[1] = pv[1]; CS.pves[2] = pv[2]; }
   }
   R.lmin = 0;
