@@ -876,9 +876,6 @@ static int batch_create(bmg_ctx** ctxs, int n_ctx, int n_chains, const int32_t* 
     Kc.max_nbh = o.max_SNP_neighborhood_size;
     Kc.dr = (int32_t)std::min<uint64_t>(Kc.max_ms, o.delay_rejection);
     Kc.max_size = b->cfg.max_model_size > 0 ? b->cfg.max_model_size : INT32_MAX;
-    // a move adds at most max_move_size loci (two columns each for AH);
-    // one column of slack
-    Kc.col_reserve = (int32_t)Kc.max_ms * (x->types[0] == BMG_AH ? 2 : 1) + 1;
     Kc.adapt_p_ms = o.adapt_p_move_size && Kc.max_ms > 1;
     Kc.adaptation = o.adaptation; Kc.flat = o.flat_proposal_dist;
     Kc.trace_iter = b->cfg.trace_every_iter;

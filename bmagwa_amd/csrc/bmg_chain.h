@@ -56,7 +56,6 @@ struct ChainConst {
   double p_learned;      // probability of a learned swap per iteration
   int32_t dr;            // delayed-rejection move-size limit (0: none)
   int32_t max_size;      // largest model (SNPs) with nonzero prior
-  int32_t col_reserve;   // most columns one iteration can add to the current model
 };
 
 // Mutable per-chain scalars (device global memory).

@@ -77,8 +77,8 @@ __device__ __forceinline__ T* gp(T* p) {
 constexpr int KMAX_LDS = 160;
 // a chain returns from the 256-column code once its model is this many
 // columns inside the smaller capacity (a change costs a store and a load of
-// the chain's state, about one iteration)
-constexpr int CAP_BACK = 8;
+// the chain's state, about 20 us; nearly every move adds fewer SNPs)
+constexpr int CAP_BACK = 12;
 struct GlobalFactor {
   double* p;
   __device__ __forceinline__ operator double*() const { return gp(p); }
@@ -177,6 +177,10 @@ struct Reg {
   int pre_slot;                          // and the slot its value words went to
   double tj_tot[2];                      // tree totals when the move began
 };
+
+// how far a chain has come: the next iteration, whether its refresh is done
+// already, and whether the other capacity's code takes over there
+struct Progress { uint64_t iter; int change, refreshed; };
 
 template <int KMAX>
 struct Ctx {
@@ -2014,6 +2018,37 @@ __device__ __forceinline__ int sample_naive(const double* cumsum, int m, double 
   return b ? __ffsll((long long)b) - 1 : m - 1;
 }
 
+// PMV move mix with one effect type (src/sampler.cpp:468-476); with a
+// learned table, a drawn swap is a learned swap with probability
+// p_learned (both swaps keep the posterior; the choice does not depend
+// on the state, and add/remove and state-change moves keep their share).
+// 0 add/remove, 1 swap, 2 state change, 3 learned swap
+template <int KMAX>
+__device__ __forceinline__ int draw_move(const Ctx<KMAX>& C, Rng& rng) {
+  const double pm[3] = {0.7, 0.7 + 0.15, 0.7 + 0.15 + 0.15};
+  const double r = rng_u01(rng) * pm[2];
+  int move = r < pm[0] ? 0 : (r < pm[1] ? 1 : 2);
+  if (move == 1 && C.R.learn_on && rng_u01(rng) < C.K.p_learned) move = 3;
+  return move;
+}
+
+// the size of an add/remove (0), swap (1) or state-change (2) move
+template <int KMAX>
+__device__ __forceinline__ int draw_move_size(const Ctx<KMAX>& C, Rng& rng, int move) {
+  const ChainConst& K = C.K;
+  uint64_t mx = K.max_ms;
+  if (move == 1) {
+    const uint64_t half = (C.D.p - C.R.c_nloci + 1) / 2;
+    mx = (K.max_ms + 1) / 2;
+    mx = mx < half ? mx : half;
+    mx = mx < (uint64_t)C.R.c_nloci ? mx : (uint64_t)C.R.c_nloci;
+  } else if (move == 2) {
+    const uint64_t a = (uint64_t)K.max_nbh * 2, b = C.D.p - 1 < K.max_ms ? C.D.p - 1 : K.max_ms;
+    mx = a < b ? a : b;
+  }
+  return sample_naive(C.S.cdf[move], (int)mx, rng_u01(rng)) + 1;
+}
+
 template <int KMAX>
 __device__ __forceinline__ void undo_dd(Ctx<KMAX>& C, int ms) {
   for (int i = 0; i < ms; ++i) {
@@ -2552,8 +2587,7 @@ __device__ __forceinline__ int move_addrem(Ctx<KMAX>& C) {
   Reg& R = C.R;
   const ChainConst& K = C.K;
   const int type = C.D.type;
-  int max_ms = (int)K.max_ms;
-  int ms = sample_naive(S.cdf[0], max_ms, rng_u01(R.rng)) + 1;
+  int ms = draw_move_size(C, R.rng, 0);
   R.movesize = ms;
   double lqf = 0, lqb = 0, lmpc = 0;
   // the move's tree writes are journalled, so a rejection puts the trees
@@ -2720,10 +2754,7 @@ __device__ __forceinline__ int move_switch(Ctx<KMAX>& C) {
   Reg& R = C.R;
   const ChainConst& K = C.K;
   uint64_t full = C.D.p - R.c_nloci;
-  uint64_t mm2 = (K.max_ms + 1) / 2;
-  uint64_t mx = mm2 < (full + 1) / 2 ? mm2 : (full + 1) / 2;
-  mx = mx < (uint64_t)R.c_nloci ? mx : (uint64_t)R.c_nloci;
-  int ms = sample_naive(S.cdf[1], (int)mx, rng_u01(R.rng)) + 1;
+  int ms = draw_move_size(C, R.rng, 1);
   R.movesize = ms;
   uint64_t nbh = (full - ms) / 2;
   if (nbh < 1) nbh = 1;
@@ -2894,9 +2925,7 @@ __device__ __forceinline__ int move_statechange(Ctx<KMAX>& C) {
   const ChainConst& K = C.K;
   const int type = C.D.type;
   uint64_t m_g = C.D.p;
-  uint64_t a = (uint64_t)K.max_nbh * 2, b = m_g - 1 < K.max_ms ? m_g - 1 : K.max_ms;
-  uint64_t mx = a < b ? a : b;
-  int ms = sample_naive(S.cdf[2], (int)mx, rng_u01(R.rng)) + 1;
+  int ms = draw_move_size(C, R.rng, 2);
   R.movesize = ms;
   uint64_t nbh = K.max_nbh < m_g / 2 ? K.max_nbh : m_g / 2;
   int mic = (int)floor(rng_u01(R.rng) * R.nloci);
@@ -3178,52 +3207,77 @@ __device__ __forceinline__ void refresh_tau2(Ctx<KMAX>& C) {
   }
 }
 
-// Iterations of one chain from iteration it0 up to `end`, to the next RB
-// point, or until the model's size asks for the other capacity's code (in
-// *change; `cap`: the launch's capacity, in the 256-column code the one to go
-// back to, or 256).  Returns the iteration reached.
+// Columns that the next move can add to the current model at its largest:
+// the move and its size follow from the stream's next draws, read ahead here
+// on a copy of the stream.  Swaps remove before they add.
 template <int KMAX>
-__device__ __forceinline__ uint64_t run_iterations(Ctx<KMAX>& C, ChainScal& CS, uint64_t it0, uint64_t end, int cap,
-                                                   int* change) {
+__device__ __forceinline__ int next_growth(Ctx<KMAX>& C) {
+  Reg& R = C.R;
+  Rng q = R.rng;
+  const int move = draw_move(C, q);
+  if (move == 1 || move == 3) return 0;
+  const int ms = draw_move_size(C, q, move);
+  const int wide = C.D.type == BMG_AH ? 2 : 1;
+  if (move == 2 || R.c_cols + wide * ms <= KMAX_LDS) return wide * ms;
+  // an add/remove move: only the SNPs drawn for addition
+  uint64_t max_adds = C.D.p - R.c_nloci, max_rems = R.c_nloci;
+  int adds = 0;
+  for (int i = 0; i < ms; ++i) {
+    int add = 1;
+    if (max_rems == 0) add = 1;
+    else if (max_adds == 0) add = 0;
+    else add = rng_u01(q) < 0.5;
+    rng_skip(q, 1);
+    if (add) { --max_adds; ++adds; }
+    else --max_rems;
+  }
+  return wide * adds;
+}
+
+// Iterations of one chain from g.iter up to `end`, to the next RB point, or
+// until the model's size asks for the other capacity's code (g.change; `cap`:
+// the launch's capacity, in the 256-column code the one to go back to, or
+// 256).
+template <int KMAX>
+__device__ __forceinline__ void run_iterations(Ctx<KMAX>& C, ChainScal& CS, Progress& g, uint64_t end, int cap) {
   Smem<KMAX>& S = C.S;
   Reg& R = C.R;
   const ChainConst& K = C.K;
   double* adapt = gp(C.A.adapt);
   uint64_t pr[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-  uint64_t iter = it0;
-  *change = 0;
+  uint64_t iter = g.iter;
+  int refreshed = g.refreshed;
+  g.change = g.refreshed = 0;
   for (; iter < end; ++iter) {
     // a chain whose current model turned non-finite stops here; the host
     // reports it (the oracle stops with an error at the same point)
     if (R.err & ERR_STOP) break;
-    // a model within one iteration's growth of the capacity continues in
-    // the 256-column code from this iteration, before any draw of it, so
-    // the trajectory is the one a 256-column launch gives; it comes back
-    // once it is CAP_BACK columns inside again
-    if (KMAX < BMG_KMAXG ? R.c_cols + K.col_reserve > cap
-                         : cap < BMG_KMAXG && R.c_cols + K.col_reserve + CAP_BACK <= cap) {
-      *change = 1;
-      break;
-    }
     const uint64_t t_it = wall_clock64();
     uint64_t t0 = t_it;
-    if ((iter + 1) % K.n_st == 0) {
+    if ((iter + 1) % K.n_st == 0 && !refreshed) {
       refresh_tau2(C);
       if (!isfinite(R.c_ll)) R.err |= ERR_NONFINITE;
       uint64_t t1 = wall_clock64(); pr[0] += t1 - t0; t0 = t1;
     }
-    // PMV move mix with one effect type (src/sampler.cpp:468-476); with a
-    // learned table, a drawn swap is a learned swap with probability
-    // p_learned (both swaps keep the posterior; the choice does not depend
-    // on the state, and add/remove and state-change moves keep their share)
-    int move;
-    {
-      const double pm[3] = {0.7, 0.7 + 0.15, 0.7 + 0.15 + 0.15};
-      double u = rng_u01(R.rng);
-      double r = u * pm[2];
-      move = r < pm[0] ? 0 : (r < pm[1] ? 1 : 2);
+    refreshed = 0;
+    // a model that the move may take past the capacity continues in the
+    // 256-column code from here, before any of the move's draws, so the
+    // trajectory is the one a 256-column launch gives; it comes back once
+    // it is CAP_BACK columns inside again and the move fits.  (Deciding by
+    // the largest move there can be, max_move_size, kept chains past 139
+    // columns, 119 with two a SNP, out of the LDS code: 500 iterations of 8
+    // chains with two columns a SNP took 148 ms instead of 135, of 16 chains at
+    // n = 10,000, p = 500,000 139 instead of 135.)
+    if (cap < BMG_KMAXG) {
+      const int most = (int)K.max_ms * (C.D.type == BMG_AH ? 2 : 1);
+      if (KMAX < BMG_KMAXG ? R.c_cols + most > cap && R.c_cols + next_growth(C) > cap
+                           : R.c_cols + CAP_BACK <= cap && R.c_cols + next_growth(C) <= cap) {
+        g.change = 1;
+        g.refreshed = (iter + 1) % K.n_st == 0;
+        break;
+      }
     }
-    if (move == 1 && R.learn_on && rng_u01(R.rng) < K.p_learned) move = 3;
+    const int move = draw_move(C, R.rng);
     int jd = 0;
     if (move == 3) {
       if (R.c_nloci > 0) jd = move_learned_swap(C);
@@ -3338,22 +3392,20 @@ __device__ __forceinline__ uint64_t run_iterations(Ctx<KMAX>& C, ChainScal& CS, 
     for (int q = 0; q < 8; ++q) S.prof[q] += pr[q];
   }
   __syncthreads();
-  return iter;
+  g.iter = iter;
 }
 
 // The chain in the code of one capacity: load, set up (mode 1) or iterate,
 // store.  Out of line: with both codes in one body the compiler runs out of
 // registers.
-struct Progress { uint64_t iter; int change; };
 template <int KMAX>
-__device__ __noinline__ Progress run_capacity(Smem<KMAX>& S, KernelArgs args, uint64_t it0, uint64_t end) {
+__device__ __noinline__ Progress run_capacity(Smem<KMAX>& S, KernelArgs args, Progress g, uint64_t end) {
   const int c = blockIdx.x;
   ChainScal& CS = args.scal[c];
   load_descriptions(S, args.data, args.consts + c, args.arrays + c);
   Reg R;
   Ctx<KMAX> C{S, R, S.D, S.K, S.A, S.prof};
   load_chain(C, CS);
-  Progress g{it0, 0};
   if (KMAX < BMG_KMAXG && args.mode == 1) {
     // setup (src/sampler.cpp:591-620): state was initialised on the host
     // with an empty model; compute its factor, then sample
@@ -3362,7 +3414,7 @@ __device__ __noinline__ Progress run_capacity(Smem<KMAX>& S, KernelArgs args, ui
     sample_beta_sigma2(C);
     refresh_tau2(C);
   } else {
-    g.iter = run_iterations(C, CS, it0, end, args.capacity, &g.change);
+    run_iterations(C, CS, g, end, args.capacity);
   }
   store_chain(C, CS);
   return g;
@@ -3383,11 +3435,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
   if (c >= args.n_chains) return;
   const ChainScal& CS = args.scal[c];
   if (args.mode == 0 && CS.rb_pending) return;   // the RB block must run first
-  Progress g{CS.n_iter, 0};
+  Progress g{CS.n_iter, 0, 0};
   const uint64_t end = g.iter + args.n_iter;
-  int large = args.mode == 0 && (args.capacity == BMG_KMAXG || CS.cols + args.consts[c].col_reserve > args.capacity);
+  int large = args.mode == 0 && (args.capacity == BMG_KMAXG || CS.cols + CAP_BACK > args.capacity);
   for (;;) {
-    g = large ? run_capacity(U.large, args, g.iter, end) : run_capacity(U.small, args, g.iter, end);
+    g = large ? run_capacity(U.large, args, g, end) : run_capacity(U.small, args, g, end);
     if (!g.change) break;
     large ^= 1;
   }
