@@ -833,7 +833,7 @@ static int batch_create(bmg_ctx** ctxs, int n_ctx, int n_chains, const int32_t* 
          o_trl = add(8 * tr_cap);
   size_t o_ths = add(4 * th_cap), o_thl = add(4 * th_loci_cap), o_thll = add(8 * th_cap),
          o_ths2 = add(8 * th_cap), o_tha = add(8 * th_cap), o_thp = add(8 * 3 * th_cap);
-  size_t o_dr = add(dr_max ? (size_t)8 << dr_max : 0);
+  size_t o_dr = add(dr_max ? (size_t)16 << dr_max : 0);
   // save_beta: every thinned sample's beta (the fixed columns plus up to two
   // per locus)
   int any_beta = 0;
