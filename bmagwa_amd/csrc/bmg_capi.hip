@@ -472,6 +472,7 @@ struct bmg_batch {
 
 struct bmg_model {
   bmg_batch* b = nullptr;
+  ModelScalars* s = nullptr;   // pinned: the state's scalars after the last method
 };
 
 static void tree_layout(DevData& D) {
@@ -1586,11 +1587,29 @@ extern "C" int bmg_batch_rb(bmg_batch* b, int chain, const double* y_hat, double
 // ----------------------------------------------------------------- model --
 extern "C" int bmg_model_kmax(void) { return 160; }
 
-static int launch_model_op(bmg_batch* b, ModelOpArgs a) {
+static int launch_model_op(bmg_model* m, ModelOpArgs a) {
+  bmg_batch* b = m->b;
   a.data = b->d_data; a.consts = b->d_consts; a.scal = b->d_scal; a.arrays = b->d_arrays;
+  a.out = m->s;
   hipLaunchKernelGGL(k_model_op, dim3(1), dim3(256), 0, b->stream, a);
   BMG_HIP(hipGetLastError());
   BMG_HIP(hipStreamSynchronize(b->stream));
+  return BMG_OK;
+}
+
+// a model on the one-chain batch b (which it owns from here on): its empty
+// state's log-likelihood computed
+static int model_open(bmg_batch* b, bmg_model** out) {
+  bmg_model* m = new bmg_model();
+  m->b = b;
+  hipError_t e = hipHostMalloc((void**)&m->s, sizeof(ModelScalars));
+  if (e != hipSuccess) { bmg_model_destroy(m); return hip_fail(e, "hipHostMalloc"); }
+  std::memset(m->s, 0, sizeof(ModelScalars));
+  ModelOpArgs a{};
+  a.op = 2;
+  int rc = launch_model_op(m, a);
+  if (rc) { bmg_model_destroy(m); return rc; }
+  *out = m;
   return BMG_OK;
 }
 
@@ -1625,14 +1644,7 @@ extern "C" int bmg_model_create(bmg_ctx* ctx, const bmg_model_prior* prior, bmg_
   K.nus2_plus_yy = prior->nus2_plus_yy;
   K.nus2 = prior->nus2_plus_yy - ctx->yy;
   BMG_HIP(hipMemcpy(b->d_consts, &K, sizeof(ChainConst), hipMemcpyHostToDevice));
-  bmg_model* m = new bmg_model();
-  m->b = b;
-  ModelOpArgs a{};
-  a.op = 2;
-  rc = launch_model_op(b, a);
-  if (rc) { bmg_batch_destroy(b); delete m; return rc; }
-  *out = m;
-  return BMG_OK;
+  return model_open(b, out);
 }
 
 extern "C" int bmg_model_create_sampler(bmg_ctx* ctx, const bmg_opts* opts, bmg_model** out) {
@@ -1647,25 +1659,16 @@ extern "C" int bmg_model_create_sampler(bmg_ctx* ctx, const bmg_opts* opts, bmg_
   bmg_batch* b = nullptr;
   int rc = batch_create(&ctx, 1, 1, &zero, &o, &cfg, 1, &b);
   if (rc) return rc;
-  bmg_model* m = new bmg_model();
-  m->b = b;
-  ModelOpArgs a{};
-  a.op = 2;
-  rc = launch_model_op(b, a);
-  if (rc) { bmg_batch_destroy(b); delete m; return rc; }
-  *out = m;
-  return BMG_OK;
+  return model_open(b, out);
 }
 
 extern "C" int bmg_model_sample_beta_sigma2(bmg_model* m) {
   if (!m) { set_error("null model"); return BMG_E_ARG; }
   ModelOpArgs a{};
   a.op = 4;
-  int rc = launch_model_op(m->b, a);
+  int rc = launch_model_op(m, a);
   if (rc) return rc;
-  ChainScal s;
-  BMG_HIP(hipMemcpy(&s, m->b->d_scal, sizeof(ChainScal), hipMemcpyDeviceToHost));
-  if (s.err & ERR_SIGMA2) { set_error("sigma2 draw did not finish (non-finite residual sum)"); return BMG_E_NUMERIC; }
+  if (m->s->err & ERR_SIGMA2) { set_error("sigma2 draw did not finish (non-finite residual sum)"); return BMG_E_NUMERIC; }
   return BMG_OK;
 }
 
@@ -1673,11 +1676,9 @@ extern "C" int bmg_model_compute_pve(bmg_model* m, double pves[3]) {
   if (!m || !pves) { set_error("null argument"); return BMG_E_ARG; }
   ModelOpArgs a{};
   a.op = 5;
-  int rc = launch_model_op(m->b, a);
+  int rc = launch_model_op(m, a);
   if (rc) return rc;
-  ChainScal s;
-  BMG_HIP(hipMemcpy(&s, m->b->d_scal, sizeof(ChainScal), hipMemcpyDeviceToHost));
-  for (int i = 0; i < 3; ++i) pves[i] = s.pves[i];
+  for (int i = 0; i < 3; ++i) pves[i] = m->s->pves[i];
   return BMG_OK;
 }
 
@@ -1716,6 +1717,7 @@ extern "C" int bmg_model_rollback(bmg_model* proposed, const bmg_model* current)
 extern "C" int bmg_model_destroy(bmg_model* m) {
   if (!m) return BMG_OK;
   bmg_batch_destroy(m->b);
+  if (m->s) (void)hipHostFree(m->s);
   delete m;
   return BMG_OK;
 }
@@ -1727,54 +1729,44 @@ extern "C" int bmg_model_add_term(bmg_model* m, uint32_t ind, int t_ind, const d
   a.op = 0; a.ind = ind; a.t_ind = t_ind; a.d0 = d[0];
   const DevData& D = m->b->h_data[0];
   a.d1 = (t_ind >= 0 && t_ind < D.n_types && D.types[t_ind] == BMG_AH) ? d[1] : 0.0;
-  int rc = launch_model_op(m->b, a);
+  int rc = launch_model_op(m, a);
   if (rc) return rc;
-  ChainScal s;
-  BMG_HIP(hipMemcpy(&s, m->b->d_scal, sizeof(ChainScal), hipMemcpyDeviceToHost));
-  if (s.err & ERR_CAPACITY) { set_error("model capacity exceeded"); return BMG_E_CAPACITY; }
+  if (m->s->err & ERR_CAPACITY) { set_error("model capacity exceeded"); return BMG_E_CAPACITY; }
   return BMG_OK;
 }
 
 extern "C" int bmg_model_remove_term(bmg_model* m, int model_ind) {
   if (!m) { set_error("null model"); return BMG_E_ARG; }
-  ChainScal s;
-  BMG_HIP(hipMemcpy(&s, m->b->d_scal, sizeof(ChainScal), hipMemcpyDeviceToHost));
-  if (model_ind < 0 || model_ind >= s.nloci) { set_error("model_ind out of range"); return BMG_E_ARG; }
+  if (model_ind < 0 || model_ind >= m->s->nloci) { set_error("model_ind out of range"); return BMG_E_ARG; }
   ModelOpArgs a{};
   a.op = 1; a.model_ind = model_ind;
-  return launch_model_op(m->b, a);
+  return launch_model_op(m, a);
 }
 
 extern "C" int bmg_model_compute_log_likelihood(bmg_model* m) {
   if (!m) { set_error("null model"); return BMG_E_ARG; }
   ModelOpArgs a{};
   a.op = 2;
-  return launch_model_op(m->b, a);
+  return launch_model_op(m, a);
 }
 
 extern "C" int bmg_model_swapadj(bmg_model* m, int col) {
   if (!m) { set_error("null model"); return BMG_E_ARG; }
-  ChainScal s;
-  BMG_HIP(hipMemcpy(&s, m->b->d_scal, sizeof(ChainScal), hipMemcpyDeviceToHost));
-  if (col < 0 || col + 1 >= s.cols) { set_error("col out of range"); return BMG_E_ARG; }
+  if (col < 0 || col + 1 >= m->s->cols) { set_error("col out of range"); return BMG_E_ARG; }
   ModelOpArgs a{};
   a.op = 3; a.model_ind = col;
-  return launch_model_op(m->b, a);
+  return launch_model_op(m, a);
 }
 
 extern "C" int bmg_model_log_likelihood(bmg_model* m, double* out) {
   if (!m || !out) { set_error("null argument"); return BMG_E_ARG; }
-  ChainScal s;
-  BMG_HIP(hipMemcpy(&s, m->b->d_scal, sizeof(ChainScal), hipMemcpyDeviceToHost));
-  *out = s.ll;
+  *out = m->s->ll;
   return BMG_OK;
 }
 
 extern "C" int bmg_model_size(bmg_model* m, int* out) {
   if (!m || !out) { set_error("null argument"); return BMG_E_ARG; }
-  ChainScal s;
-  BMG_HIP(hipMemcpy(&s, m->b->d_scal, sizeof(ChainScal), hipMemcpyDeviceToHost));
-  *out = s.nloci;
+  *out = m->s->nloci;
   return BMG_OK;
 }
 
@@ -1791,9 +1783,13 @@ extern "C" int bmg_model_copy(bmg_model* dst, const bmg_model* src) {
   bmg_batch* a = src->b;
   bmg_batch* b = dst->b;
   if (a->kmax != b->kmax || a->h_data[0].p != b->h_data[0].p) { set_error("incompatible models"); return BMG_E_ARG; }
-  BMG_HIP(hipMemcpy(b->pool, a->pool, a->per_chain, hipMemcpyDeviceToDevice));
-  // the pool copy moved every array; the scalar block carries the rest
-  BMG_HIP(hipMemcpy(b->d_scal, a->d_scal, sizeof(ChainScal), hipMemcpyDeviceToDevice));
+  // every array (what follows them, the delayed-rejection scratch and the
+  // saved betas, is not the model's), then the scalar block; the methods
+  // leave both streams idle
+  BMG_HIP(hipMemcpyAsync(b->pool, a->pool, std::min(a->per_chain, b->per_chain), hipMemcpyDeviceToDevice, b->stream));
+  BMG_HIP(hipMemcpyAsync(b->d_scal, a->d_scal, sizeof(ChainScal), hipMemcpyDeviceToDevice, b->stream));
+  BMG_HIP(hipStreamSynchronize(b->stream));
+  *dst->s = *src->s;
   return BMG_OK;
 }
 

@@ -145,6 +145,13 @@ struct KernelArgs {
   int capacity;
 };
 
+// what the host reads after a Model method: in pinned host memory, which the
+// kernel writes itself, so a call waits for its kernel and copies nothing
+struct ModelScalars {
+  double ll, pves[3];
+  int32_t cols, nloci, err, pad;
+};
+
 // one Model method on a one-chain state (the drop-in Model API)
 struct ModelOpArgs {
   const bmg::DevData* data;
@@ -156,6 +163,7 @@ struct ModelOpArgs {
   uint32_t ind;
   int t_ind, model_ind;
   double d0, d1;
+  ModelScalars* out;   // pinned host memory
 };
 
 namespace bmg {

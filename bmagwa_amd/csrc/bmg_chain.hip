@@ -3433,8 +3433,13 @@ __global__ __launch_bounds__(256) void k_model_op(ModelOpArgs a) {
   R.lmin = 0;
   commit(C);
   store_chain(C, CS);
+  if (threadIdx.x == 0) {
+    a.out->ll = R.c_ll;
+    a.out->cols = R.c_cols; a.out->nloci = R.c_nloci; a.out->err = R.err;
+    if (a.op == 5)
+      for (int q = 0; q < 3; ++q) a.out->pves[q] = CS.pves[q];
+  }
 }
-
 #endif
 
 #if BMG_UNIT(1)
