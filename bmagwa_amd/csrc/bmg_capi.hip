@@ -446,7 +446,6 @@ struct bmg_batch {
   int device = 0;
   hipStream_t stream = nullptr;
   // RB scratch
-  double* r = nullptr; size_t r_bytes = 0;
   double* xa = nullptr; size_t xa_bytes = 0;
   double* xh = nullptr; size_t xh_bytes = 0;
   double* rsum = nullptr;
@@ -557,8 +556,7 @@ static int launch_chain_kernel(bmg_batch* b, uint64_t n_iter, int mode) {
   return BMG_OK;
 }
 
-static int ensure_rb_scratch(bmg_batch* b, int nv, uint32_t n_pad, uint64_t p) {
-  if (ensure((void**)&b->r, &b->r_bytes, sizeof(double) * nv * n_pad)) return BMG_E_HIP;
+static int ensure_rb_scratch(bmg_batch* b, int nv, uint64_t p) {
   if (ensure((void**)&b->xa, &b->xa_bytes, sizeof(double) * nv * p)) return BMG_E_HIP;
   if (ensure((void**)&b->xh, &b->xh_bytes, sizeof(double) * nv * p)) return BMG_E_HIP;
   return BMG_OK;
@@ -572,17 +570,14 @@ static int rb_block_ds(bmg_batch* b, int ds, const std::vector<int>& chains, int
   int per = 16 / digits;
   for (size_t s0 = 0; s0 < chains.size(); s0 += per) {
     int nv = (int)std::min<size_t>(per, chains.size() - s0);
-    if (ensure_rb_scratch(b, nv, D.n_pad, D.p)) return BMG_E_HIP;
+    if (ensure_rb_scratch(b, nv, D.p)) return BMG_E_HIP;
     BMG_HIP(hipMemcpyAsync(b->d_list, chains.data() + s0, sizeof(int) * nv, hipMemcpyHostToDevice,
                            b->stream));
-    if (launch_residuals(c->y, D.n, D.n_pad, b->d_arrays, b->d_list, nv, b->r, b->rsum, b->stream)) {
-      set_error("residual kernel launch failed"); return BMG_E_HIP;
-    }
     int t = D.type;
-    int rc = launch_scan(c, b->r, nv, t == BMG_AH ? 0 : t, digits, b->xa, b->stream);
+    int rc = launch_scan_chains(c, b->d_arrays, b->d_list, nv, t == BMG_AH ? 0 : t, digits, b->rsum, b->xa, b->stream);
     if (rc) return rc;
     if (t == BMG_AH) {
-      rc = launch_scan(c, b->r, nv, 1, digits, b->xh, b->stream);
+      rc = launch_scan_chains(c, b->d_arrays, b->d_list, nv, 1, digits, b->rsum, b->xh, b->stream);
       if (rc) return rc;
     }
     b->n_scans += (t == BMG_AH) ? 2 : 1;
@@ -728,7 +723,7 @@ extern "C" int bmg_batch_destroy(bmg_batch* b) {
   hipFree(b->pool); hipFree(b->d_data); hipFree(b->d_consts); hipFree(b->d_scal); hipFree(b->d_arrays);
   for (float* w : b->lw_dev) hipFree(w);
   for (LearnDS* L : b->learn) learn_destroy(L);
-  hipFree(b->r); hipFree(b->xa); hipFree(b->xh); hipFree(b->rsum); hipFree(b->d_list);
+  hipFree(b->xa); hipFree(b->xh); hipFree(b->rsum); hipFree(b->d_list);
   if (b->graph_exec) hipGraphExecDestroy(b->graph_exec);
   if (b->graph) hipGraphDestroy(b->graph);
   hipFree(b->d_glist);
@@ -1083,7 +1078,7 @@ static int steady_state(bmg_batch* b) {
 
 // the buffers a captured segment points at; a change means a rebuild
 static std::vector<const void*> graph_signature(bmg_batch* b) {
-  std::vector<const void*> v = {b->r, b->xa, b->xh, b->rsum, b->d_glist};
+  std::vector<const void*> v = {b->xa, b->xh, b->rsum, b->d_glist};
   for (bmg_ctx* c : b->ctxs) { v.push_back(c->dig); v.push_back(c->acc); v.push_back(c->scale); }
   return v;
 }
@@ -1104,7 +1099,7 @@ static int build_graph(bmg_batch* b) {
   if (!b->d_glist) BMG_HIP(hipMalloc(&b->d_glist, sizeof(int) * b->n_chains));
   BMG_HIP(hipMemcpy(b->d_glist, order.data(), sizeof(int) * order.size(), hipMemcpyHostToDevice));
   for (size_t ds = 0; ds < b->ctxs.size(); ++ds)
-    if (ensure_rb_scratch(b, per, b->h_data[ds].n_pad, b->h_data[ds].p)) return BMG_E_HIP;
+    if (ensure_rb_scratch(b, per, b->h_data[ds].p)) return BMG_E_HIP;
   int scans = 0;
   BMG_HIP(hipStreamBeginCapture(b->stream, hipStreamCaptureModeRelaxed));
   int rc = launch_chain_kernel(b, b->n_rao, 0);
@@ -1115,12 +1110,9 @@ static int build_graph(bmg_batch* b) {
     for (size_t s0 = ds_off[ds]; s0 < ds_off[ds + 1] && !rc; s0 += per) {
       const int nv = (int)std::min<size_t>(per, ds_off[ds + 1] - s0);
       const int* list = b->d_glist + s0;
-      if (launch_residuals(c->y, D.n, D.n_pad, b->d_arrays, list, nv, b->r, b->rsum, b->stream)) {
-        set_error("residual kernel launch failed"); rc = BMG_E_HIP; break;
-      }
       const int t = D.type;
-      rc = launch_scan(c, b->r, nv, t == BMG_AH ? 0 : t, digits, b->xa, b->stream);
-      if (!rc && t == BMG_AH) rc = launch_scan(c, b->r, nv, 1, digits, b->xh, b->stream);
+      rc = launch_scan_chains(c, b->d_arrays, list, nv, t == BMG_AH ? 0 : t, digits, b->rsum, b->xa, b->stream);
+      if (!rc && t == BMG_AH) rc = launch_scan_chains(c, b->d_arrays, list, nv, 1, digits, b->rsum, b->xh, b->stream);
       scans += (t == BMG_AH) ? 2 : 1;
       if (!rc && launch_rb_finalize(b->d_data, b->d_consts, b->d_scal, b->d_arrays, list, nv, BMG_KMAXG, D.p,
                                     b->xa, b->xh, b->rsum, b->stream)) {

@@ -7,6 +7,9 @@
 #include <mutex>
 #include <vector>
 
+#include <hip/hip_runtime.h>
+
+#include "bmg_chain.h"
 #include "bmg_device.h"
 #include "bmg_internal.h"
 
@@ -171,38 +174,67 @@ __global__ void k_synth(uint32_t seed, uint32_t n, uint64_t p, uint32_t W32,
 // (v_mfma_i32_16x16x64_i8): A = 16 SNPs x 64 individuals (2-bit codes
 // expanded to int8 in registers), B = 64 individuals x 16 digit columns
 // (vector v, digit d at column v*D + d).  x^T r = 2^e sum_d 256^d C_d.
-__global__ void k_absmax(const double* __restrict__ r, uint32_t n_pad, int nvec,
-                         double* __restrict__ scale, int digits) {
-  __shared__ double red[8];
-  int v = blockIdx.x;
-  double m = 0.0;
-  for (uint32_t i = threadIdx.x; i < n_pad; i += blockDim.x) m = fmax(m, fabs(r[v * (size_t)n_pad + i]));
-  m = wave_max(m);
-  __syncthreads();
-  if ((threadIdx.x & 63) == 0) red[threadIdx.x / 64] = m;
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    double t = 0;
-    for (int i = 0; i < (int)(blockDim.x / 64); ++i) t = fmax(t, red[i]);
-    int e = 0;
-    if (t > 0) { frexp(t, &e); }          // t < 2^e
-    scale[v] = ldexp(1.0, e - (8 * digits - 2));
+//
+// k_scan_prepare: the scale and the digit planes of every vector.  Each of
+// the PREP_WGS workgroups of a vector finds the vector's largest magnitude
+// (and, for a chain's residual y - y_hat, its sum, in the same fixed order)
+// by itself, a read of L2 that costs less than a second launch, and then
+// splits its part of the individuals.  (One workgroup of 256 lanes for the
+// residual, one for the maximum and a launch for the digits took 21 + 19 + 4
+// us at n = 10,000, most of it loads waited for one at a time.  With this and
+// the results formed by the scan itself, a scan of 3 vectors at n = 10,000, p =
+// 500,000 went from 282 to 245 us, one of 2,000 x 13,000 from 20 to 15.)
+#define PREP_WGS 8
+#define PREP_LANES 1024
+template <bool CHAIN>
+__global__ __launch_bounds__(PREP_LANES) void k_scan_prepare(const double* __restrict__ r, uint32_t n, uint32_t n_pad,
+                                                             const ChainArrays* __restrict__ arrays,
+                                                             const int* __restrict__ list, int digits,
+                                                             double* __restrict__ scale, double* __restrict__ rsum,
+                                                             int8_t* __restrict__ dig) {
+  __shared__ double red[2][PREP_LANES / 64];
+  const int v = blockIdx.y;
+  const double* __restrict__ yh = CHAIN ? arrays[list[v]].y_hat : nullptr;
+  const double* __restrict__ rv = CHAIN ? r : r + (size_t)v * n_pad;   // CHAIN: y
+  auto value = [&](uint32_t i) -> double { return CHAIN ? (i < n ? rv[i] - yh[i] : 0.0) : rv[i]; };
+  double m = 0.0, s = 0.0;
+  for (uint32_t i0 = threadIdx.x; i0 < n_pad; i0 += 4 * PREP_LANES) {
+    double x[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) x[u] = i0 + u * PREP_LANES < n_pad ? value(i0 + u * PREP_LANES) : 0.0;
+#pragma unroll
+    for (int u = 0; u < 4; ++u) { m = fmax(m, fabs(x[u])); s += x[u]; }
   }
-}
-
-__global__ void k_digits(const double* __restrict__ r, uint32_t n_pad, int nvec, int digits,
-                         const double* __restrict__ scale, int8_t* __restrict__ dig) {
-  uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-  int v = blockIdx.y;
-  if (i >= n_pad) return;
-  long long R = llrint(r[v * (size_t)n_pad + i] / scale[v]);
-  // within each group of 16 individuals, individual 4j + s sits at byte
-  // 4s + j: the order in which the scan kernel splits a genotype word
-  const uint32_t l = i & 15u, pos = (i & ~15u) | (4u * (l & 3u) + (l >> 2));
-  for (int d = 0; d < digits; ++d) {
-    int dg = (int)(((R + 128) & 0xFF)) - 128;
-    dig[(size_t)(v * digits + d) * n_pad + pos] = (int8_t)dg;
-    R = (R - dg) >> 8;
+  m = wave_max(m);
+  if (CHAIN) s = wave_sum(s);
+  if ((threadIdx.x & 63) == 0) { red[0][threadIdx.x / 64] = m; red[1][threadIdx.x / 64] = s; }
+  __syncthreads();
+  m = 0.0;
+  s = 0.0;
+  for (int i = 0; i < PREP_LANES / 64; ++i) { m = fmax(m, red[0][i]); s += red[1][i]; }
+  int e = 0;
+  if (m > 0) { frexp(m, &e); }          // m < 2^e
+  const double sc = ldexp(1.0, e - (8 * digits - 2));
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    scale[v] = sc;
+    if (CHAIN) rsum[v] = s;
+  }
+  // 16 individuals a lane: individual 4j + k sits at byte 4k + j, the order
+  // in which the scan kernel splits a genotype word
+  for (uint32_t w = blockIdx.x * PREP_LANES + threadIdx.x; w < n_pad / 16; w += PREP_WGS * PREP_LANES) {
+    long long R[16];
+#pragma unroll
+    for (int l = 0; l < 16; ++l) R[l] = llrint(value(16 * w + l) / sc);
+    for (int d = 0; d < digits; ++d) {
+      uint32_t out[4] = {0, 0, 0, 0};
+#pragma unroll
+      for (int l = 0; l < 16; ++l) {
+        const int dg = (int)((R[l] + 128) & 0xFF) - 128;
+        out[l & 3] |= (uint32_t)(uint8_t)dg << (8 * (l >> 2));
+        R[l] = (R[l] - dg) >> 8;
+      }
+      *(uint4*)(dig + (size_t)(v * digits + d) * n_pad + 16 * w) = make_uint4(out[0], out[1], out[2], out[3]);
+    }
   }
 }
 
@@ -239,7 +271,9 @@ template <int NT, int CODING, int WAVES, bool ATOMIC>
 __global__ __launch_bounds__(64 * WAVES) void k_scan_mfma(const uint32_t* __restrict__ g, uint64_t p,
                                                           uint32_t W32, const int8_t* __restrict__ dig,
                                                           int NC, uint32_t n_pad, uint32_t tile_words,
-                                                          int32_t* __restrict__ acc) {
+                                                          int32_t* __restrict__ acc, int digits,
+                                                          const double* __restrict__ scale,
+                                                          double* __restrict__ out) {
   extern __shared__ int8_t sdig[];  // NC x (tile_words * 16 + 16), tile_words a multiple of 32
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const uint32_t w0 = blockIdx.y * tile_words;
@@ -259,6 +293,11 @@ __global__ __launch_bounds__(64 * WAVES) void k_scan_mfma(const uint32_t* __rest
   const int row = lane & 15, grp = lane >> 4;
   const int col = row;
   const int8_t* bcol = sdig + (size_t)min(col, NC - 1) * ld + grp * 64;
+  // this lane's vector: its scale, its row of the result
+  const bool stores = col < NC && col % digits == 0;
+  const int vec = min(col, NC - 1) / digits;
+  const double sc = ATOMIC ? 0.0 : scale[vec];
+  double* __restrict__ orow = ATOMIC ? nullptr : out + (size_t)vec * p;
   const uint64_t per_blk = (uint64_t)WAVES * NT * 16;
   const uint64_t n_blk = (p + per_blk - 1) / per_blk;
   if ((uint64_t)blockIdx.x >= n_blk) return;
@@ -306,17 +345,36 @@ __global__ __launch_bounds__(64 * WAVES) void k_scan_mfma(const uint32_t* __rest
       }
     }
     if (++cw == steps) {
-      // lane holds C[4 * grp + r][col] of this block; rows past p land in
-      // the accumulator's padding, columns past NC in slots the combine
-      // never reads: the stores need no guard
+      // lane holds C[4 * grp + r][col] of this block
       const uint64_t base = (cb * WAVES + wave) * (NT * 16);
 #pragma unroll
       for (int t = 0; t < NT; ++t) {
+        if (ATOMIC) {
+          // rows past p land in the accumulator's padding, columns past NC
+          // in slots the combine never reads: the adds need no guard
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          int32_t* dst = acc + (base + t * 16 + 4 * grp + r) * 16 + col;
-          if (ATOMIC) atomicAdd(dst, c[t][r]);
-          else *dst = c[t][r];
+          for (int r = 0; r < 4; ++r) atomicAdd(acc + (base + t * 16 + 4 * grp + r) * 16 + col, c[t][r]);
+        } else {
+          // sum_d 256^d C_d: after D - 1 rounds of "mine plus 256 times the
+          // next lane's" the lane of a vector's digit 0 holds it whole; the
+          // lane of a vector stores four SNPs' results
+          double o[4];
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            const long long own = c[t][r];
+            long long x = own;
+            for (int k = 1; k < digits; ++k) {
+              const uint32_t lo = (uint32_t)dpp_i32<0x101, 0xf>((int)(uint32_t)x);          // row_shl:1
+              const uint32_t hi = (uint32_t)dpp_i32<0x101, 0xf>((int)(uint32_t)(x >> 32));
+              x = own + (long long)(((uint64_t)hi << 32 | lo) << 8);
+            }
+            o[r] = (double)x * sc;
+          }
+          const uint64_t j = base + t * 16 + 4 * grp;
+          if (stores) {
+#pragma unroll
+            for (int r = 0; r < 4; ++r) if (j + r < p) orow[j + r] = o[r];
+          }
         }
         c[t] = v4i{0, 0, 0, 0};
       }
@@ -648,26 +706,37 @@ static int scan_check(int nvec, int digits) {
   return BMG_OK;
 }
 
-static int scan_digits(bmg_ctx* c, const double* r_dev, int nvec, int digits, const ScanBufs& B,
-                       hipStream_t s) {
-  hipLaunchKernelGGL(k_absmax, dim3(nvec), dim3(256), 0, s, r_dev, c->n_pad, nvec, B.scale, digits);
-  hipLaunchKernelGGL(k_digits, dim3((c->n_pad + 255) / 256, nvec), dim3(256), 0, s, r_dev,
-                     c->n_pad, nvec, digits, B.scale, B.dig);
+// where the vectors come from: device rows of n_pad doubles, or y - y_hat of
+// the chains in `list` (whose sums go to rsum)
+struct ScanSource {
+  const double* r;
+  const ChainArrays* arrays;
+  const int* list;
+  double* rsum;
+};
+
+static int scan_digits(bmg_ctx* c, const ScanSource& src, int nvec, int digits, const ScanBufs& B, hipStream_t s) {
+  if (src.arrays)
+    hipLaunchKernelGGL(k_scan_prepare<true>, dim3(PREP_WGS, nvec), dim3(PREP_LANES), 0, s, (const double*)c->y, c->n,
+                       c->n_pad, src.arrays, src.list, digits, B.scale, src.rsum, B.dig);
+  else
+    hipLaunchKernelGGL(k_scan_prepare<false>, dim3(PREP_WGS, nvec), dim3(PREP_LANES), 0, s, src.r, c->n, c->n_pad,
+                       src.arrays, src.list, digits, B.scale, src.rsum, B.dig);
   BMG_HIP(hipGetLastError());
   return BMG_OK;
 }
 
-static int scan_prepare(bmg_ctx* c, const double* r_dev, int nvec, int digits, hipStream_t s, ScanBufs* B) {
+static int scan_prepare(bmg_ctx* c, const ScanSource& src, int nvec, int digits, hipStream_t s, ScanBufs* B) {
   int rc = scan_check(nvec, digits);
   if (rc) return rc;
   int NC = nvec * digits;
   if (ensure((void**)&c->dig, &c->dig_bytes, (size_t)NC * c->n_pad)) return BMG_E_HIP;
   // p rows plus one block of the largest scan shape (16 waves x 4 tiles x 16
-  // SNPs) for the unguarded stores of the last block
+  // SNPs) for the unguarded adds of the last block
   if (ensure((void**)&c->acc, &c->acc_bytes, (size_t)(c->p + 1024) * 16 * sizeof(int32_t))) return BMG_E_HIP;
   if (!c->scale) BMG_HIP(hipMalloc(&c->scale, sizeof(double) * 16));
   *B = ScanBufs{c->dig, c->acc, c->scale};
-  return scan_digits(c, r_dev, nvec, digits, *B, s);
+  return scan_digits(c, src, nvec, digits, *B, s);
 }
 
 struct ScanShape {
@@ -707,47 +776,56 @@ static void scan_clear(bmg_ctx* c, const ScanShape& sh, const ScanBufs& B, hipSt
 }
 
 template <int NT, int CODING, bool ATOMIC>
-static void scan_mfma_w(bmg_ctx* c, int NC, const ScanShape& sh, const ScanBufs& B, hipStream_t s) {
+static void scan_mfma_w(bmg_ctx* c, int NC, int digits, const ScanShape& sh, const ScanBufs& B, double* out,
+                        hipStream_t s) {
   dim3 grid(sh.gx, sh.n_tiles);
   switch (sh.waves) {
     case 16:
       hipLaunchKernelGGL((k_scan_mfma<NT, CODING, 16, ATOMIC>), grid, dim3(1024), sh.lds, s, c->g, c->p, c->W32,
-                         B.dig, NC, c->n_pad, sh.tile_words, B.acc);
+                         B.dig, NC, c->n_pad, sh.tile_words, B.acc, digits, B.scale, out);
       break;
     case 8:
       hipLaunchKernelGGL((k_scan_mfma<NT, CODING, 8, ATOMIC>), grid, dim3(512), sh.lds, s, c->g, c->p, c->W32,
-                         B.dig, NC, c->n_pad, sh.tile_words, B.acc);
+                         B.dig, NC, c->n_pad, sh.tile_words, B.acc, digits, B.scale, out);
       break;
     default:
       hipLaunchKernelGGL((k_scan_mfma<NT, CODING, 4, ATOMIC>), grid, dim3(256), sh.lds, s, c->g, c->p, c->W32,
-                         B.dig, NC, c->n_pad, sh.tile_words, B.acc);
+                         B.dig, NC, c->n_pad, sh.tile_words, B.acc, digits, B.scale, out);
   }
 }
 
 template <int CODING>
-static void scan_mfma_c(bmg_ctx* c, int NC, const ScanShape& sh, const ScanBufs& B, hipStream_t s) {
+static void scan_mfma_c(bmg_ctx* c, int NC, int digits, const ScanShape& sh, const ScanBufs& B, double* out,
+                        hipStream_t s) {
   if (sh.atomic) {
-    if (sh.nt == 4) scan_mfma_w<4, CODING, true>(c, NC, sh, B, s);
-    else scan_mfma_w<2, CODING, true>(c, NC, sh, B, s);
+    if (sh.nt == 4) scan_mfma_w<4, CODING, true>(c, NC, digits, sh, B, out, s);
+    else scan_mfma_w<2, CODING, true>(c, NC, digits, sh, B, out, s);
   } else {
-    if (sh.nt == 4) scan_mfma_w<4, CODING, false>(c, NC, sh, B, s);
-    else scan_mfma_w<2, CODING, false>(c, NC, sh, B, s);
+    if (sh.nt == 4) scan_mfma_w<4, CODING, false>(c, NC, digits, sh, B, out, s);
+    else scan_mfma_w<2, CODING, false>(c, NC, digits, sh, B, out, s);
   }
 }
 
-static void scan_mfma(bmg_ctx* c, int NC, int coding, const ScanShape& sh, const ScanBufs& B, hipStream_t s) {
+static void scan_mfma(bmg_ctx* c, int NC, int coding, int digits, const ScanShape& sh, const ScanBufs& B, double* out,
+                      hipStream_t s) {
   switch (coding) {
-    case 0: scan_mfma_c<0>(c, NC, sh, B, s); break;
-    case 1: scan_mfma_c<1>(c, NC, sh, B, s); break;
-    case 2: scan_mfma_c<2>(c, NC, sh, B, s); break;
-    default: scan_mfma_c<3>(c, NC, sh, B, s); break;
+    case 0: scan_mfma_c<0>(c, NC, digits, sh, B, out, s); break;
+    case 1: scan_mfma_c<1>(c, NC, digits, sh, B, out, s); break;
+    case 2: scan_mfma_c<2>(c, NC, digits, sh, B, out, s); break;
+    default: scan_mfma_c<3>(c, NC, digits, sh, B, out, s); break;
   }
 }
 
+// X^T R of the prepared digits into out.  A shape whose workgroups hold all
+// individuals writes the results itself; several individual tiles add into
+// the accumulator, which a second kernel turns into results.
 static int scan_kernel(bmg_ctx* c, int nvec, int coding, int digits, const ScanShape& sh, const ScanBufs& B,
-                       hipStream_t s) {
+                       double* out, hipStream_t s) {
   scan_clear(c, sh, B, s);
-  scan_mfma(c, nvec * digits, coding, sh, B, s);
+  scan_mfma(c, nvec * digits, coding, digits, sh, B, out, s);
+  if (sh.atomic)
+    hipLaunchKernelGGL(k_scan_combine, dim3((unsigned)((c->p + 255) / 256), nvec), dim3(256), 0, s, B.acc, c->p, nvec,
+                       digits, B.scale, out);
   BMG_HIP(hipGetLastError());
   return BMG_OK;
 }
@@ -755,10 +833,10 @@ static int scan_kernel(bmg_ctx* c, int nvec, int coding, int digits, const ScanS
 // Autotuner: the first scan of a context with NC digit columns times every
 // candidate shape (SNP tiles per wave, LDS tile width, grid size) on the
 // prepared digits -- HIP events on the scan's stream, best of two launches,
-// the accumulator clear included -- and keeps the fastest for the context's
+// the accumulator's clear and combine included -- and keeps the fastest for the context's
 // lifetime.  A candidate the runtime refuses to launch is skipped.
-static int scan_tuned_shape(bmg_ctx* c, int nvec, int coding, int digits, const ScanBufs& B, hipStream_t s,
-                            ScanShape* out) {
+static int scan_tuned_shape(bmg_ctx* c, int nvec, int coding, int digits, const ScanBufs& B, double* out_dev,
+                            hipStream_t s, ScanShape* out) {
   const int NC = nvec * digits;
   if (c->scan_tw[NC]) {
     *out = make_shape(c, NC, c->scan_nt[NC], c->scan_wv[NC], c->scan_tw[NC], c->scan_gx[NC]);
@@ -793,9 +871,7 @@ static int scan_tuned_shape(bmg_ctx* c, int nvec, int coding, int digits, const 
     bool ok = true;
     for (int r = 0; r < 2 && ok; ++r) {
       (void)hipEventRecord(e0, s);
-      scan_clear(c, cand[i], B, s);
-      scan_mfma(c, NC, coding, cand[i], B, s);
-      if (hipGetLastError() != hipSuccess) { ok = false; break; }
+      if (scan_kernel(c, nvec, coding, digits, cand[i], B, out_dev, s)) { ok = false; break; }
       (void)hipEventRecord(e1, s);
       if (hipEventSynchronize(e1) != hipSuccess) { ok = false; break; }
       float t = 0;
@@ -818,29 +894,34 @@ static int scan_tuned_shape(bmg_ctx* c, int nvec, int coding, int digits, const 
   return BMG_OK;
 }
 
-int launch_scan(bmg_ctx* c, const double* r_dev, int nvec, int coding, int digits,
-                double* out_dev, hipStream_t s) {
+static int scan_run(bmg_ctx* c, const ScanSource& src, int nvec, int coding, int digits, double* out_dev,
+                    hipStream_t s) {
   ScanBufs B;
-  int rc = scan_prepare(c, r_dev, nvec, digits, s, &B);
+  int rc = scan_prepare(c, src, nvec, digits, s, &B);
   if (rc) return rc;
   ScanShape sh;
-  rc = scan_tuned_shape(c, nvec, coding, digits, B, s, &sh);
+  rc = scan_tuned_shape(c, nvec, coding, digits, B, out_dev, s, &sh);
   if (rc) return rc;
-  rc = scan_kernel(c, nvec, coding, digits, sh, B, s);
-  if (rc) return rc;
-  hipLaunchKernelGGL(k_scan_combine, dim3((unsigned)((c->p + 255) / 256), nvec), dim3(256), 0, s,
-                     B.acc, c->p, nvec, digits, B.scale, out_dev);
-  BMG_HIP(hipGetLastError());
-  return BMG_OK;
+  return scan_kernel(c, nvec, coding, digits, sh, B, out_dev, s);
+}
+
+int launch_scan(bmg_ctx* c, const double* r_dev, int nvec, int coding, int digits,
+                double* out_dev, hipStream_t s) {
+  return scan_run(c, ScanSource{r_dev, nullptr, nullptr, nullptr}, nvec, coding, digits, out_dev, s);
+}
+
+int launch_scan_chains(bmg_ctx* c, const ChainArrays* arrays, const int* list, int nvec, int coding, int digits,
+                       double* rsum, double* out_dev, hipStream_t s) {
+  return scan_run(c, ScanSource{nullptr, arrays, list, rsum}, nvec, coding, digits, out_dev, s);
 }
 
 int launch_scan_timed(bmg_ctx* c, const double* r_dev, int nvec, int coding, int digits,
                       double* out_dev, int reps, double* ms, hipStream_t s) {
   ScanBufs B;
-  int rc = scan_prepare(c, r_dev, nvec, digits, s, &B);
+  int rc = scan_prepare(c, ScanSource{r_dev, nullptr, nullptr, nullptr}, nvec, digits, s, &B);
   if (rc) return rc;
   ScanShape sh;
-  rc = scan_tuned_shape(c, nvec, coding, digits, B, s, &sh);
+  rc = scan_tuned_shape(c, nvec, coding, digits, B, out_dev, s, &sh);
   if (rc) return rc;
   hipEvent_t e0, e1;
   BMG_HIP(hipEventCreate(&e0));
@@ -851,7 +932,7 @@ int launch_scan_timed(bmg_ctx* c, const double* r_dev, int nvec, int coding, int
   for (int r = 0; r < reps && !rc; ++r) {
     scan_clear(c, sh, B, s);
     BMG_HIP(hipEventRecord(e0, s));
-    scan_mfma(c, nvec * digits, coding, sh, B, s);
+    scan_mfma(c, nvec * digits, coding, digits, sh, B, out_dev, s);
     BMG_HIP(hipGetLastError());
     BMG_HIP(hipEventRecord(e1, s));
     BMG_HIP(hipEventSynchronize(e1));
@@ -861,8 +942,9 @@ int launch_scan_timed(bmg_ctx* c, const double* r_dev, int nvec, int coding, int
   }
   hipEventDestroy(e0); hipEventDestroy(e1);
   *ms = total / (reps > 0 ? reps : 1);
-  hipLaunchKernelGGL(k_scan_combine, dim3((unsigned)((c->p + 255) / 256), nvec), dim3(256), 0, s,
-                     B.acc, c->p, nvec, digits, B.scale, out_dev);
+  if (sh.atomic)
+    hipLaunchKernelGGL(k_scan_combine, dim3((unsigned)((c->p + 255) / 256), nvec), dim3(256), 0, s,
+                       B.acc, c->p, nvec, digits, B.scale, out_dev);
   BMG_HIP(hipGetLastError());
   return BMG_OK;
 }
@@ -915,19 +997,14 @@ int launch_scan_noalloc(bmg_ctx* c, const double* r_dev, int nvec, int coding, i
   uint8_t* b8 = (uint8_t*)base;
   ScanBufs B{(int8_t*)(b8 + SCAN_SCRATCH_ACC_ROWS * 16 * 4), (int32_t*)b8,
              (double*)(b8 + SCAN_SCRATCH_ACC_ROWS * 16 * 4 + SCAN_SCRATCH_DIG)};
-  rc = scan_digits(c, r_dev, nvec, digits, B, s);
+  rc = scan_digits(c, ScanSource{r_dev, nullptr, nullptr, nullptr}, nvec, digits, B, s);
   if (rc) return rc;
   // the shape the tuner picked for this width if it ran, else the fixed one
   // (no timing here: tuning creates events)
   const int NC = nvec * digits;
   ScanShape sh = c->scan_tw[NC] ? make_shape(c, NC, c->scan_nt[NC], c->scan_wv[NC], c->scan_tw[NC], c->scan_gx[NC])
                                 : make_shape(c, NC, 2, 8, tile_for(NC, 163840), 256);
-  rc = scan_kernel(c, nvec, coding, digits, sh, B, s);
-  if (rc) return rc;
-  hipLaunchKernelGGL(k_scan_combine, dim3((unsigned)((c->p + 255) / 256), nvec), dim3(256), 0, s,
-                     B.acc, c->p, nvec, digits, B.scale, out_dev);
-  BMG_HIP(hipGetLastError());
-  return BMG_OK;
+  return scan_kernel(c, nvec, coding, digits, sh, B, out_dev, s);
 }
 
 // plain 16-byte copy: the reference kernel of known traffic against which

@@ -46,6 +46,7 @@ struct bmg_ctx {
 };
 
 namespace bmg {
+struct ChainArrays;
 void set_error(const std::string& msg);
 int hip_fail(hipError_t e, const char* what);
 
@@ -60,6 +61,9 @@ int launch_synth(bmg_ctx* c, uint32_t seed, const double* thresh_dev, const doub
                  const uint64_t* blk_start_dev, uint64_t n_blocks, hipStream_t s);
 int launch_scan(bmg_ctx* c, const double* r_dev, int nvec, int coding, int digits,
                 double* out_dev, hipStream_t s);
+// the scan of y - y_hat of the chains in `list` (their sums to rsum)
+int launch_scan_chains(bmg_ctx* c, const ChainArrays* arrays, const int* list, int nvec, int coding, int digits,
+                       double* rsum, double* out_dev, hipStream_t s);
 // the same scan with its scratch in a file-scope device array (no allocation)
 int launch_scan_noalloc(bmg_ctx* c, const double* r_dev, int nvec, int coding, int digits,
                         double* out_dev, hipStream_t s);

@@ -5,8 +5,6 @@
 #include "bmg_chain.h"
 
 namespace bmg {
-int launch_residuals(const double* y, uint32_t n, uint32_t n_pad, const ChainArrays* arrays,
-                     const int* list, int nv, double* r, double* rsum, hipStream_t s);
 int launch_rb_finalize(const DevData* data, const ChainConst* consts, const ChainScal* scal,
                        const ChainArrays* arrays, const int* list, int nv, int kmax, uint64_t p,
                        const double* xa, const double* xh, const double* rsum, hipStream_t s);

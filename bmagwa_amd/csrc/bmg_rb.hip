@@ -12,26 +12,6 @@
 
 using namespace bmg;
 
-// r_v = y - y_hat of chain list[v] (zero past n); sums of r per vector
-// r = y - y_hat for chain list[v], and rsum[v] = sum of r: one workgroup per
-// vector, so the sum is reduced in a fixed order (the RB PIPs do not depend
-// on the order in which workgroups finish)
-__global__ void k_residuals(const double* __restrict__ y, uint32_t n, uint32_t n_pad,
-                            const ChainArrays* __restrict__ arrays, const int* __restrict__ list,
-                            double* __restrict__ r, double* __restrict__ rsum) {
-  __shared__ double red[8];
-  int v = blockIdx.y;
-  const double* yh = arrays[list[v]].y_hat;
-  double s = 0.0;
-  for (uint32_t i = threadIdx.x; i < n_pad; i += blockDim.x) {
-    double ri = i < n ? y[i] - yh[i] : 0.0;
-    r[(size_t)v * n_pad + i] = ri;
-    s += ri;
-  }
-  s = block_sum(s, red);
-  if (threadIdx.x == 0) rsum[v] = s;
-}
-
 __device__ inline double rb_prior_add(const ChainConst& K, double Ns_t, double n_old) {
   return (log(K.g_a + n_old) - log(K.g_b + K.m_g - n_old - 1)) +
          (log(K.tp_type + Ns_t) - log(K.tp_sum + n_old));
@@ -211,12 +191,6 @@ __global__ void k_tree_total(const DevData* __restrict__ data, const ChainConst*
 }
 
 namespace bmg {
-
-int launch_residuals(const double* y, uint32_t n, uint32_t n_pad, const ChainArrays* arrays,
-                     const int* list, int nv, double* r, double* rsum, hipStream_t s) {
-  hipLaunchKernelGGL(k_residuals, dim3(1, nv), dim3(256), 0, s, y, n, n_pad, arrays, list, r, rsum);
-  return hipGetLastError() == hipSuccess ? 0 : -1;
-}
 
 int launch_rb_finalize(const DevData* data, const ChainConst* consts, const ChainScal* scal,
                        const ChainArrays* arrays, const int* list, int nv, int kmax, uint64_t p,
