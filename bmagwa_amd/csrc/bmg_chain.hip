@@ -172,6 +172,8 @@ struct Reg {
   int err;
   int learn_on;
   int tj_on, tj_n;                       // journal active, entries
+  long long warm;                        // SNP a pick has drawn (or -1): see warm_next
+  int warm_add;                          // ... for addition
   long long pre_snp;                     // SNP whose dots are in iacc2 (or -1)
   int pre_slot;                          // and the slot its value words went to
   double tj_tot[2];                      // tree totals when the move began
@@ -316,22 +318,44 @@ __device__ __forceinline__ void column_dots_np(Ctx<KMAX>& C, uint64_t snp_new, i
   for (uint32_t p0 = 0; p0 < W4; p0 += SPAN * NP) {
     uint32_t ne[NP][4], no[NP][4];            // even / odd fields of the new column
     uint32_t off[NP];                         // byte offset of this lane's pieces in a column
-    uint32_t s_one = 0, s_self = 0;
+    uint4 raw[NP];
 #pragma unroll
     for (int q = 0; q < NP; ++q) {
       const uint32_t pc = p0 + t + q * SPAN;
       off[q] = (pc < W4 ? pc : W4 - 1) * 16;
-      const uint4 v = wn[off[q] / 16];
-      const uint32_t xs[4] = {v.x, v.y, v.z, v.w};
+      raw[q] = wn[off[q] / 16];
+    }
+    // group g sums columns me + g + GRP k; every group runs group 0's rounds
+    const int n_col = cols - me;
+    const int rounds = n_col > 0 ? ((n_col + GRP - 1) / GRP + UC - 1) / UC : 0;
+    auto column = [&](int r, int u) { return me + grp + (UC * r + u) * GRP; };
+    auto load = [&](int r, uint4 (&w)[UC][NP]) {
+#pragma unroll
+      for (int u = 0; u < UC; ++u) {
+        const int c = column(r, u);
+        const uint32_t base = (uint32_t)S.slot[c < cols ? c : cols - 1] * W * 4;
+#pragma unroll
+        for (int q = 0; q < NP; ++q) w[u][q] = *(const uint4*)(xcol + (base + off[q]));
+      }
+    };
+    // the first columns are on their way while the new one arrives (from
+    // HBM, where the model's columns are in L2)
+    uint4 wa[UC][NP], wb[UC][NP];
+    if (rounds > 0) load(0, wa);
+    uint32_t s_one = 0, s_self = 0;
+#pragma unroll
+    for (int q = 0; q < NP; ++q) {
+      const bool in = p0 + t + q * SPAN < W4;
+      const uint32_t xs[4] = {raw[q].x, raw[q].y, raw[q].z, raw[q].w};
       uint32_t vw[4];
 #pragma unroll
       for (int u = 0; u < 4; ++u) {
-        vw[u] = pc < W4 ? value_word(xs[u], coding) : 0u;
+        vw[u] = in ? value_word(xs[u], coding) : 0u;
         ne[q][u] = vw[u] & 0x33333333u;
         no[q][u] = (vw[u] >> 2) & 0x33333333u;
       }
       if (grp == 0) {
-        if (pc < W4) *(uint4*)((char*)xnew + off[q]) = make_uint4(vw[0], vw[1], vw[2], vw[3]);
+        if (in) *(uint4*)((char*)xnew + off[q]) = make_uint4(vw[0], vw[1], vw[2], vw[3]);
 #pragma unroll
         for (int u = 0; u < 4; ++u) {
           s_one = __builtin_amdgcn_udot8(0x11111111u, ne[q][u], s_one, false);
@@ -348,19 +372,6 @@ __device__ __forceinline__ void column_dots_np(Ctx<KMAX>& C, uint64_t snp_new, i
       const int a = group_sum((int)s_one), b = group_sum((int)s_self);
       if (grp == 0) { put_sum(0, a); put_sum(cols, b); }
     }
-    // group g sums columns me + g + GRP k; every group runs group 0's rounds
-    const int n_col = cols - me;
-    const int rounds = n_col > 0 ? ((n_col + GRP - 1) / GRP + UC - 1) / UC : 0;
-    auto column = [&](int r, int u) { return me + grp + (UC * r + u) * GRP; };
-    auto load = [&](int r, uint4 (&w)[UC][NP]) {
-#pragma unroll
-      for (int u = 0; u < UC; ++u) {
-        const int c = column(r, u);
-        const uint32_t base = (uint32_t)S.slot[c < cols ? c : cols - 1] * W * 4;
-#pragma unroll
-        for (int q = 0; q < NP; ++q) w[u][q] = *(const uint4*)(xcol + (base + off[q]));
-      }
-    };
     auto sum = [&](int r, const uint4 (&w)[UC][NP]) {
       int v[UC];
 #pragma unroll
@@ -386,8 +397,6 @@ __device__ __forceinline__ void column_dots_np(Ctx<KMAX>& C, uint64_t snp_new, i
         if (c < cols) put_sum(c, v[u]);
       }
     };
-    uint4 wa[UC][NP], wb[UC][NP];
-    if (rounds > 0) load(0, wa);
     for (int r = 0; r < rounds; r += 2) {
       if (r + 1 < rounds) load(r + 1, wb);
       sum(r, wa);
@@ -410,6 +419,7 @@ __device__ __forceinline__ void column_dots(Ctx<KMAX>& C, uint64_t snp_new, int 
   if (W4 <= 16) column_dots_np<KMAX, T0, NTH, 16, 1>(C, snp_new, coding, cols, xnew, acc);
   else if (W4 <= 32) column_dots_np<KMAX, T0, NTH, 32, 1>(C, snp_new, coding, cols, xnew, acc);
   else if (W4 <= 64) column_dots_np<KMAX, T0, NTH, 64, 1>(C, snp_new, coding, cols, xnew, acc);
+  else if (W4 <= 128) column_dots_np<KMAX, T0, NTH, 64, 2>(C, snp_new, coding, cols, xnew, acc);
   else if (W4 <= 192) column_dots_np<KMAX, T0, NTH, 64, 3>(C, snp_new, coding, cols, xnew, acc);
   else column_dots_np<KMAX, T0, NTH, 64, 5>(C, snp_new, coding, cols, xnew, acc);
 }
@@ -742,10 +752,11 @@ __device__ __forceinline__ void downdate_w0(Smem<KMAX>& S, double* L, int m, int
 // The downdate on wave 0, while wave 1 moves the rows above cr of the later
 // columns down by one column, in ascending order of destination (every source
 // lies above every earlier destination, so a batch never overwrites what a
-// later one reads; the two waves touch disjoint entries), and waves 1-3 do
-// the extra work, which touches neither the factor nor v.
+// later one reads; the two waves touch disjoint entries).  With work to do
+// ahead, which touches neither the factor nor v and lasts longer than the
+// downdate, waves 1-3 do that and wave 0 moves the rows afterwards.
 template <int KMAX, typename Extra>
-__device__ __forceinline__ void chol_downdate(Smem<KMAX>& S, int m, int cr, Extra extra) {
+__device__ __forceinline__ void chol_downdate(Smem<KMAX>& S, int m, int cr, bool ahead, Extra extra) {
   double* L = S.L;
   if (wave_id() == 0) {
     const int n = m - 1 - cr;
@@ -753,33 +764,32 @@ __device__ __forceinline__ void chol_downdate(Smem<KMAX>& S, int m, int cr, Extr
     else if (KMAX <= 128 || n <= 128) downdate_w0<KMAX, 2>(S, L, m, cr);
     else if (KMAX <= 192 || n <= 192) downdate_w0<KMAX, 3>(S, L, m, cr);
     else downdate_w0<KMAX, 4>(S, L, m, cr);
-  } else {
-    if (wave_id() == 1) {
-      // rows [0, cr) of logical columns [cr, m - 2]: physical column jl + 1
-      // -> jl, element k = (jl - cr) * cr + i in ascending order
-      constexpr int DEEP = KMAX <= KMAX_LDS ? 4 : 16;
-      const int total = (m - 1 - cr) * cr;
-      const float rcr = cr > 0 ? 1.0f / (float)cr : 0.0f;
-      for (int k0 = 0; k0 < total; k0 += 64 * DEEP) {
-        double x[DEEP];
-        int to[DEEP];
-#pragma unroll
-        for (int u = 0; u < DEEP; ++u) {
-          const int k = k0 + 64 * u + lane_id();
-          int q = (int)((float)k * rcr);
-          if (q * cr > k) --q;
-          if ((q + 1) * cr <= k) ++q;
-          const int jl = cr + q, i = k - q * cr;
-          to[u] = P(jl) + i;
-          x[u] = k < total ? L[P(jl + 1) + i] : 0.0;
-        }
-#pragma unroll
-        for (int u = 0; u < DEEP; ++u)
-          if (k0 + 64 * u + lane_id() < total) L[to[u]] = x[u];
-      }
-    }
-    extra();
   }
+  if (wave_id() == (ahead ? 0 : 1)) {
+    // rows [0, cr) of logical columns [cr, m - 2]: physical column jl + 1
+    // -> jl, element k = (jl - cr) * cr + i in ascending order
+    constexpr int DEEP = KMAX <= KMAX_LDS ? 4 : 16;
+    const int total = (m - 1 - cr) * cr;
+    const float rcr = cr > 0 ? 1.0f / (float)cr : 0.0f;
+    for (int k0 = 0; k0 < total; k0 += 64 * DEEP) {
+      double x[DEEP];
+      int to[DEEP];
+#pragma unroll
+      for (int u = 0; u < DEEP; ++u) {
+        const int k = k0 + 64 * u + lane_id();
+        int q = (int)((float)k * rcr);
+        if (q * cr > k) --q;
+        if ((q + 1) * cr <= k) ++q;
+        const int jl = cr + q, i = k - q * cr;
+        to[u] = P(jl) + i;
+        x[u] = k < total ? L[P(jl + 1) + i] : 0.0;
+      }
+#pragma unroll
+      for (int u = 0; u < DEEP; ++u)
+        if (k0 + 64 * u + lane_id() < total) L[to[u]] = x[u];
+    }
+  }
+  if (ahead && wave_id() != 0) extra();
   __syncthreads();
 }
 
@@ -970,6 +980,33 @@ __device__ __forceinline__ double group_total(double v) {
   return readlane_d(v, 0) + readlane_d(v, 32);
 }
 
+// While wave 0 walks a tree for the next pick, wave 1 reads what the SNP of
+// the pick before will need (its genotypes if it is to be added, its entries
+// in the other tree, its weight there and its x.y), so that HBM's latency, and
+// the address translation's, is not waited for when the move is applied.
+// The values are dropped: the reads bring the lines into L2.
+template <int KMAX>
+__device__ __forceinline__ void warm_next(Ctx<KMAX>& C) {
+  if (C.R.warm < 0) return;
+  if (wave_id() == 1) {
+    const int lane = lane_id();
+    const uint64_t j = (uint64_t)C.R.warm;
+    const double* other = C.R.warm_add ? gp(C.A.tree_rem) : gp(C.A.tree_add);
+    const double* w = C.R.warm_add ? gp(C.A.q_rem) : gp(C.A.q_add);
+    double x = other[C.D.lev_off[0] + 64 * (j >> 6) + lane] + w[j];
+    if (C.D.top >= 1) x += other[C.D.lev_off[1] + 64 * (j >> 12) + lane];
+    uint32_t g = 0;
+    if (C.R.warm_add) {
+      const double* xy = gp(C.D.xy[C.D.type == BMG_AH ? 0 : C.D.type]);
+      if (xy) x += xy[j];
+      const uint4* row = (const uint4*)(gp(C.D.g) + j * C.D.W32);
+      for (uint32_t q = lane; q < C.D.W32 / 4; q += 64) g ^= row[q].x;
+    }
+    asm volatile("" : : "v"(x), "v"(g));
+  }
+  C.R.warm = -1;
+}
+
 // draw an index with probability w_i / total (wave 0 computes, all return)
 template <int KMAX>
 __device__ __forceinline__ uint64_t tree_pick(Ctx<KMAX>& C, int tr, double u) {
@@ -1006,6 +1043,7 @@ __device__ __forceinline__ void tree_set(Ctx<KMAX>& C, int tr, uint64_t i, int z
   double* g0 = tr == 0 ? gp(C.A.tree_add) : gp(C.A.tree_rem);
   const double* w = tr == 0 ? gp(C.A.q_add) : gp(C.A.q_rem);
   double total;
+  warm_next(C);
   if (wave_id() == 0) {
     const int lane = lane_id();
     double nv = zero ? 0.0 : w[i];
@@ -1057,6 +1095,7 @@ __device__ __forceinline__ void tree_set(Ctx<KMAX>& C, int tr, uint64_t i, int z
 template <int KMAX>
 __device__ __forceinline__ uint64_t tree_pick_zero(Ctx<KMAX>& C, int tr, double u, double* w_out) {
   double* g0 = tr == 0 ? gp(C.A.tree_add) : gp(C.A.tree_rem);
+  warm_next(C);
   if (wave_id() == 0) {
     const int lane = lane_id();
     double total = tr == 0 ? C.R.tot_add : C.R.tot_rem;
@@ -1410,13 +1449,12 @@ __device__ __forceinline__ void update_on_remove_impl(Ctx<KMAX>& C, int x_ind, l
     if (next >= 0 && !C.D.mixed && C.D.type != BMG_AH && C.D.me <= 1 && R.cols < KMAX)
       nslot = alloc_slot(C);
     auto ahead = [&]() {
-      if (nslot >= 0)
-        column_dots<KMAX, 64, BMG_BLOCK - 64>(C, (uint64_t)next, C.D.type, R.cols,
-                                              gp(C.A.xcol) + (size_t)nslot * C.D.W32, S.iacc2);
+      column_dots<KMAX, 64, BMG_BLOCK - 64>(C, (uint64_t)next, C.D.type, R.cols,
+                                            gp(C.A.xcol) + (size_t)nslot * C.D.W32, S.iacc2);
     };
     const uint64_t ta = wall_clock64();
     // v follows the downdate's rotations (no re-solve)
-    chol_downdate(S, k, x_ind, ahead);
+    chol_downdate(S, k, x_ind, nslot >= 0, ahead);
     if (nslot >= 0) { R.pre_snp = next; R.pre_slot = nslot; }
     const uint64_t tb = wall_clock64();
     if (threadIdx.x == 0) { C.prof[16] += tb - ta; C.prof[17] += wall_clock64() - tb; }
@@ -2541,6 +2579,7 @@ __device__ __forceinline__ int move_addrem(Ctx<KMAX>& C) {
       ind = tree_pick_zero(C, 1, u, &wv);   // wv = q_rem[ind]
       lqf += log(wv) - log(tot);
     }
+    R.warm = (long long)ind; R.warm_add = add;
     if (threadIdx.x == 0) {
       S.mi_isadd[i] = (uint8_t)add; S.mi[i] = ind; S.mi_map[i] = add ? (int64_t)ind : -1;
     }
@@ -3022,6 +3061,7 @@ __device__ __forceinline__ void load_chain(Ctx<KMAX>& C, const ChainScal& CS) {
   R.learn_on = CS.learn_on && C.D.lw != nullptr && C.D.lH >= 1 && C.D.lH <= BMG_LH_MAX;
   R.tj_on = 0; R.tj_n = 0; R.tj_tot[0] = R.tj_tot[1] = 0.0;
   R.pre_snp = -1; R.pre_slot = -1;
+  R.warm = -1; R.warm_add = 0;
   const double* vec = gp(C.A.vec);
   const int32_t* idx = gp(C.A.idx);
   copy_factor(S.L, gp(C.A.Lcur), 0, P(R.cols));
