@@ -21,7 +21,6 @@ using namespace bmg;
 // kernels of bmg_chain.hip and bmg_data.hip
 __global__ void k_chains(KernelArgs);
 __global__ void k_model_op(ModelOpArgs);
-__global__ void k_restride(const uint8_t*, uint64_t, uint32_t, uint32_t, uint8_t*);
 
 static thread_local std::string g_err;
 
@@ -124,17 +123,15 @@ extern "C" int bmg_ctx_create(int device, const uint8_t* bed_body, uint32_t n, u
   // upload in the reference layout, then re-stride on the device
   uint32_t stride_raw = (n + 3) / 4;
   uint8_t* raw = nullptr;
-  hipError_t e = hipMalloc(&raw, (size_t)stride_raw * p);
+  hipError_t e = hipMalloc(&raw, (size_t)stride_raw * p + RAW_PAD);
   if (e != hipSuccess) { bmg_ctx_destroy(c); *out = nullptr; return hip_fail(e, "hipMalloc(raw)"); }
   e = hipMemcpy(raw, bed_body, (size_t)stride_raw * p, hipMemcpyHostToDevice);
   if (e == hipSuccess) {
-    unsigned gy = (unsigned)std::min<uint64_t>(p, 65535), gz = (unsigned)((p + gy - 1) / gy);
-    hipLaunchKernelGGL(k_restride, dim3((c->W32 * 4 + 255) / 256, gy, gz), dim3(256), 0, c->stream, raw,
-                       p, stride_raw, c->W32, (uint8_t*)c->g);
+    rc = launch_restride(raw, c, c->stream);
     e = hipStreamSynchronize(c->stream);
   }
   hipFree(raw);
-  if (e != hipSuccess) { bmg_ctx_destroy(c); *out = nullptr; return hip_fail(e, "restride"); }
+  if (rc || e != hipSuccess) { bmg_ctx_destroy(c); *out = nullptr; return rc ? rc : hip_fail(e, "restride"); }
   if ((rc = ctx_prepare(c, recode))) { bmg_ctx_destroy(c); *out = nullptr; return rc; }
   if ((rc = bmg_ctx_set_y(c, y))) { bmg_ctx_destroy(c); *out = nullptr; return rc; }
   return BMG_OK;

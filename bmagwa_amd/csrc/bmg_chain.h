@@ -168,9 +168,7 @@ struct ModelOpArgs {
 
 namespace bmg {
 
-// out[j] = x_j . y for every SNP j of D under `coding`, summed in exactly
-// the order the chain kernel's per-add dot uses, so the chain reads the
-// same double it would have computed
+// out[j] = x_j . y for every SNP j of D under `coding` (bmg_data.hip)
 int launch_xy_all(const DevData& D, int coding, double* out, hipStream_t s);
 
 }  // namespace bmg

@@ -222,10 +222,9 @@ __device__ __forceinline__ int coding_of_type(int type, int second) {
   return type == 4 ? (second ? 1 : 0) : type;
 }
 
-// x_j^T y (FP64) for one SNP/coding
-// x . y of one SNP's packed row: lane-strided words, 16 fields each in
-// order, then the workgroup sum (the order both the per-add dot and the
-// set-up table use)
+// x_j^T y (FP64) of one SNP's packed row, where no table was made at set-up
+// (the Model API): lane-strided words, 16 fields each in order, then the
+// workgroup sum
 __device__ __forceinline__ double dot_y_block(const uint32_t* __restrict__ w, uint32_t W,
                                               const double* __restrict__ y, int coding, double* red) {
   double s = 0.0;
@@ -248,20 +247,10 @@ __device__ __forceinline__ double dot_y_block(const uint32_t* __restrict__ w, ui
 #endif
 #define BMG_UNIT(u) (BMG_CHAIN_UNIT == 0 || BMG_CHAIN_UNIT == (u))
 
-#if BMG_UNIT(1)
-__global__ __launch_bounds__(BMG_BLOCK) void k_xy_all(DevData D, int coding, double* __restrict__ out) {
-  __shared__ double red[8];
-  for (uint64_t j = blockIdx.x; j < D.p; j += gridDim.x) {
-    const double v = dot_y_block(D.g + j * D.W32, D.W32, D.y, coding, red);
-    if (threadIdx.x == 0) out[j] = v;
-  }
-}
-#endif
-
 template <int KMAX>
 __device__ __forceinline__ double snp_dot_y(Ctx<KMAX>& C, uint64_t snp, int coding) {
   const double* pre = gp(C.D.xy[coding]);
-  if (pre) return pre[snp];   // precomputed at set-up in this same order
+  if (pre) return pre[snp];   // made at set-up
   return dot_y_block(gp(C.D.g) + snp * C.D.W32, C.D.W32, gp(C.D.y), coding, C.S.red);
 }
 
@@ -3491,16 +3480,4 @@ __global__ __launch_bounds__(256) void k_model_op(ModelOpArgs a) {
       for (int q = 0; q < 3; ++q) a.out->pves[q] = CS.pves[q];
   }
 }
-#endif
-
-#if BMG_UNIT(1)
-namespace bmg {
-
-int launch_xy_all(const DevData& D, int coding, double* out, hipStream_t s) {
-  const unsigned grid = (unsigned)std::min<uint64_t>(D.p, 65536);
-  hipLaunchKernelGGL(k_xy_all, dim3(grid), dim3(BMG_BLOCK), 0, s, D, coding, out);
-  return hipGetLastError() == hipSuccess ? BMG_OK : BMG_E_HIP;
-}
-
-}  // namespace bmg
 #endif

@@ -53,6 +53,9 @@ int hip_fail(hipError_t e, const char* what);
 // kernels launched from the C ABI (bmg_data.hip)
 int ctx_prepare(bmg_ctx* c, int recode);
 int ctx_self_moments(bmg_ctx* c);
+// the raw .bed body (readable RAW_PAD bytes past its end) into c's rows
+constexpr size_t RAW_PAD = 32;
+int launch_restride(const uint8_t* raw, bmg_ctx* c, hipStream_t s);
 int launch_decode(bmg_ctx* c, const uint64_t* snps_dev, uint64_t count, int coding,
                   double* out_dev, hipStream_t s);
 // genotypes of a subset of a pool dataset's individuals into c (same p)
