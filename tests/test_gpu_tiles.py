@@ -1,0 +1,121 @@
+"""Kernels at the edges of their tiles: the column dots at every group width
+and piece count (and past one pass), the sweeps and the downdate on both sides
+of 64 and 128 columns, the scan's results and digits at odd sizes, the raw
+body's rows at every alignment."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def bmg():
+    import bmagwa_amd
+    bmagwa_amd.lib()
+    return bmagwa_amd
+
+
+def genotypes(n, p, seed):
+    """p x n genotypes and their packed body."""
+    rng = np.random.default_rng(seed)
+    maf = rng.uniform(0.1, 0.5, size=(p, 1))
+    G = (rng.random((p, n)) < maf).astype(np.uint8) + (rng.random((p, n)) < maf)
+    code = np.zeros((p, (n + 3) // 4 * 4), np.uint8)
+    code[:, :n] = np.array([0, 2, 3], np.uint8)[G]
+    body = (code.reshape(p, -1, 4) << np.array([0, 2, 4, 6], np.uint8)).sum(2, dtype=np.uint8)
+    return G, body.ravel()
+
+
+CODED = {"A": [0., 1., 2.], "H": [0., 1., 0.], "D": [0., 1., 1.], "R": [0., 0., 1.]}
+
+
+# 16 / 32 / 64 lanes a column, then 2, 3 and 5 pieces a lane, then two passes
+@pytest.mark.parametrize("n", [37, 1024, 1025, 2049, 4097, 8193, 12289, 20481])
+def test_column_dots(bmg, n):
+    """X^T X of a model with terms of every coding: whole numbers, exact."""
+    types = ("A", "H", "D", "R")
+    G, body = genotypes(n, 12, n)
+    y = np.random.default_rng(n).normal(size=n)
+    ctx = bmg.Ctx(n, 12, body, y, types=types)
+    m = bmg.Model(ctx, n_plus_nu=n + 1.0, nus2_plus_yy=1.0 + float(y @ y), inv_tau2_e0=0.0)
+    X = [np.ones(n)]
+    for j in range(11):
+        m.add_term(j, j % 4, 3.0)
+        X.append(np.array(CODED[types[j % 4]])[G[j]])
+    X = np.array(X)
+    xx = m.get()["xx"]
+    assert np.array_equal(np.triu(xx), np.triu(X @ X.T))
+    m.close()
+    ctx.close()
+
+
+# columns before the removal; the removed term; n - 1 columns follow it
+@pytest.mark.parametrize("k,rm", [(2, 0), (9, 0), (9, 4), (9, 8), (64, 0), (65, 0), (66, 0), (66, 60), (129, 0),
+                                  (130, 1), (130, 70), (135, 0), (135, 127), (135, 134)])
+def test_downdate_and_sweeps(bmg, k, rm):
+    """Factor, v and log-likelihood after a removal (and an addition after
+    it) equal a fresh float64 factorisation.  Both are backward stable, so
+    entries agree to a small multiple of 2^-52 times the condition number,
+    here below 1e4: 1e-10 of the largest entry."""
+    n = 700
+    G, body = genotypes(n, k + 1, 11 * k + rm)
+    rng = np.random.default_rng(k)
+    y = rng.normal(size=n)
+    d = rng.uniform(5.0, 50.0, size=k + 1)
+    ctx = bmg.Ctx(n, k + 1, body, y)
+    n_nu, nus2_yy = n + 1.0, 1.0 + float(y @ y)
+    m = bmg.Model(ctx, n_plus_nu=n_nu, nus2_plus_yy=nus2_yy, inv_tau2_e0=0.0)
+    for j in range(k):
+        m.add_term(j, 0, d[j])
+    order = list(range(k))
+
+    def check():
+        X = np.concatenate([np.ones((1, n)), G[order].astype(float)])
+        dd = np.concatenate([[0.0], d[order]])
+        U = np.linalg.cholesky(X @ X.T + np.diag(dd)).T
+        v = np.linalg.solve(U.T, X @ y)
+        s = m.get()
+        assert np.allclose(np.triu(s["l"]), U, rtol=0, atol=1e-10 * np.abs(U).max())
+        assert np.allclose(s["v"], v, rtol=0, atol=1e-10 * np.abs(v).max())
+        ll = 0.5 * np.log(dd[1:]).sum() - np.log(np.diag(U)).sum() - 0.5 * n_nu * np.log(nus2_yy - v @ v)
+        assert abs(s["loglik"] - ll) < 1e-10 * abs(ll)
+
+    check()
+    m.remove_term(rm)
+    del order[rm]
+    check()
+    m.add_term(k, 0, d[k])
+    order.append(k)
+    check()
+    m.compute_log_likelihood()
+    check()
+    m.close()
+    ctx.close()
+
+
+@pytest.mark.parametrize("n,p,nvec,digits,coding", [(5, 1, 1, 1, 0), (63, 3, 3, 5, 0), (513, 66, 2, 6, 1),
+                                                    (1000, 131, 16, 1, 2), (2500, 1025, 3, 4, 3),
+                                                    (17000, 259, 3, 5, 0)])
+def test_scan_results_at_odd_sizes(bmg, n, p, nvec, digits, coding):
+    """Residuals of whole numbers are represented exactly, so X^T R is exact
+    (one and several individual tiles, every digit count)."""
+    G, body = genotypes(n, p, n + p)
+    rng = np.random.default_rng(p)
+    R = rng.integers(-7, 8, size=(nvec, n)).astype(float)
+    ctx = bmg.Ctx(n, p, body, np.zeros(n))
+    X = np.array(CODED["AHDR"[coding]])[G]
+    assert np.array_equal(ctx.scan_xtr(R, coding=coding, digits=digits), R @ X.T)
+    ctx.close()
+
+
+@pytest.mark.parametrize("n", [2, 5, 63, 64, 65, 66, 67, 68, 1021, 2047])
+@pytest.mark.parametrize("p", [1, 3, 8])
+def test_raw_body_rows(bmg, n, p):
+    """Rows of every byte alignment arrive whole; moments are exact."""
+    G, body = genotypes(n, p, 7 * n + p)
+    ctx = bmg.Ctx(n, p, body, np.zeros(n))
+    assert np.array_equal(ctx.read_body(), body)
+    s = G.astype(np.int64).sum(1)
+    assert np.array_equal(ctx.self_moments()[:, 0], s.astype(float))
+    assert ctx.missing_count() == 0
+    ctx.close()
