@@ -157,8 +157,44 @@ struct Smem {
   long long bci[4];
 };
 
+// The chain's stream with its next 64 blocks at hand, one in each lane of the
+// wave: a Philox block is ten rounds of dependent 32-bit multiplies, about
+// 1,000 cycles, and every lane would compute the same one for each draw.  A
+// draw is a read of its lane; the stream itself is unchanged.  (With the
+// DPP scan below a pick went from 3.6 to 3.0 us, and with the terms' draws in
+// parallel 500 iterations of 16 chains over 10,000 SNPs from 122.8 to 118.6 ms.)
+struct ChainRng : Rng {
+  uint64_t base;                         // counter of lane 0's block
+  uint32_t w[4];                         // this lane's block
+};
+struct Words { uint32_t w[4]; };
+static __device__ __noinline__ Words rng_block_at(uint32_t k0, uint32_t k1, uint64_t c, uint32_t c2, uint32_t c3) {
+  Words o;
+  o.w[0] = (uint32_t)c; o.w[1] = (uint32_t)(c >> 32); o.w[2] = c2; o.w[3] = c3;
+  philox10(o.w[0], o.w[1], o.w[2], o.w[3], k0, k1);
+  return o;
+}
+// the lane that holds the next block; the stream moves on by one
+__device__ __forceinline__ int rng_next_lane(ChainRng& r) {
+  const uint64_t c = (uint64_t)r.c1 << 32 | r.c0;
+  uint32_t at = __builtin_amdgcn_readfirstlane(c - r.base < 64 ? (uint32_t)(c - r.base) : 64u);
+  if (at >= 64) {
+    const Words o = rng_block_at(r.k0, r.k1, c + (threadIdx.x & 63), r.c2, r.c3);
+    r.base = c;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) r.w[q] = o.w[q];
+    at = 0;
+  }
+  if (++r.c0 == 0) ++r.c1;
+  return (int)at;
+}
+__device__ __forceinline__ double rng_u01(ChainRng& r) {
+  const int at = rng_next_lane(r);
+  return words_u01(__builtin_amdgcn_readlane(r.w[0], at), __builtin_amdgcn_readlane(r.w[1], at));
+}
+
 struct Reg {
-  Rng rng;
+  ChainRng rng;
   int cols, nloci, Ns[5];
   double syx, ldq, ldl, ll;
   int c_cols, c_nloci, c_Ns[5];
@@ -914,55 +950,23 @@ __device__ __forceinline__ double dpp_d(double v) {
   return *reinterpret_cast<double*>(&h);
 }
 
-// the value of the lane 16 below (lanes 16..63): rows 1 and 3 from a row
-// swap, row 2 from a half swap followed by a row swap
-__device__ __forceinline__ double from_row_below(double v) {
-  const int row = (threadIdx.x & 63) >> 4;
-  int2 h = *reinterpret_cast<int2*>(&v), o;
-  {
-    const auto a = __builtin_amdgcn_permlane32_swap((unsigned)h.x, (unsigned)h.x, false, false);
-    const auto b = __builtin_amdgcn_permlane16_swap((unsigned)a[0], (unsigned)h.x, false, false);
-    o.x = (int)(row == 2 ? b[1] : b[0]);
-  }
-  {
-    const auto a = __builtin_amdgcn_permlane32_swap((unsigned)h.y, (unsigned)h.y, false, false);
-    const auto b = __builtin_amdgcn_permlane16_swap((unsigned)a[0], (unsigned)h.y, false, false);
-    o.y = (int)(row == 2 ? b[1] : b[0]);
-  }
-  return *reinterpret_cast<double*>(&o);
-}
-
-// the value of the lane 32 below (lanes 32..63)
-__device__ __forceinline__ double from_half_below(double v) {
-  int2 h = *reinterpret_cast<int2*>(&v), o;
-  o.x = (int)__builtin_amdgcn_permlane32_swap((unsigned)h.x, (unsigned)h.x, false, false)[0];
-  o.y = (int)__builtin_amdgcn_permlane32_swap((unsigned)h.y, (unsigned)h.y, false, false)[0];
-  return *reinterpret_cast<double*>(&o);
-}
-
-// inclusive Hillis-Steele scan over the wave (offsets 1, 2, ..., 32, each
-// lane adding the value `offset` lanes below).  Offset 1 is a wave shift
-// (DPP), 16 and 32 are lane swaps, 2-8 cross-lane reads; every lane adds
-// the same operands in the same order at every offset whichever move
-// brings them, so the sums are the plain shuffle scan's bit for bit.
-__device__ __forceinline__ double wave_scan(double v) {
-  const int lane = threadIdx.x & 63;
-  { const double t = dpp_d<0x138>(v); if (lane >= 1) v = v + t; }   // wave_shr:1
-#pragma unroll
-  for (int d = 2; d < 16; d <<= 1) {
-    const double t = __shfl_up(v, d, 64);
-    if (lane >= d) v = v + t;
-  }
-  { const double t = from_row_below(v); if (lane >= 16) v = v + t; }
-  { const double t = from_half_below(v); if (lane >= 32) v = v + t; }
+// inclusive scan by DPP adds alone (rows of 16, then the rows' totals): the
+// picks' descent, which needs the sums only to compare and to carry
+__device__ __forceinline__ double dpp_scan(double v) {
+  v += dpp_f64<0x111, 0xf>(v);   // row_shr 1, 2, 4, 8
+  v += dpp_f64<0x112, 0xf>(v);
+  v += dpp_f64<0x114, 0xf>(v);
+  v += dpp_f64<0x118, 0xf>(v);
+  v += dpp_f64<0x142, 0xa>(v);   // row_bcast 15, 31
+  v += dpp_f64<0x143, 0xc>(v);
   return v;
 }
 
-// the last element of wave_scan(v), in every lane: lane 63's scan value is
-// a balanced pairwise sum ((v62 + v63) + (v60 + v61)) + ..., which a
-// butterfly over pairs, quads, eights, rows and halves forms with the same
-// operands (partners by DPP quad permutations and mirrors, then lane
-// swaps), so it is bit-identical without the scan's serial reads
+// a group's sum in every lane, in the order the trees are built with: the
+// last element of the Hillis-Steele scan is a balanced pairwise sum ((v62 +
+// v63) + (v60 + v61)) + ..., which a butterfly over pairs, quads, eights, rows
+// and halves forms with the same operands (partners by DPP quad permutations
+// and mirrors, then lane swaps)
 __device__ __forceinline__ double group_total(double v) {
   v = v + dpp_d<0xB1>(v);    // quad_perm [1,0,3,2]
   v = v + dpp_d<0x4E>(v);    // quad_perm [2,3,0,1]
@@ -1018,7 +1022,7 @@ __device__ __forceinline__ uint64_t tree_pick(Ctx<KMAX>& C, int tr, double u) {
     long long res = 0;
     for (int h = C.D.top; h >= 0; --h) {
       double c = tree_val(C, tr, h, 64 * g + lane);
-      double s = wave_scan(c);
+      double s = dpp_scan(c);
       unsigned long long m1 = __ballot(c > 0.0 && r < carry + s);
       unsigned long long nz = __ballot(c > 0.0);
       int pick = m1 ? (__ffsll((long long)m1) - 1) : (nz ? 63 - __clzll((long long)nz) : -1);
@@ -1109,7 +1113,7 @@ __device__ __forceinline__ uint64_t tree_pick_zero(Ctx<KMAX>& C, int tr, double 
       double c = tree_val(C, tr, h, 64 * g + lane);
 #pragma unroll
       for (int q = 0; q < BMG_TREE_LEV; ++q) if (q == h) cl[q] = c;
-      double s = wave_scan(c);
+      double s = dpp_scan(c);
       unsigned long long m1 = __ballot(c > 0.0 && r < carry + s);
       unsigned long long nz = __ballot(c > 0.0);
       int pick = m1 ? (__ffsll((long long)m1) - 1) : (nz ? 63 - __clzll((long long)nz) : -1);
@@ -1658,18 +1662,75 @@ __device__ __forceinline__ double prior_rem(const ChainConst& K, const int (&Ns)
          (log(K.tp_sum + n_old - 1) - log(K.tp_type + sel(Ns, type) - 1));
 }
 
-template <int KMAX>
-__device__ __forceinline__ double draw_inv_tau2(Ctx<KMAX>& C, int term) {
-  if (C.K.use_ind)
-    return 1.0 / (C.R.alpha2 * rng_sinvchi2(C.R.rng, C.K.nu_tau2[term], C.K.s2_tau2[term]));
-  return sel(C.R.ita2, term);
+// Draws on the chain's stream, one per term in term order, a term per thread:
+// a thread starts its term where the stream would be if every earlier term of
+// the round took one trial (two Philox blocks); the first term after which
+// that does not hold ends the round, and the next round restarts from the
+// stream position it left.  The draws are the sequential loop's, value for
+// value; a draw alone takes about 1.2 us.  draw(r, i): term i's value from the
+// stream r; out[0 .. count) receives them (LDS).
+template <int KMAX, typename Draw>
+__device__ __forceinline__ void draw_terms(Ctx<KMAX>& C, int first, int count, double* out, Draw draw) {
+  Smem<KMAX>& S = C.S;
+  Reg& R = C.R;
+  uint64_t base = (uint64_t)R.rng.c0 | ((uint64_t)R.rng.c1 << 32);
+  __syncthreads();
+  while (first < count) {
+    const int i = first + (int)threadIdx.x;
+    long long stop = count;          // first term whose stream use differs
+    uint64_t next = 0;
+    double v = 0.0;
+    if (i < count) {
+      const uint64_t start = base + 2ull * (uint64_t)threadIdx.x;
+      Rng r = R.rng;
+      r.c0 = (uint32_t)start; r.c1 = (uint32_t)(start >> 32);
+      v = draw(r, i);
+      next = (uint64_t)r.c0 | ((uint64_t)r.c1 << 32);
+      if (next - start != 2) stop = i;
+      if (i == first + BMG_BLOCK - 1 && stop == count) stop = i;
+    }
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) {
+      const long long w = __shfl_xor(stop, o, 64);
+      stop = w < stop ? w : stop;
+    }
+    if (lane_id() == 0) S.redi[wave_id()] = stop;
+    __syncthreads();
+    stop = S.redi[0];
+    for (int w = 1; w < BMG_BLOCK / 64; ++w) stop = S.redi[w] < stop ? S.redi[w] : stop;
+    // terms first..stop are final; the stream continues after term stop
+    if (i <= stop && i < count) out[i] = v;
+    if (i == stop) S.bci[3] = (long long)next;
+    __syncthreads();
+    if (stop >= count) {
+      base += 2ull * (uint64_t)(count - first);
+      first = count;
+    } else {
+      base = (uint64_t)S.bci[3];
+      first = (int)stop + 1;
+    }
+    __syncthreads();
+  }
+  R.rng.c0 = (uint32_t)base; R.rng.c1 = (uint32_t)(base >> 32);
 }
 
+// the prior precisions of the next n_add new terms, in order, in S.mu (whose
+// own contents a change of the model makes void); new_term picks the k-th's
 template <int KMAX>
-__device__ __forceinline__ void prepare_add_new_term(Ctx<KMAX>& C, double* d2) {
-  int type = C.D.type;
-  if (type == 4) { d2[0] = draw_inv_tau2(C, 0); d2[1] = draw_inv_tau2(C, 1); }
-  else d2[0] = draw_inv_tau2(C, type);
+__device__ __forceinline__ void draw_new_terms(Ctx<KMAX>& C, int n_add) {
+  if (!C.K.use_ind || n_add == 0) return;
+  const int w = C.D.type == 4 ? 2 : 1;
+  const double a2 = C.R.alpha2;
+  draw_terms(C, 0, w * n_add, C.S.mu, [&](Rng& r, int i) {
+    const int t = w == 2 ? i & 1 : C.D.type;
+    return 1.0 / (a2 * rng_sinvchi2(r, C.K.nu_tau2[t], C.K.s2_tau2[t]));
+  });
+}
+template <int KMAX>
+__device__ __forceinline__ void new_term(Ctx<KMAX>& C, int k, double* d2) {
+  const int type = C.D.type, w = type == 4 ? 2 : 1;
+  for (int q = 0; q < w; ++q)
+    d2[q] = C.K.use_ind ? C.S.mu[w * k + q] : sel(C.R.ita2, w == 2 ? q : type);
 }
 
 // ------------------------------------------------- beta / sigma2 / pve ----
@@ -1940,55 +2001,14 @@ __device__ __forceinline__ void sample_alpha_and_tau2(Ctx<KMAX>& C) {
   // sample_tau2
   double a2s2 = R.alpha2 * R.sigma2;
   if (K.use_ind) {
-    // one draw per term, in term order on the chain's stream, computed a
-    // term per thread: a thread starts its term where the stream would be
-    // if every earlier term of the round took one trial (two Philox
-    // blocks); the first term after which that does not hold ends the
-    // round, and the next round restarts from the stream position it left.
-    // The draws are the sequential loop's, value for value.
-    uint64_t base = (uint64_t)R.rng.c0 | ((uint64_t)R.rng.c1 << 32);
-    int first = C.D.me;   // the covariates' precisions are fixed
-    while (first < R.beta_len) {
-      const int i = first + (int)threadIdx.x;
-      long long stop = R.beta_len;     // first term whose stream use differs
-      uint64_t next = 0;
-      if (i < R.beta_len) {
-        const uint64_t start = base + 2ull * (uint64_t)threadIdx.x;
-        Rng r = R.rng;
-        r.c0 = (uint32_t)start; r.c1 = (uint32_t)(start >> 32);
-        const int t = S.xtype[i];
-        const double nu = K.nu_tau2[t] + 1.0;
-        const double s2 = (K.nus2_tau2[t] + S.beta[i] * S.beta[i] / a2s2) / nu;
-        const double dv = 1.0 / (R.alpha2 * rng_sinvchi2(r, nu, s2));
-        next = (uint64_t)r.c0 | ((uint64_t)r.c1 << 32);
-        if (next - start != 2) stop = i;
-        S.work[i] = dv;
-        if (i == first + BMG_BLOCK - 1 && stop == R.beta_len) stop = i;
-      }
-#pragma unroll
-      for (int o = 32; o > 0; o >>= 1) {
-        const long long w = __shfl_xor(stop, o, 64);
-        stop = w < stop ? w : stop;
-      }
-      __syncthreads();
-      if (lane_id() == 0) S.redi[wave_id()] = stop;
-      __syncthreads();
-      stop = S.redi[0];
-      for (int w = 1; w < BMG_BLOCK / 64; ++w) stop = S.redi[w] < stop ? S.redi[w] : stop;
-      // terms first..stop are final; the stream continues after term stop
-      if (i <= stop && i < R.beta_len) S.d[i] = S.work[i];
-      if (i == stop) S.bci[3] = (long long)next;
-      __syncthreads();
-      if (stop >= R.beta_len) {
-        base += 2ull * (uint64_t)(R.beta_len - first);
-        first = R.beta_len;
-      } else {
-        base = (uint64_t)S.bci[3];
-        first = (int)stop + 1;
-      }
-      __syncthreads();
-    }
-    R.rng.c0 = (uint32_t)base; R.rng.c1 = (uint32_t)(base >> 32);
+    // (the covariates' precisions are fixed)
+    const double a2 = R.alpha2;
+    draw_terms(C, C.D.me, R.beta_len, S.d, [&](Rng& r, int i) {
+      const int t = S.xtype[i];
+      const double nu = K.nu_tau2[t] + 1.0;
+      const double s2 = (K.nus2_tau2[t] + S.beta[i] * S.beta[i] / a2s2) / nu;
+      return 1.0 / (a2 * rng_sinvchi2(r, nu, s2));
+    });
   } else {
     double b2[4] = {0, 0, 0, 0}; double mt[4] = {0, 0, 0, 0};
     for (int i = C.D.me; i < R.beta_len; ++i) {
@@ -2061,7 +2081,7 @@ __device__ __forceinline__ int sample_naive(const double* cumsum, int m, double 
 // on the state, and add/remove and state-change moves keep their share).
 // 0 add/remove, 1 swap, 2 state change, 3 learned swap
 template <int KMAX>
-__device__ __forceinline__ int draw_move(const Ctx<KMAX>& C, Rng& rng) {
+__device__ __forceinline__ int draw_move(const Ctx<KMAX>& C, ChainRng& rng) {
   const double pm[3] = {0.7, 0.7 + 0.15, 0.7 + 0.15 + 0.15};
   const double r = rng_u01(rng) * pm[2];
   int move = r < pm[0] ? 0 : (r < pm[1] ? 1 : 2);
@@ -2071,7 +2091,7 @@ __device__ __forceinline__ int draw_move(const Ctx<KMAX>& C, Rng& rng) {
 
 // the size of an add/remove (0), swap (1) or state-change (2) move
 template <int KMAX>
-__device__ __forceinline__ int draw_move_size(const Ctx<KMAX>& C, Rng& rng, int move) {
+__device__ __forceinline__ int draw_move_size(const Ctx<KMAX>& C, ChainRng& rng, int move) {
   const ChainConst& K = C.K;
   uint64_t mx = K.max_ms;
   if (move == 1) {
@@ -2398,7 +2418,7 @@ __device__ __forceinline__ uint64_t dr_second_stage(Ctx<KMAX>& C, int n, double 
     for (uint64_t base = 0; base < half; base += 64) {
       const uint64_t idx = base + lane;
       const double x = idx < half ? p[idx] : 0.0;
-      const double mine = sum + wave_scan(x);
+      const double mine = sum + dpp_scan(x);
       sum = readlane_d(mine, 63);
       if (idx < half) p[idx] = mine;
     }
@@ -2609,7 +2629,10 @@ __device__ __forceinline__ int move_addrem(Ctx<KMAX>& C) {
     remove_term(C, mind, i == last_rem ? first_add : -1);
   }
   double d2[2];
-  for (int i = 0; i < ms; ++i) {
+  int n_add = 0;
+  for (int i = 0; i < ms; ++i) n_add += S.mi_isadd[i];
+  draw_new_terms(C, n_add);
+  for (int i = 0, k = 0; i < ms; ++i) {
     if (!S.mi_isadd[i]) continue;
     uint64_t ind = S.mi[i];
     long long next = -1;   // the move's next addition, whose dots are formed ahead
@@ -2617,7 +2640,7 @@ __device__ __forceinline__ int move_addrem(Ctx<KMAX>& C) {
       if (S.mi_isadd[j]) { next = (long long)S.mi[j]; break; }
     tree_set(C, 1, ind, 0);
     lmpc += prior_add(K, R.Ns, R.nloci, type);
-    prepare_add_new_term(C, d2);
+    new_term(C, k++, d2);
     add_term(C, (uint32_t)ind, 0, d2, next);
   }
   R.pre_snp = -1;
@@ -2781,10 +2804,11 @@ __device__ __forceinline__ int move_switch(Ctx<KMAX>& C) {
     remove_term(C, mir);
   }
   double d2[2];
+  draw_new_terms(C, ms);
   for (int i = 0; i < ms; ++i) {
     uint64_t ia = S.mi_add[i];
     int t_ind = S.mark_val[i];
-    prepare_add_new_term(C, d2);
+    new_term(C, i, d2);
     add_term(C, (uint32_t)ia, t_ind, d2);
   }
   R.n_marks = 0;
@@ -2868,7 +2892,8 @@ __device__ __forceinline__ int move_learned_swap(Ctx<KMAX>& C) {
   if (threadIdx.x == 0) { S.mi_rem[0] = (uint64_t)j; S.mi_add[0] = (uint64_t)k; }
   remove_term(C, mir);
   double d2[2];
-  prepare_add_new_term(C, d2);
+  draw_new_terms(C, 1);
+  new_term(C, 0, d2);
   add_term(C, (uint32_t)k, t_ind, d2);
   double log_r = R.ll - R.c_ll + lq;
   if (log_r >= 0 || log(rng_u01(R.rng)) <= log_r) {
@@ -2947,10 +2972,11 @@ __device__ __forceinline__ int move_statechange(Ctx<KMAX>& C) {
   }
   double d2[2];
   int t_ind = 0;
+  draw_new_terms(C, ms_add);
   for (int i = 0; i < ms_add; ++i) {
     uint64_t ia = S.mi_add[i];
     lmpc += prior_add(K, R.Ns, R.nloci, type);
-    prepare_add_new_term(C, d2);
+    new_term(C, i, d2);
     // the next addition's dots are formed during this one's sweep
     add_term(C, (uint32_t)ia, t_ind, d2, i + 1 < ms_add ? (long long)S.mi_add[i + 1] : -1);
   }
@@ -3029,8 +3055,9 @@ template <int KMAX>
 __device__ __forceinline__ void load_chain(Ctx<KMAX>& C, const ChainScal& CS) {
   Smem<KMAX>& S = C.S;
   Reg& R = C.R;
-  R.rng = rng_make(C.K.seed, C.K.chain_id, 0, 0);
+  (Rng&)R.rng = rng_make(C.K.seed, C.K.chain_id, 0, 0);
   R.rng.c0 = CS.rng_c0; R.rng.c1 = CS.rng_c1;
+  R.rng.base = ((uint64_t)R.rng.c1 << 32 | R.rng.c0) - 64;   // no block at hand
   R.cols = R.c_cols = CS.cols;
   R.nloci = R.c_nloci = CS.nloci;
   for (int q = 0; q < 5; ++q) R.Ns[q] = R.c_Ns[q] = CS.Ns[q];
@@ -3178,7 +3205,7 @@ __device__ __forceinline__ void refresh_tau2(Ctx<KMAX>& C) {
 template <int KMAX>
 __device__ __forceinline__ int next_growth(Ctx<KMAX>& C) {
   Reg& R = C.R;
-  Rng q = R.rng;
+  ChainRng q = R.rng;
   const int move = draw_move(C, q);
   if (move == 1 || move == 3) return 0;
   const int ms = draw_move_size(C, q, move);
