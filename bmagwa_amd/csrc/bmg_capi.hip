@@ -816,7 +816,7 @@ static int batch_create(bmg_ctx** ctxs, int n_ctx, int n_chains, const int32_t* 
   size_t o_ta = add(8 * tmax), o_tr = add(8 * tmax);
   size_t o_pp = add(8 * pmax), o_pr = add(8 * pmax), o_prr = add(8 * pmax);
   // per-column arrays for BMG_KMAXG columns whatever the launch capacity K:
-  // a chain that leaves K continues in the 256-column kernel on the same state
+  // a chain that leaves K goes on with its factor in HBM on the same state
   const size_t G = BMG_KMAXG;
   size_t o_L = add(8 * G * (G + 1) / 2), o_xx = add(8 * G * G);
   size_t o_Lw = add(8 * (G * (G + 1) / 2 + BMG_LPAD));

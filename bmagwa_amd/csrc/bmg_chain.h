@@ -104,7 +104,7 @@ struct ChainArrays {
   double* tree_add; double* tree_rem;    // tree_size each
   double* p_proposal; double* p_rao; double* p_r;  // p
   double* Lcur;              // packed upper factor, BMG_KMAXG (BMG_KMAXG+1) / 2
-  double* Lwork;             // the same size: working factor of the 256-column kernel
+  double* Lwork;             // the same size: working factor past the LDS capacity
   double* xxs;               // BMG_KMAXG x BMG_KMAXG slot matrix
   uint32_t* xcol;            // BMG_KMAXG x W32: packed genotypes of each slot's column
   double* y_hat;             // n_pad

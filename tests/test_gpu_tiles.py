@@ -49,6 +49,36 @@ def test_column_dots(bmg, n):
     ctx.close()
 
 
+# one group width each, and two passes
+@pytest.mark.parametrize("n", [37, 1025, 4097, 20481])
+def test_column_dots_of_a_pair(bmg, n):
+    """Two columns a term, the second's dots formed during the first's sweep:
+    X^T X exact while terms are added, removed and added again."""
+    G, body = genotypes(n, 14, n + 1)
+    y = np.random.default_rng(n).normal(size=n)
+    ctx = bmg.Ctx(n, 14, body, y, types=("AH",))
+    m = bmg.Model(ctx, n_plus_nu=n + 1.0, nus2_plus_yy=1.0 + float(y @ y), inv_tau2_e0=0.0)
+    terms = []
+
+    def check():
+        X = np.array([np.ones(n)] + [np.array(CODED[c])[G[j]] for j in terms for c in "AH"])
+        assert np.array_equal(np.triu(m.get()["xx"]), np.triu(X @ X.T))
+
+    for j in range(10):
+        m.add_term(j, 0, [3.0, 4.0])
+        terms.append(j)
+    check()
+    for i in (7, 0, 3):
+        m.remove_term(i)
+        del terms[i]
+    for j in range(10, 14):
+        m.add_term(j, 0, [2.0, 5.0])
+        terms.append(j)
+    check()
+    m.close()
+    ctx.close()
+
+
 # columns before the removal; the removed term; n - 1 columns follow it
 @pytest.mark.parametrize("k,rm", [(2, 0), (9, 0), (9, 4), (9, 8), (64, 0), (65, 0), (66, 0), (66, 60), (129, 0),
                                   (130, 1), (130, 70), (135, 0), (135, 127), (135, 134)])
