@@ -2343,15 +2343,26 @@ __device__ __forceinline__ double exhaustive_modelset(Ctx<KMAX>& C, int cl, int 
   const int w = C.D.type == BMG_AH ? 2 : 1;
   const int nT = w * n;                 // the block's columns: the last n loci
   const int c0 = R.cols - nT;           // after the fixed columns and the other loci
-  for (int c = 0; c < nT; ++c)
-    for (int r = threadIdx.x; r <= c; r += BMG_BLOCK) S.ex_L[P(c) + r] = S.L[P(c0 + c) + c0 + r];
+  // each column scaled by a power of two to a diagonal entry in [1/2, 1): the
+  // walk's rotations act on rows and do not see it, and its products of up to
+  // 40 diagonal entries stay far inside the exponent's range whatever the
+  // precisions (an entry is at least sqrt(d)); the exponents go back in with
+  // the loci's log d
+  for (int c = 0; c < nT; ++c) {
+    const int e = __builtin_amdgcn_frexp_exp(S.L[P(c0 + c) + c0 + c]);
+    for (int r = threadIdx.x; r <= c; r += BMG_BLOCK) S.ex_L[P(c) + r] = ldexp(S.L[P(c0 + c) + c0 + r], -e);
+  }
   for (int i = threadIdx.x; i < nT; i += BMG_BLOCK) S.ex_v[i] = S.v[c0 + i];
-  // per locus: half its columns' log d, and the prior change of the q-th one
-  // (src/prior.hpp:144-158, one effect type: it depends on the number alone)
+  // per locus: half its columns' log d less the logarithm of their scale, and
+  // the prior change of the q-th one (src/prior.hpp:144-158, one effect type:
+  // it depends on the number alone)
   if ((int)threadIdx.x < n) {
     const int q = threadIdx.x, type = C.D.type;
     double ld = 0.0;
-    for (int k = 0; k < w; ++k) ld += 0.5 * log(S.d[c0 + w * q + k]);
+    for (int k = 0; k < w; ++k) {
+      const int c = c0 + w * q + k;
+      ld += 0.5 * log(S.d[c]) - (double)__builtin_amdgcn_frexp_exp(S.L[P(c) + c]) * 0x1.62e42fefa39efp-1;   // ln 2
+    }
     S.ex_ld[q] = ld;
     int Ns[5] = {0, 0, 0, 0, 0};
     put(Ns, type, cl + q);

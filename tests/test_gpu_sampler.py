@@ -451,3 +451,31 @@ def test_save_beta_matches_oracle(bmg, tmp_path):
     base = str(tmp_path / "sb")
     b.write_outputs(0, base)
     assert np.array_equal(np.fromfile(base + "_beta.dat", dtype=np.float64), got)
+
+
+@pytest.mark.parametrize("seed", [17, 18])
+def test_delayed_rejection_under_a_tight_prior(bmg, seed):
+    """Effects with prior variances of 1e-18, two columns a SNP and moves of
+    up to 20 SNPs: each of the up to 40 columns that a move toggles has a
+    factor diagonal of about 1e9, so the determinant of a sub-model passes the
+    largest double from 35 columns on.  Its logarithm does not, and the second
+    stage's choices are the oracle's."""
+    n, p, n_iter = 20000, 90, 40
+    rng = np.random.default_rng(99)
+    maf = rng.uniform(0.1, 0.5, size=(p, 1))
+    G = (rng.random((p, n)) < maf).astype(np.uint8) + (rng.random((p, n)) < maf)
+    code = np.array([0, 2, 3], np.uint8)[G].reshape(p, -1, 4)
+    body = (code << np.array([0, 2, 4, 6], np.uint8)).sum(2, dtype=np.uint8).ravel()
+    y = rng.normal(size=p) @ G + rng.normal(scale=3.0, size=n)
+    cfg = synth.sampler_cfg(n, p, 45, types="AH", seed=seed, n_rao=20, n_rao_burnin=2, thin=10, var_qg=100.0,
+                            n_sample_tau2_and_missing=10, max_move_size=20, delay_rejection=20, p_move_size=0.01,
+                            adapt_p_move_size=0, s2_tau2=[1e-18] * 4, do_n_iter=n_iter)
+    s = oracle_run(cfg, body, y, n_iter)
+    ctx = bmg.Ctx(n, p, body, y, types=("AH",))
+    b = bmg.Batch([ctx], [0], [cfg], dict(trace_every_iter=1))
+    b.setup()
+    b.run(n_iter)
+    tr = b.trace(0)
+    compare(tr, s.trace(), n_iter)
+    # moves of 18 SNPs and more reached the second stage, which kept a part
+    assert ((tr["jd"] > 0) & (tr["jd"] < tr["ms"]) & (tr["move"] != 1) & (tr["ms"] >= 18)).any()
