@@ -2027,14 +2027,16 @@ __device__ __forceinline__ void xmoments(Ctx<KMAX>& C, const double* coef, int L
 
 // src/model.hpp:345-392: shares of var(E beta_E) (covariates beyond the
 // constant), var(X_g beta_g) and var(y_hat) in var(y_hat) + sigma2
-// (need_y: leave y_hat too.  Nothing reads the one of a sample that no RB scan
-// follows, and without covariates each is formed anew; with them a model
-// without loci adds to the one it holds, so every sample's is formed.)
+// (need_y: leave y_hat too; the sums then come with it, and belong to it also
+// where a caller has changed its model since it drew beta.  Nothing reads the
+// y_hat of a sample that no RB scan follows, and without covariates each is
+// formed anew; with them a model without loci adds to the one it holds, so
+// every sample's is formed.)
 template <int KMAX>
 __device__ __forceinline__ void compute_pve(Ctx<KMAX>& C, double* pves, int need_y) {
   double s[8];
   if (need_y || C.D.me > 1) xbeta(C, s, 1);
-  if (C.D.me == 1) xmoments(C, C.S.beta, C.R.beta_len, s);
+  else xmoments(C, C.S.beta, C.R.beta_len, s);
   const double n = (double)C.D.n;
   const bool ce = C.D.me > 1, cg = C.R.nloci > 0;
   pves[2] = ce ? (s[6] - s[5] * s[5] / n) / (n - 1) : 0.0;

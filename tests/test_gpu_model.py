@@ -296,3 +296,29 @@ def test_residual_term_in_the_cancelling_regime(bmg):
     assert g["syx"] == pytest.approx(s_true, rel=1e-3)
     assert g["syx"] == pytest.approx(om.get()["syx"], rel=1e-6)
     assert np.isfinite(m.log_likelihood())
+
+
+def test_pve_is_of_the_returned_fit_without_a_new_draw(bmg):
+    """Terms removed and added after the last draw of beta: the shares are
+    the variance of the y_hat that the call leaves, as with a new draw."""
+    n, p = 400, 600
+    body, y, cfg = _sampler_dataset(n, p, 41)
+    ctx = bmg.Ctx(n, p, body, y)
+    m = bmg.Model(ctx, cfg=cfg)
+
+    def check():
+        pve = m.compute_pve()
+        _, s2, yh = m.beta()
+        want = yh.var(ddof=1) / (yh.var(ddof=1) + s2)
+        assert np.allclose(pve, [want, want, 0.0], rtol=1e-10, atol=0)
+
+    for j in (17, 120, 250, 333, 480, 555):
+        m.add_term(j, 0, 0.05)
+    m.sample_beta_sigma2()
+    check()
+    m.remove_term(5)
+    m.remove_term(4)
+    m.add_term(77, 0, 0.05)
+    check()
+    m.sample_beta_sigma2()
+    check()
