@@ -1,9 +1,12 @@
 """Kernels at the edges of their tiles: the column dots at every group width
-and piece count (and past one pass), the sweeps and the downdate on both sides
-of 64 and 128 columns, the scan's results and digits at odd sizes, the raw
-body's rows at every alignment."""
+and piece count (and past one pass), on four waves and ahead on three, the
+sweeps and the downdate on both sides of 64 and 128 columns, the scan's
+results and digits at odd sizes, the raw body's rows at every alignment."""
 import numpy as np
 import pytest
+
+import oracle
+from bmagwa_amd import synth
 
 pytestmark = pytest.mark.gpu
 
@@ -52,8 +55,8 @@ def test_column_dots(bmg, n):
 # one group width each, and two passes
 @pytest.mark.parametrize("n", [37, 1025, 4097, 20481])
 def test_column_dots_of_a_pair(bmg, n):
-    """Two columns a term, the second's dots formed during the first's sweep:
-    X^T X exact while terms are added, removed and added again."""
+    """Two columns a term: X^T X exact while terms are added, removed and
+    added again (a Model forms each column's dots on all four waves)."""
     G, body = genotypes(n, 14, n + 1)
     y = np.random.default_rng(n).normal(size=n)
     ctx = bmg.Ctx(n, 14, body, y, types=("AH",))
@@ -76,6 +79,39 @@ def test_column_dots_of_a_pair(bmg, n):
         terms.append(j)
     check()
     m.close()
+    ctx.close()
+
+
+# both sides of every group width and piece count, then two and three passes
+@pytest.mark.parametrize("types", ["A", "AH"])
+@pytest.mark.parametrize("n", [37, 1024, 1025, 2048, 2049, 4097, 8192, 8193, 12288, 12289, 20480, 20481, 40961])
+def test_column_dots_formed_ahead(bmg, n, types):
+    """A chain's moves of several SNPs, whose next columns' dots three waves
+    form beside a sweep or a downdate (with the tree write and the row move
+    that go with it): the dots are whole numbers, so moves and sizes are the
+    oracle's and log-likelihoods agree to 1e-10, as for every trajectory."""
+    p, n_iter = 48, 400
+    G, body = genotypes(n, p, n)
+    rng = np.random.default_rng(n)
+    y = rng.normal(size=12) @ G[:12] + rng.normal(scale=3.0, size=n)
+    cfg = synth.sampler_cfg(n, p, 12, types=types, seed=5, n_rao=50, n_rao_burnin=2, max_move_size=10,
+                            p_move_size=0.1, adapt_p_move_size=0, do_n_iter=n_iter)
+    s = oracle.Sampler(cfg, oracle.Data(n, p, body, y))
+    s.init_flat()
+    assert s.setup() == 0
+    s.iterate(n_iter)
+    want = s.trace()
+    ctx = bmg.Ctx(n, p, body, y, types=(types,))
+    b = bmg.Batch([ctx], [0], [cfg], dict(trace_every_iter=1))
+    b.setup()
+    b.run(n_iter)
+    got = b.trace(0)
+    for key in ("move", "jd", "ms", "size"):
+        assert np.array_equal(got[key], want[key]), key
+    assert np.allclose(got["loglik"], want["loglik"], rtol=1e-10, atol=0)
+    # moves of several SNPs were accepted, so their columns are in the model
+    assert ((got["move"] == 0) & (got["jd"] > 2)).any()
+    b.close()
     ctx.close()
 
 
