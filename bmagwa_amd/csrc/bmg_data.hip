@@ -108,29 +108,30 @@ __global__ void k_counts(const uint32_t* __restrict__ g, uint64_t p, uint32_t W3
   if (lane == 0) { out[3 * j] = c1; out[3 * j + 1] = c2; out[3 * j + 2] = (long long)n - miss; }
 }
 
-// out[j] = x_j . y of every SNP under `coding`: a wave per XY_SNPS SNPs, a
+// out[j] = x_j . y of every SNP under `coding`: WAVES waves share SNPS SNPs, a
 // word (16 individuals) of each a lane, so the lane's 16 values of y are read
 // once for all of them.  Bound by the conversions and multiply-adds (one each
 // per genotype).  (A workgroup per SNP read y once per SNP: 1.3 ms for 100,000
 // SNPs of 10,000 individuals.)
-#define XY_SNPS 8
+template <int SNPS, int WAVES>
 __global__ __launch_bounds__(256) void k_xy_all(const uint32_t* __restrict__ g, uint64_t p, uint32_t W32,
                                                 const double* __restrict__ y, int coding, double* __restrict__ out) {
-  const uint64_t j0 = (blockIdx.x * (uint64_t)4 + threadIdx.x / 64) * XY_SNPS;
-  if (j0 >= p) return;
-  const int lane = threadIdx.x & 63;
-  double acc[XY_SNPS];
+  __shared__ double part[4][SNPS];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const uint64_t j0 = (blockIdx.x * (uint64_t)(4 / WAVES) + wave / WAVES) * SNPS;
+  if (j0 >= p) return;   // with WAVES = 4: the whole workgroup
+  double acc[SNPS];
 #pragma unroll
-  for (int s = 0; s < XY_SNPS; ++s) acc[s] = 0.0;
-  for (uint32_t k = lane; k < W32; k += 64) {
-    uint32_t w[XY_SNPS];
+  for (int s = 0; s < SNPS; ++s) acc[s] = 0.0;
+  for (uint32_t k = wave % WAVES * 64 + lane; k < W32; k += 64 * WAVES) {
+    uint32_t w[SNPS];
 #pragma unroll
-    for (int s = 0; s < XY_SNPS; ++s) w[s] = g[min(j0 + s, p - 1) * W32 + k];
+    for (int s = 0; s < SNPS; ++s) w[s] = g[min(j0 + s, p - 1) * W32 + k];
     double yy[16];
 #pragma unroll
     for (int f = 0; f < 16; f += 2) *(double2*)(yy + f) = *(const double2*)(y + 16 * (size_t)k + f);
 #pragma unroll
-    for (int s = 0; s < XY_SNPS; ++s) {
+    for (int s = 0; s < SNPS; ++s) {
       const uint32_t lo = w[s] & BMG_EVEN, hi = (w[s] >> 1) & BMG_EVEN;
       const uint32_t v = coding == 0 ? hi + (hi & lo) : (coding == 1 ? hi & ~lo : (coding == 2 ? hi : hi & lo));
 #pragma unroll
@@ -138,9 +139,16 @@ __global__ __launch_bounds__(256) void k_xy_all(const uint32_t* __restrict__ g, 
     }
   }
 #pragma unroll
-  for (int s = 0; s < XY_SNPS; ++s) {
+  for (int s = 0; s < SNPS; ++s) {
     const double t = wave_sum(acc[s]);
-    if (lane == 0 && j0 + s < p) out[j0 + s] = t;
+    if (WAVES > 1) part[wave][s] = t;
+    else if (lane == 0 && j0 + s < p) out[j0 + s] = t;
+  }
+  if (WAVES > 1) {
+    static_assert(WAVES == 1 || WAVES == 4, "a wave or a workgroup");
+    __syncthreads();
+    if (threadIdx.x < SNPS && j0 + threadIdx.x < p)
+      out[j0 + threadIdx.x] = ((part[0][threadIdx.x] + part[1][threadIdx.x]) + part[2][threadIdx.x]) + part[3][threadIdx.x];
   }
 }
 
@@ -733,8 +741,17 @@ int launch_restride(const uint8_t* raw, bmg_ctx* c, hipStream_t s) {
 }
 
 int launch_xy_all(const DevData& D, int coding, double* out, hipStream_t s) {
-  hipLaunchKernelGGL(k_xy_all, dim3((unsigned)((D.p + 4 * XY_SNPS - 1) / (4 * XY_SNPS))), dim3(256), 0, s, D.g, D.p,
-                     D.W32, D.y, coding, out);
+  // With few SNPs, eight a wave leave most of the chip idle and a wave long at
+  // work; a workgroup then takes a SNP.  Set-up of a batch at p = 128 / 1,024 /
+  // 2,048 / 8,192, in us: at n = 10,000 a workgroup a SNP 44 / 51 / 61 / 117,
+  // eight a wave 57 / 58 / 58 / 60; at n = 200,000 86 / 225 / 397 / 1,431 and
+  // 328 / 353 / 355 / 408.
+  constexpr uint64_t FEW_SNPS = 1536;
+  if (D.p < FEW_SNPS)
+    hipLaunchKernelGGL((k_xy_all<1, 4>), dim3((unsigned)D.p), dim3(256), 0, s, D.g, D.p, D.W32, D.y, coding, out);
+  else
+    hipLaunchKernelGGL((k_xy_all<8, 1>), dim3((unsigned)((D.p + 31) / 32)), dim3(256), 0, s, D.g, D.p, D.W32, D.y,
+                       coding, out);
   BMG_HIP(hipGetLastError());
   return BMG_OK;
 }

@@ -115,6 +115,36 @@ def test_column_dots_formed_ahead(bmg, n, types):
     ctx.close()
 
 
+# a workgroup a SNP below 1,536 SNPs, then groups of eight, whole and ragged
+@pytest.mark.parametrize("n,p,types", [(15, 60, "A"), (4097, 60, "R"), (1030, 1535, "AH"), (1030, 1536, "A"),
+                                       (1030, 1537, "D"), (515, 1543, "AH")])
+def test_xy_table(bmg, n, p, types):
+    """The table of x.y that a chain's additions read: a wrong entry shows in
+    the first model that holds its SNP.  The sums of either form are within
+    n ulps of the oracle's; trajectories agree to 1e-10 as elsewhere."""
+    n_iter = 300
+    G, body = genotypes(n, p, n + p)
+    rng = np.random.default_rng(p)
+    y = rng.normal(size=10) @ G[p - 10:] + rng.normal(scale=2.0, size=n)
+    cfg = synth.sampler_cfg(n, p, 10, types=types, seed=9, n_rao=50, n_rao_burnin=2, max_move_size=10, do_n_iter=n_iter)
+    s = oracle.Sampler(cfg, oracle.Data(n, p, body, y))
+    s.init_flat()
+    assert s.setup() == 0
+    s.iterate(n_iter)
+    want = s.trace()
+    ctx = bmg.Ctx(n, p, body, y, types=(types,))
+    b = bmg.Batch([ctx], [0], [cfg], dict(trace_every_iter=1))
+    b.setup()
+    b.run(n_iter)
+    got = b.trace(0)
+    for key in ("move", "jd", "ms", "size"):
+        assert np.array_equal(got[key], want[key]), key
+    assert np.allclose(got["loglik"], want["loglik"], rtol=1e-10, atol=0)
+    assert got["size"].max() > 0
+    b.close()
+    ctx.close()
+
+
 # columns before the removal; the removed term; n - 1 columns follow it
 @pytest.mark.parametrize("k,rm", [(2, 0), (9, 0), (9, 4), (9, 8), (64, 0), (65, 0), (66, 0), (66, 60), (129, 0),
                                   (130, 1), (130, 70), (135, 0), (135, 127), (135, 134)])
