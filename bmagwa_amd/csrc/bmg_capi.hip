@@ -7,6 +7,8 @@
 #include <cmath>
 #include <cstdio>
 #include <cstring>
+#include <memory>
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -466,10 +468,51 @@ struct bmg_batch {
   std::vector<double*> xy_dev;
 };
 
+// Pinned memory for the scalars of 64 models.  A dataset hands out one page
+// (and takes another where 64 models live); its models hold on to theirs, so
+// the page goes with the last of them and the dataset.  (Pinned memory of each
+// model's own made creating and closing one 25-45 us longer, of 225.)
+namespace bmg {
+struct ScalarPage {
+  ModelScalars* at = nullptr;
+  std::mutex mu;
+  uint64_t used = 0;
+  ScalarPage() = default;
+  ScalarPage(const ScalarPage&) = delete;
+  ~ScalarPage() { if (at) (void)hipHostFree(at); }
+  ModelScalars* take() {
+    std::lock_guard<std::mutex> lock(mu);
+    if (!~used) return nullptr;
+    const int i = __builtin_ctzll(~used);
+    used |= 1ull << i;
+    return at + i;
+  }
+  void give(ModelScalars* s) {
+    std::lock_guard<std::mutex> lock(mu);
+    used &= ~(1ull << (s - at));
+  }
+};
+}  // namespace bmg
+
 struct bmg_model {
   bmg_batch* b = nullptr;
   ModelScalars* s = nullptr;   // pinned: the state's scalars after the last method
+  std::shared_ptr<ScalarPage> page;
 };
+
+static int model_scalars(bmg_ctx* c, bmg_model* m) {
+  std::lock_guard<std::mutex> lock(c->scalars_mu);
+  if (c->scalars) m->s = c->scalars->take();
+  if (!m->s) {
+    auto page = std::make_shared<ScalarPage>();
+    BMG_HIP(hipHostMalloc((void**)&page->at, 64 * sizeof(ModelScalars)));
+    c->scalars = page;
+    m->s = page->take();
+  }
+  m->page = c->scalars;
+  std::memset((void*)m->s, 0, sizeof(ModelScalars));
+  return BMG_OK;
+}
 
 static void tree_layout(DevData& D) {
   uint64_t len = (D.p + 63) / 64 * 64;
@@ -1588,15 +1631,14 @@ static int launch_model_op(bmg_model* m, ModelOpArgs a) {
 
 // a model on the one-chain batch b (which it owns from here on): its empty
 // state's log-likelihood computed
-static int model_open(bmg_batch* b, bmg_model** out) {
+static int model_open(bmg_ctx* ctx, bmg_batch* b, bmg_model** out) {
   bmg_model* m = new bmg_model();
   m->b = b;
-  hipError_t e = hipHostMalloc((void**)&m->s, sizeof(ModelScalars));
-  if (e != hipSuccess) { bmg_model_destroy(m); return hip_fail(e, "hipHostMalloc"); }
-  std::memset(m->s, 0, sizeof(ModelScalars));
+  int rc = model_scalars(ctx, m);
+  if (rc) { bmg_model_destroy(m); return rc; }
   ModelOpArgs a{};
   a.op = 2;
-  int rc = launch_model_op(m, a);
+  rc = launch_model_op(m, a);
   if (rc) { bmg_model_destroy(m); return rc; }
   *out = m;
   return BMG_OK;
@@ -1633,7 +1675,7 @@ extern "C" int bmg_model_create(bmg_ctx* ctx, const bmg_model_prior* prior, bmg_
   K.nus2_plus_yy = prior->nus2_plus_yy;
   K.nus2 = prior->nus2_plus_yy - ctx->yy;
   BMG_HIP(hipMemcpy(b->d_consts, &K, sizeof(ChainConst), hipMemcpyHostToDevice));
-  return model_open(b, out);
+  return model_open(ctx, b, out);
 }
 
 extern "C" int bmg_model_create_sampler(bmg_ctx* ctx, const bmg_opts* opts, bmg_model** out) {
@@ -1648,7 +1690,7 @@ extern "C" int bmg_model_create_sampler(bmg_ctx* ctx, const bmg_opts* opts, bmg_
   bmg_batch* b = nullptr;
   int rc = batch_create(&ctx, 1, 1, &zero, &o, &cfg, 1, &b);
   if (rc) return rc;
-  return model_open(b, out);
+  return model_open(ctx, b, out);
 }
 
 extern "C" int bmg_model_sample_beta_sigma2(bmg_model* m) {
@@ -1706,7 +1748,7 @@ extern "C" int bmg_model_rollback(bmg_model* proposed, const bmg_model* current)
 extern "C" int bmg_model_destroy(bmg_model* m) {
   if (!m) return BMG_OK;
   bmg_batch_destroy(m->b);
-  if (m->s) (void)hipHostFree(m->s);
+  if (m->s) m->page->give(m->s);
   delete m;
   return BMG_OK;
 }

@@ -147,7 +147,7 @@ struct KernelArgs {
 
 // what the host reads after a Model method: in pinned host memory, which the
 // kernel writes itself, so a call waits for its kernel and copies nothing
-struct ModelScalars {
+struct alignas(64) ModelScalars {
   double ll, pves[3];
   int32_t cols, nloci, err, pad;
 };

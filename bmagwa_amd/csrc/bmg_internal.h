@@ -3,10 +3,14 @@
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>
+#include <memory>
+#include <mutex>
 #include <string>
 #include <vector>
 
 #include "../../include/bmagwa_hip.h"
+
+namespace bmg { struct ScalarPage; }
 
 struct bmg_ctx {
   int device = 0;
@@ -43,6 +47,9 @@ struct bmg_ctx {
   int no_tune = 0;  // inside a graph capture: no timed tuning (default shape)
   uint32_t scan_tw[17] = {0};
   unsigned scan_gx[17] = {0};
+  // pinned memory that the dataset's models take their scalars from
+  std::mutex scalars_mu;
+  std::shared_ptr<bmg::ScalarPage> scalars;
 };
 
 namespace bmg {

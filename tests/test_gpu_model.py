@@ -322,3 +322,50 @@ def test_pve_is_of_the_returned_fit_without_a_new_draw(bmg):
     check()
     m.sample_beta_sigma2()
     check()
+
+
+def test_many_models_of_one_dataset(bmg):
+    """More models than one page of scalars holds (64), closed out of order
+    and replaced, also by several threads at once and after their dataset:
+    each keeps its own state."""
+    import threading
+    n, p = 300, 200
+    body, y, cfg = _sampler_dataset(n, p, 7)
+    ctx = bmg.Ctx(n, p, body, y)
+
+    def make(j):
+        m = bmg.Model(ctx, cfg=cfg)
+        m.add_term(j, 0, 3.0)
+        return m
+
+    want = {}
+    for j in range(140):
+        m = make(j)
+        want[j] = m.log_likelihood()
+        m.close()
+    assert len(set(want.values())) > 130
+    live = {j: make(j) for j in range(70)}
+    for j in range(0, 70, 3):
+        live.pop(j).close()
+    for j in range(70, 140):
+        live[j] = make(j)
+    failed = []
+
+    def work(t):
+        for j in range(t, 140, 4):
+            m = make(j)
+            if m.size() != 1 or m.log_likelihood() != want[j]:
+                failed.append(j)
+            m.close()
+
+    threads = [threading.Thread(target=work, args=(t,)) for t in range(4)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not failed
+    for j, m in live.items():
+        assert m.size() == 1 and m.log_likelihood() == want[j]
+    ctx.close()
+    for m in live.values():
+        m.close()
