@@ -369,3 +369,25 @@ def test_many_models_of_one_dataset(bmg):
     ctx.close()
     for m in live.values():
         m.close()
+
+
+@pytest.mark.parametrize("dr", [0, 8])
+def test_model_copies_between_pools_of_one_and_two_sizes(bmg, dr):
+    """A copy takes the whole state along: both models go on alike, whether
+    their pools are of one size (one copy) or of two."""
+    n, p = 300, 200
+    body, y, cfg = _sampler_dataset(n, p, 7)
+    ctx = bmg.Ctx(n, p, body, y)
+    a = bmg.Model(ctx, cfg=dict(cfg, delay_rejection=8))
+    b = bmg.Model(ctx, cfg=dict(cfg, delay_rejection=dr))
+    for j in (3, 50, 120, 7):
+        a.add_term(j, 0, 3.0)
+    for dst, src in ((b, a), (a, b)):
+        dst.commit_from(src)
+        assert dst.size() == src.size() and dst.log_likelihood() == src.log_likelihood()
+        for m in (a, b):
+            m.add_term(90, 0, 2.0)
+            m.remove_term(1)
+        sa, sb = a.get(), b.get()
+        assert all(np.array_equal(sa[k], sb[k]) for k in sa)
+        a.sample_beta_sigma2()
