@@ -112,9 +112,10 @@ def test_factor_in_hbm_matches_oracle(bmg, types, ld, dr):
 
 def test_models_beyond_the_lds_capacity(bmg):
     """220 causal SNPs at h2 = 0.9 (n = 2,000, p = 3,000): the models grow past
-    the 160 columns an LDS-resident factor holds, the batch picks the
-    256-column capacity from the prior, and the trajectory over 3,000
-    iterations is the oracle's."""
+    the 160 columns an LDS-resident factor holds, so the chain goes on with its
+    factor in HBM, and on to more than 193 columns, where the sweeps and the
+    downdate take four entries a lane; the trajectory over 3,000 iterations is
+    the oracle's."""
     n, p, nc, n_iter = 2000, 3000, 220, 3000
     thresh, rho, _ = synth.snp_layout(p, (0.05, 0.5), None, 77)
     body = oracle.synth_genotypes(77, n, p, thresh, rho)
@@ -130,6 +131,9 @@ def test_models_beyond_the_lds_capacity(bmg):
     tr = b.trace(0)
     compare(tr, s.trace(), n_iter)
     assert tr["size"].max() > 160
+    # accepted removals from models of more than 193 columns
+    size = tr["size"].astype(int)
+    assert ((size[1:] < size[:-1]) & (size[:-1] + 1 > 193)).sum() > 20
     assert np.allclose(b.p_rao(0), s.p_rao(), rtol=1e-8, atol=1e-10)
 
 
@@ -156,6 +160,30 @@ def test_chains_leave_a_small_capacity_with_the_same_trajectory(bmg, capacity):
     compare(tr, s.trace(), n_iter)
     assert tr["size"].max() + 1 > capacity - 21
     assert np.allclose(b.p_rao(0), s.p_rao(), rtol=1e-8, atol=1e-10)
+
+
+def test_two_column_models_cross_a_small_capacity_both_ways(bmg):
+    """Two columns a SNP and a capacity of 64: the next move's growth, two
+    columns a SNP, takes the chain to the factor in HBM and back several times,
+    and the trajectory is the oracle's."""
+    n, p, nc, n_iter = 1000, 400, 26, 2000
+    thresh, rho, _ = synth.snp_layout(p, (0.05, 0.5), None, 77)
+    body = oracle.synth_genotypes(77, n, p, thresh, rho)
+    dec = lambda snps: np.stack([oracle.decode(body, n, int(j), 0) for j in snps])
+    y, causal, _ = synth.phenotype(dec, n, p, nc, 0.3, 77, dominance=True)
+    cfg = synth.sampler_cfg(n, p, nc, types="AH", seed=4, n_rao=100, n_rao_burnin=5, thin=10, do_n_iter=n_iter)
+    s = oracle_run(cfg, body, y, n_iter)
+    ctx = bmg.Ctx(n, p, body, y, types=("AH",))
+    b = bmg.Batch([ctx], [0], [cfg], dict(trace_every_iter=1, capacity=64))
+    b.setup()
+    b.run(n_iter)
+    tr = b.trace(0)
+    compare(tr, s.trace(), n_iter)
+    # past 64 columns (so in HBM) and 12 inside again (so back), in turn
+    cols = 2 * tr["size"].astype(int) + 1
+    where = np.sign((cols > 64).astype(int) - (cols <= 52).astype(int))
+    where = where[where != 0]
+    assert (np.diff(where) != 0).sum() >= 8
 
 
 def test_models_past_the_device_limit_stop_with_an_error(bmg):
