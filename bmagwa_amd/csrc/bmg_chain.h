@@ -115,7 +115,9 @@ struct ChainArrays {
   uint32_t* th_size; uint32_t* th_loci; double* th_ll; double* th_s2; double* th_alpha;
   double* th_pve;        // 3 per thinned sample (src/model.hpp:345-392)
   double* th_beta;       // save_beta: beta of every thinned sample, concatenated
-  double* dr_lp;         // 2 x 2^dr: second-stage log-probabilities (null: dr == 0)
+  // 2 x 2^dr (null: dr == 0), by sub-model of the second stage: its factor
+  // block's determinant, later its log-probability; its residual term
+  double* dr_lp;
 };
 
 // error flags of a chain; the flags in ERR_STOP stop the chain

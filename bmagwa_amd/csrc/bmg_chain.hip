@@ -8,9 +8,11 @@
 // is uniform; the O(n k) parts use all 256 threads and the O(k^2) triangular
 // and Givens sweeps use wave 0.  Triangular solves and the Cholesky
 // factorisation are right-looking: each element receives its subtractions in
-// the same order as the netlib loops of the CPU oracle, so with contraction
-// off the factors agree bit for bit; only the inner products differ in
-// summation order.
+// the same order as the netlib loops of the CPU oracle, but fused, with
+// reciprocals in place of divisions, and a removal's rotations are found by
+// another method, so factors agree to rounding and log-likelihoods to 1e-10.
+// Compiled with contraction off, so that only the fused steps written out are
+// fused.
 #include <hip/hip_runtime.h>
 #include <math.h>
 
@@ -162,7 +164,7 @@ struct Smem {
 // 1,000 cycles, and every lane would compute the same one for each draw.  A
 // draw is a read of its lane; the stream itself is unchanged.  (With the
 // DPP scan below a pick went from 3.6 to 3.0 us, and with the terms' draws in
-// parallel 500 iterations of 16 chains over 10,000 SNPs from 122.8 to 118.6 ms.)
+// parallel 500 iterations of 16 chains over 500,000 SNPs from 122.8 to 118.6 ms.)
 struct ChainRng : Rng {
   uint64_t base;                         // counter of lane 0's block
   uint32_t w[4];                         // this lane's block
@@ -234,32 +236,7 @@ struct Ctx {
 __device__ __forceinline__ int lane_id() { return threadIdx.x & 63; }
 __device__ __forceinline__ int wave_id() { return threadIdx.x >> 6; }
 
-// broadcast a value computed on wave 0 lane 0 to every thread
-template <int KMAX>
-__device__ __forceinline__ double bcast_d(Smem<KMAX>& S, double v) {
-  __syncthreads();
-  if (threadIdx.x == 0) S.bcd[0] = v;
-  __syncthreads();
-  double r = S.bcd[0];
-  __syncthreads();
-  return r;
-}
-template <int KMAX>
-__device__ __forceinline__ long long bcast_i(Smem<KMAX>& S, long long v) {
-  __syncthreads();
-  if (threadIdx.x == 0) S.bci[0] = v;
-  __syncthreads();
-  long long r = S.bci[0];
-  __syncthreads();
-  return r;
-}
-
 // ------------------------------------------------------------ genotypes ---
-__device__ __forceinline__ int coding_of_type(int type, int second) {
-  // AH splits into A then H (src/model.hpp:254-258)
-  return type == 4 ? (second ? 1 : 0) : type;
-}
-
 // a column of SNP `snp` under one coding, as one number (-1: none)
 __device__ __forceinline__ long long column_key(long long snp, int coding) {
   return snp < 0 ? -1 : snp * 4 + coding;
@@ -441,8 +418,12 @@ __device__ __forceinline__ void column_dots_np(Ctx<KMAX>& C, uint64_t snp_new, i
 }
 
 // the group width and pieces per lane for the column length: the narrowest
-// group that holds a column in one piece a lane, and from 64 pieces on the
-// fewest pieces a lane that hold it (at most five, then several passes)
+// group that holds a column in one piece a lane, and from 64 pieces on two,
+// three or five pieces a lane, the fewest of these that hold it; longer columns
+// (past 20,480 individuals) go in passes of five.  (A column just past a line
+// pays for the pieces that it leaves empty: 300 iterations of 8 chains of
+// 50-70 SNPs take 25.0 ms at n = 12,288 and 35.5 at 14,000, 33.2 at 20,480 and
+// 45.7 at 20,481, 48.8 at 25,000, 75.5 at 50,000.)
 template <int KMAX, int T0, int NTH>
 __device__ __forceinline__ void column_dots(Ctx<KMAX>& C, uint64_t snp_new, int coding, int cols, uint32_t* xnew,
                                             int32_t* acc) {
@@ -1021,36 +1002,6 @@ __device__ __forceinline__ void warm_next(Ctx<KMAX>& C) {
   C.R.warm = -1;
 }
 
-// draw an index with probability w_i / total (wave 0 computes, all return)
-template <int KMAX>
-__device__ __forceinline__ uint64_t tree_pick(Ctx<KMAX>& C, int tr, double u) {
-  if (wave_id() == 0) {
-    const int lane = lane_id();
-    double total = tr == 0 ? C.R.tot_add : C.R.tot_rem;
-    double r = u * total, carry = 0.0;
-    uint64_t g = 0;
-    long long res = 0;
-    for (int h = C.D.top; h >= 0; --h) {
-      double c = tree_val(C, tr, h, 64 * g + lane);
-      double s = dpp_scan(c);
-      unsigned long long m1 = __ballot(c > 0.0 && r < carry + s);
-      unsigned long long nz = __ballot(c > 0.0);
-      int pick = m1 ? (__ffsll((long long)m1) - 1) : (nz ? 63 - __clzll((long long)nz) : -1);
-      if (pick < 0) { res = -1; break; }
-      double sp = readlane_d(s, pick > 0 ? pick - 1 : 0);   // uniform lane: a scalar read
-      if (pick > 0) carry = carry + sp;
-      g = 64 * g + (uint64_t)pick;
-      res = (long long)g;
-    }
-    if (lane == 0) C.S.bci[1] = res;
-  }
-  __syncthreads();
-  long long r = C.S.bci[1];
-  __syncthreads();
-  if (r < 0) { C.R.err |= ERR_TREE; r = 0; }
-  return (uint64_t)r;
-}
-
 // set leaf i to its weight (unzero) or 0 (zero) and update the path; the
 // new total goes to S.bcd[1].  One wave.
 template <int KMAX>
@@ -1134,10 +1085,10 @@ __device__ __forceinline__ void job_finish(Ctx<KMAX>& C) {
   tree_set(C, tr, C.R.job_ind, 0);
 }
 
-// Pick a leaf with probability w_i / total and zero it (a tree_pick then a
-// tree_set(zero)), reusing the groups the descent read: the path's sums are
-// recomputed from them in tree_set's order, so the tree ends up exactly as
-// after the two calls.  *w_out: the picked leaf's weight.
+// Pick a leaf with probability w_i / total and zero it, reusing the groups the
+// descent read: the path's sums are recomputed from them in tree_set's order,
+// so the tree ends up exactly as after a tree_set(zero) of the leaf.  *w_out:
+// the picked leaf's weight.
 template <int KMAX>
 __device__ __forceinline__ uint64_t tree_pick_zero(Ctx<KMAX>& C, int tr, double u, double* w_out) {
   double* g0 = tr == 0 ? gp(C.A.tree_add) : gp(C.A.tree_rem);
@@ -3516,6 +3467,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
     Smem<KMAX_LDS> small;
     Smem<BMG_KMAXG> large;
   } U;
+  // (a workgroup has a compute unit to itself)
+  static_assert(sizeof(U) <= 160 * 1024, "a workgroup has 160 KB of LDS");
   const int c = blockIdx.x;
   if (c >= args.n_chains) return;
   const ChainScal& CS = args.scal[c];

@@ -187,42 +187,11 @@ __device__ inline long long block_sum_i64(long long v, long long* red) {
 // --------------------------------------------------------- genotype bits --
 // A 32-bit word holds 16 individuals, individual i at bits 2 (i % 16).
 // Codes (src/data.cpp:36): 00 -> 0, 01 -> missing, 10 -> 1, 11 -> 2.
-// Per coding the value is p1 + p2 with two bit planes (even bit positions):
-//   A: p1 = hi, p2 = hi & lo      H: p1 = hi & ~lo      D: p1 = hi
-//   R: p1 = hi & lo               (missing counts as 0, as the reference's
-// precompute sees it before missing values are sampled).
+// With hi and lo the fields' bits (at even positions), the value is
+//   A: hi + (hi & lo)      H: hi & ~lo      D: hi      R: hi & lo
+// (missing counts as 0, as the reference's precompute sees it before missing
+// values are sampled).
 #define BMG_EVEN 0x55555555u
-
-__device__ __host__ inline void planes(uint32_t w, int coding, uint32_t& p1, uint32_t& p2) {
-  uint32_t lo = w & BMG_EVEN, hi = (w >> 1) & BMG_EVEN;
-  switch (coding) {
-    case 0: p1 = hi; p2 = hi & lo; break;
-    case 1: p1 = hi & ~lo; p2 = 0; break;
-    case 2: p1 = hi; p2 = 0; break;
-    default: p1 = hi & lo; p2 = 0; break;
-  }
-}
-
-// exact integer dot of two SNP columns (codings ca, cb) over `nw` words
-__device__ inline long long dot_planes(uint32_t a, uint32_t b, int ca, int cb) {
-  uint32_t a1, a2, b1, b2;
-  planes(a, ca, a1, a2);
-  planes(b, cb, b1, b2);
-  return (long long)(__popc(a1 & b1) + __popc(a1 & b2) + __popc(a2 & b1) + __popc(a2 & b2));
-}
-
-// 16 genotype values of a word as four words of int8 (value 0, 1 or 2)
-__device__ inline void word_to_i8x16(uint32_t w, int coding, uint32_t out[4]) {
-  uint32_t p1, p2;
-  planes(w, coding, p1, p2);
-  uint32_t v = p1 + p2;  // each 2-bit field holds the value (<= 2, no carry)
-#pragma unroll
-  for (int b = 0; b < 4; ++b) {
-    uint32_t x = (v >> (8 * b)) & 0xFFu;            // fields f3 f2 f1 f0
-    uint32_t t = (x | (x << 12)) & 0x000F000Fu;     // f1f0 | f3f2 << 16
-    out[b] = (t | (t << 6)) & 0x03030303u;          // f0, f1, f2, f3 bytes
-  }
-}
 
 __device__ inline double code_value(uint32_t c, int coding) {
   // reference tables (src/genotype_tables.hpp), -1 for missing
