@@ -2222,13 +2222,31 @@ __device__ __forceinline__ void exh_moveleft(Smem<KMAX>& S, int w, int nT, int& 
 // receives the product of the sub-model's block diagonal and lp[2^n + i] its
 // residual term.  w: columns per locus.  Wave 0 only (lane 0 stores).  Out of
 // line: inlined, its registers crowd the kernel's hot loops.
+//
+// First each column is scaled by a power of two to a diagonal entry in
+// [1/2, 1).  The walk's rotations act on rows and do not see it, and its
+// products of up to 40 diagonal entries stay far inside the exponent's range
+// whatever the precisions (an entry is at least sqrt(d)); the exponents go back
+// in with the loci's log d.
 template <int KMAX>
 __device__ __noinline__ void exh_walk(Smem<KMAX>& S, int nT_any, int w_any, int n_any, double* lp_any) {
   double* lp = gp(lp_any);
   const int nT = __builtin_amdgcn_readfirstlane(nT_any), w = __builtin_amdgcn_readfirstlane(w_any);
   const int n = __builtin_amdgcn_readfirstlane(n_any);
-  const bool st = lane_id() == 0;
+  const int lane = lane_id();
+  const bool st = lane == 0;
   const uint64_t all = 1ull << n;
+  if (lane < n) {
+    int e = 0;
+    for (int k = 0; k < w; ++k) e += __builtin_amdgcn_frexp_exp(exl(S, w * lane + k, w * lane + k));
+    S.ex_ld[lane] -= (double)e * 0x1.62e42fefa39efp-1;   // ln 2
+  }
+  for (int c = 0; c < nT; ++c) {
+    const int e = __builtin_amdgcn_frexp_exp(exl(S, c, c));
+    wave_sync();
+    if (lane <= c) exl(S, lane, c) = ldexp(exl(S, lane, c), -e);
+  }
+  wave_sync();
   unsigned __int128 ci = 0;      // walk order, five bits a position
   for (int i = 0; i < BMG_DR_MAX + 2; ++i) ci |= (unsigned __int128)(unsigned)i << (5 * i);
   // positions k - 1 and k trade places
@@ -2296,26 +2314,15 @@ __device__ __forceinline__ double exhaustive_modelset(Ctx<KMAX>& C, int cl, int 
   const int w = C.D.type == BMG_AH ? 2 : 1;
   const int nT = w * n;                 // the block's columns: the last n loci
   const int c0 = R.cols - nT;           // after the fixed columns and the other loci
-  // each column scaled by a power of two to a diagonal entry in [1/2, 1): the
-  // walk's rotations act on rows and do not see it, and its products of up to
-  // 40 diagonal entries stay far inside the exponent's range whatever the
-  // precisions (an entry is at least sqrt(d)); the exponents go back in with
-  // the loci's log d
-  for (int c = 0; c < nT; ++c) {
-    const int e = __builtin_amdgcn_frexp_exp(S.L[P(c0 + c) + c0 + c]);
-    for (int r = threadIdx.x; r <= c; r += BMG_BLOCK) S.ex_L[P(c) + r] = ldexp(S.L[P(c0 + c) + c0 + r], -e);
-  }
+  for (int c = 0; c < nT; ++c)
+    for (int r = threadIdx.x; r <= c; r += BMG_BLOCK) S.ex_L[P(c) + r] = S.L[P(c0 + c) + c0 + r];
   for (int i = threadIdx.x; i < nT; i += BMG_BLOCK) S.ex_v[i] = S.v[c0 + i];
-  // per locus: half its columns' log d less the logarithm of their scale, and
-  // the prior change of the q-th one (src/prior.hpp:144-158, one effect type:
-  // it depends on the number alone)
+  // per locus: half its columns' log d, and the prior change of the q-th one
+  // (src/prior.hpp:144-158, one effect type: it depends on the number alone)
   if ((int)threadIdx.x < n) {
     const int q = threadIdx.x, type = C.D.type;
     double ld = 0.0;
-    for (int k = 0; k < w; ++k) {
-      const int c = c0 + w * q + k;
-      ld += 0.5 * log(S.d[c]) - (double)__builtin_amdgcn_frexp_exp(S.L[P(c) + c]) * 0x1.62e42fefa39efp-1;   // ln 2
-    }
+    for (int k = 0; k < w; ++k) ld += 0.5 * log(S.d[c0 + w * q + k]);
     S.ex_ld[q] = ld;
     int Ns[5] = {0, 0, 0, 0, 0};
     put(Ns, type, cl + q);
