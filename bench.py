@@ -72,10 +72,10 @@ SEED = 20261202 + 4000
 HBM_PEAK_GBS = 8000.0
 # HBM bytes per launch of the tuned scan at this workload, from rocprofv3
 # FETCH_SIZE / WRITE_SIZE passes scaled by a copy kernel of known traffic
-# (profiles/kernels_scan_band_copy_n10000_p500000.md): fetch 2 x 626,386.4
-# KiB, write 31,264 KiB
+# (profiles/kernels_scan_band_copy_n10000_p500000.md): fetch 2 x 626,782.8
+# KiB, write 11,719.1 KiB
 SCAN_TRAFFIC = dict(n=10000, p=500000, nvec=3, digits=5,
-                    fetch_bytes=int(2 * 626737.6 * 1024), write_bytes=int(31269.7 * 1024),
+                    fetch_bytes=int(2 * 626782.8 * 1024), write_bytes=int(11719.1 * 1024),
                     source="profiles/kernels_scan_band_copy_n10000_p500000.md")
 INT8_PEAK_TOPS = 5000.0
 
