@@ -191,7 +191,7 @@ def test_c5_largest_dataset(bmg):
     """n = 50,000, p = 1,000,000 (12.5 GB packed), MAF ~ U(0.01, 0.5), 300
     causal SNPs: the scan is exact on representable residuals (sampled SNPs
     against int64 sums), band rows equal the oracle's, and two chains of the
-    256-column kernel with the 200-SNP limit equal the oracle's for 100
+    256-column code with the 200-SNP limit equal the oracle's for 100
     iterations (no RB block inside the run)."""
     n, p = 50000, 1000000
     seed = synth.seed_of(5)

@@ -141,7 +141,7 @@ def test_models_beyond_the_lds_capacity(bmg):
 def test_chains_leave_a_small_capacity_with_the_same_trajectory(bmg, capacity):
     """The same growing models (n = 2,000, p = 3,000, 220 causal, h2 = 0.9)
     in a launch of 64 or 160 columns: a chain whose model comes within one
-    move of the capacity continues in the 256-column kernel from that
+    move of the capacity continues in the 256-column code from that
     iteration, and the trajectory over 2,000 iterations is still the
     oracle's (nothing is rejected for want of room)."""
     n, p, nc, n_iter = 2000, 3000, 220, 2000
